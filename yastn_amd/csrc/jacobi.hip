@@ -65,6 +65,16 @@ __device__ __attribute__((always_inline)) inline double dpp_move(double v) {
   return __hiloint2double(hi, lo);
 }
 
+// The value of the next / previous lane within each row of 16 lanes, cyclically (row_ror by 15 and by 1).
+__device__ __attribute__((always_inline)) inline double row_next(double v) { return dpp_move<0x12F>(v); }
+__device__ __attribute__((always_inline)) inline double row_prev(double v) { return dpp_move<0x121>(v); }
+__device__ __attribute__((always_inline)) inline double2 row_next(double2 v) {
+  return make_double2(row_next(v.x), row_next(v.y));
+}
+__device__ __attribute__((always_inline)) inline double2 row_prev(double2 v) {
+  return make_double2(row_prev(v.x), row_prev(v.y));
+}
+
 __device__ __attribute__((always_inline)) inline double read_lane(double v, int l) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
                           __builtin_amdgcn_readlane(__double2loint(v), l));
@@ -961,6 +971,287 @@ __global__ void __launch_bounds__(kInnerThreads)
   for (int st = st0; st < s1; st += kInnerThreads / 64) {
     if (st != st0) stripe_load<CPLX, KS>(a, stripe_col(st), stripe_rows(st), stripe_idx(st), nc, lane);
     stripe_mul_store<CPLX, KS>(a, stripe_col(st), stripe_rows(st), stripe_idx(st), Q, nq, nc, lane);
+  }
+}
+
+// 1 / sqrt(x) from the hardware approximation (2^-23) and one Newton-Raphson step (2^-45).
+__device__ __attribute__((always_inline)) inline double rsq_half(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+
+// The rotation of rotation() in a shorter chain of dependent operations: with d = b - a, r = sqrt(d^2 + 4 |g|^2)
+// and m = |d| + r, tan(theta) = 2 |g| / m, so c = m / n and s e^{i phi} = sgn(d) 2 g / n with n^2 = m^2 + 4 |g|^2:
+// two reciprocal square roots and no division.  An error of r only tilts the angle (the next sweep sees it); an
+// error of 1 / n scales c and s alike and is removed to rounding by one Newton step on c^2 + s^2 = 1, so that the
+// rotations stay orthogonal (c is exactly 1 for tiny angles).  Squares that leave the exponent range take
+// rotation() itself.  Returns false with c = 1, s = 0 where rotation() does not rotate.
+template <bool CPLX>
+__device__ __attribute__((always_inline)) inline bool rotation_short(double a, double b, double gr, double gi,
+                                                                     double tol2, double floor2, double& c,
+                                                                     double& sr, double& si) {
+  const double g2 = CPLX ? gr * gr + gi * gi : gr * gr;
+  const double g4 = 4.0 * g2;
+  const double d = b - a;
+  const double h = fma(d, d, g4);
+  const bool go = (g2 > tol2 * a * b) & (a > floor2) & (b > floor2);
+  const double m = fma(h, rsq_half(h), fabs(d));
+  const double z = rsq_half(fma(m, m, g4));
+  const double c0 = m * z, f0 = copysign(2.0 * z, d);
+  const double e = 0.5 * fma(-g4, z * z, fma(-c0, c0, 1.0));
+  const double f = fma(f0, e, f0);
+  c = go ? fma(c0, e, c0) : 1.0;
+  sr = go ? gr * f : 0.0;
+  si = CPLX && go ? gi * f : 0.0;
+  if (go && !(h > 1e-280 && h < 1e280)) {
+    double s, er, ei;
+    rotation(a, b, gr, gi, 0.0, 0.0, c, s, er, ei);
+    sr = s * er;
+    si = CPLX ? s * ei : 0.0;
+  }
+  return go;
+}
+
+// Inner sweep and update of one job for panels of 16 columns (the width the host plans use): the same rotations in
+// the same order as panel_inner_kernel, by 256 threads.  What bounds a round of the panel Jacobi is the latency of
+// this sweep, 16 (cross) or 15 (intra) rotations deep, so the layout keeps a sub-round short:
+//  - thread (k, l) = (tid / 16, tid % 16) owns the 2 x 2 block of G of pair slots k and l, [[A, C], [D, B]] =
+//    G([I_k, J_k], [I_l, J_l]), in registers.  The second panel moves past the first one by one place per sub-round
+//    instead of the pairing changing, so slot k always pairs I_k with J_k and no index is looked up.
+//  - every 16 lanes compute the rotations of all 16 slots (lane l slot l) from the three entries of each that
+//    the owners left in LDS: no wave waits for another one's parameters, and there is one barrier per sub-round.
+//    A stays in its registers, C moves by a DPP row rotation, D and B through LDS (double buffered).
+//  - the accumulated rotation stays in registers too, rows k and k + 16 of Q per thread; a step of it needs only
+//    the lane's own rotation and a DPP move.
+// In-kernel clocks, 440-row pairs: partial sums 2.5 us, sweep 6.0 us (complex 3.5 and 8.9), against 3 and 13.5 us
+// with 1024 threads, G and Q in LDS and two barriers per sub-round, where one lane computed a slot's parameters while
+// the others waited.  The update holds Q's fragments in registers and reads each stripe one ahead of the products.
+// Kernel time per round: 13.7 us against 21.9 (27 blocks up to 198 x 198), 12.5 against 20 (one 440 x 440 block).
+// Panels of 32 columns with 1024 threads of the same layout move W and V half as often but measured slower
+// (440 x 440: 10.4 against 7.9 ms; four complex 1100 x 1100: 124 against 116 ms).
+constexpr int kPairThreads = 256;
+template <bool CPLX>
+__global__ void __launch_bounds__(kPairThreads)
+    panel_pair_kernel(const int64_t* __restrict__ blocks, const int32_t* __restrict__ jobs,
+                         typename Num<CPLX>::T* __restrict__ work, const double* __restrict__ floors,
+                         const double* __restrict__ part, int32_t* __restrict__ state, int sweep, int maxch) {
+  typedef Num<CPLX> N;
+  typedef typename N::T T;
+  constexpr int b = 16, KS = 8, nq = 33;
+  __shared__ T s_G[2][2][16][17];   // cross: [buffer][D, B][k][l]; intra: [buffer][0] is G
+  __shared__ double s_a[2][16];
+  __shared__ T s_g[2][16];
+  __shared__ T s_Q[32 * nq];        // column c at s_Q + c nq
+  if (sweep_done(state, sweep)) return;
+  const int32_t* jb = jobs + 3 * (int64_t)blockIdx.x;
+  const BlockDesc d = load_desc(blocks + (int64_t)jb[0] * YH_SVD_WORDS);
+  const PanelPair pp = panel_pair(d, jb, b);
+  const int64_t p = pp.p;
+  const int nc = pp.nc;
+  const bool intra = pp.intra;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int k = tid >> 4, l = tid & 15;
+  // ---- this workgroup's share of the update: the 16-row stripes of W (p rows) then V (q rows), cut into
+  // gridDim.y slices; each wave's first stripe is read now, so that its loads overlap the sweep (nothing
+  // writes W or V of this pair before the update)
+  T* const Wd = work + d.work_off;
+  const int sw = (int)((p + 15) / 16), sv = (int)((pp.q + 15) / 16);
+  const int per = (sw + sv + (int)gridDim.y - 1) / (int)gridDim.y;
+  const int s0 = (int)blockIdx.y * per, s1 = min(sw + sv, s0 + per);
+  auto stripe_col = [&](int st) {  // column c of stripe st's matrix (W, or V after sw stripes)
+    const bool isv = st >= sw;
+    T* X = isv ? Wd + p * pp.q : Wd;
+    const int64_t ldx = isv ? pp.q : p;
+    return [=](int c) { return X + pp.col(c) * ldx; };
+  };
+  auto stripe_rows = [&](int st) { return st >= sw ? (int)pp.q : (int)p; };
+  auto stripe_idx = [&](int st) { return st >= sw ? st - sw : st; };
+  T x[KS];
+  int st = s0 + wave;
+  if (st < s1) stripe_load<CPLX, KS>(x, stripe_col(st), stripe_rows(st), stripe_idx(st), nc, lane);
+  // ---- G: sums of the chunks' partial tiles (16 x 16 row-major, so thread (k, l) reads its own entries), all
+  // loads of a group in flight, summed in chunk order
+  T A = N::make(0.0, 0.0), C = A, B = A, D = A;
+  {
+    constexpr int kSumGroup = 8, kStep = 256 * (CPLX ? 2 : 1);
+    const int nch = (int)((p + kGramRows - 1) / kGramRows);
+    const double* src = part + (int64_t)blockIdx.x * maxch * 3 * kStep + tid;
+    const double* zero = (const double*)kZeroElt + tid;
+    double sum[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+    for (int c0 = 0; c0 < nch; c0 += kSumGroup) {
+      double v[kSumGroup][3][2];
+#pragma unroll
+      for (int g = 0; g < kSumGroup; ++g)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const bool ok = (c0 + g < nch) & (t == 0 || !intra);
+          const double* s = src + ((int64_t)(c0 + g) * 3 + t) * kStep;
+          v[g][t][0] = *(ok ? s : zero);
+          if constexpr (CPLX) v[g][t][1] = *(ok ? s + 256 : zero);
+        }
+#pragma unroll
+      for (int g = 0; g < kSumGroup; ++g)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          sum[t][0] += v[g][t][0];
+          if constexpr (CPLX) sum[t][1] += v[g][t][1];
+        }
+    }
+    A = N::make(sum[0][0], sum[0][1]);
+    C = N::make(sum[1][0], sum[1][1]);
+    B = N::make(sum[2][0], sum[2][1]);
+  }
+  const double tol = DBL_EPSILON * sqrt((double)(p > 1 ? p : 1));
+  const double tol2 = tol * tol, floor2 = floors[jb[0]];
+  bool any = false;
+  // one step of the block: rows by the rotation of slot k (J^H), columns by that of slot l (J)
+  auto turn = [&](double ck, double srk, double sik, double cl, double srl, double sil) {
+    apply_rot<CPLX>(A, D, ck, 1.0, srk, -sik);
+    apply_rot<CPLX>(C, B, ck, 1.0, srk, -sik);
+    apply_rot<CPLX>(A, C, cl, 1.0, srl, sil);
+    apply_rot<CPLX>(D, B, cl, 1.0, srl, sil);
+  };
+  if (!intra) {
+    T u0 = N::make(k == l ? 1.0 : 0.0, 0.0), u1 = N::make(0.0, 0.0);  // Q(k, I_l), Q(k + 16, I_l)
+    T v0 = u1, v1 = u0;                                              // Q(k, J_l), Q(k + 16, J_l)
+    s_G[0][0][l][k] = N::conj(C);
+    s_G[0][1][k][l] = B;
+    if (k == l) {
+      s_a[0][l] = N::re(A);
+      s_g[0][l] = C;
+    }
+    __syncthreads();
+    for (int s = 0; s < b; ++s) {
+      const int w = s & 1, k1 = s ? (k + 1) & 15 : k, l1 = s ? (l + 1) & 15 : l;  // the second panel moves up one place
+      const T gl = s_g[w][l];
+      const double al = s_a[w][l], bl = N::re(s_G[w][1][l1][l1]);
+      D = s_G[w][0][k1][l];
+      B = s_G[w][1][k1][l1];
+      double cl, srl, sil;
+      const bool go = rotation_short<CPLX>(al, bl, N::re(gl), N::im(gl), tol2, floor2, cl, srl, sil);
+      if (__any(go)) {
+        any = true;
+        const int from = (lane & 48) + k;  // a lane of this row of 16 that holds slot k
+        const double ck = __shfl(cl, from), srk = __shfl(srl, from), sik = CPLX ? __shfl(sil, from) : 0.0;
+        turn(ck, srk, sik, cl, srl, sil);
+        apply_rot<CPLX>(u0, v0, cl, 1.0, srl, sil);
+        apply_rot<CPLX>(u1, v1, cl, 1.0, srl, sil);
+      }
+      if (s + 1 < b) {
+        s_G[w ^ 1][0][k][l] = D;
+        s_G[w ^ 1][1][k][l] = B;
+        if (k == l) s_a[w ^ 1][l] = N::re(A);
+        if (l == ((k + 1) & 15)) s_g[w ^ 1][k] = C;
+        C = row_next(C);
+        __syncthreads();
+      }
+      v0 = row_next(v0);
+      v1 = row_next(v1);
+    }
+    if (any) {  // the same in every wave
+      s_Q[l * nq + k] = u0;
+      s_Q[l * nq + k + 16] = u1;
+      s_Q[(l + 16) * nq + k] = v0;
+      s_Q[(l + 16) * nq + k + 16] = v1;
+    }
+  } else {
+    // one panel against itself: the circle order of its 16 columns as a ring of 15 places, 8 slots; the lanes
+    // and rows beyond 8 repeat those below (every column of the panel past its width is zero and never rotates)
+    const int k8 = k & 7, l8 = l & 7;
+    auto from_top = [](int i) { return i == 0 ? 0 : i == 1 ? 8 : i - 1; };
+    auto from_bot = [](int i) { return i == 7 ? 7 : 9 + i; };
+    T u0 = N::make(k == l8 ? 1.0 : 0.0, 0.0), v0 = N::make(k == l8 + 8 ? 1.0 : 0.0, 0.0);  // Q(k, top l8), Q(k, bottom l8)
+    s_G[0][0][k][l] = A;
+    __syncthreads();
+    for (int s = 0; s < b - 1; ++s) {
+      const int w = s & 1;
+      const int rt = s ? from_top(k8) : k8, rb = s ? from_bot(k8) : k8 + 8;
+      const int ct = s ? from_top(l8) : l8, cb = s ? from_bot(l8) : l8 + 8;
+      const T gl = s_G[w][0][ct][cb];
+      const double al = N::re(s_G[w][0][ct][ct]), bl = N::re(s_G[w][0][cb][cb]);
+      A = s_G[w][0][rt][ct];
+      C = s_G[w][0][rt][cb];
+      D = s_G[w][0][rb][ct];
+      B = s_G[w][0][rb][cb];
+      double cl, srl, sil;
+      const bool go = rotation_short<CPLX>(al, bl, N::re(gl), N::im(gl), tol2, floor2, cl, srl, sil);
+      if (__any(go)) {
+        any = true;
+        const int from = (lane & 48) + k8;
+        const double ck = __shfl(cl, from), srk = __shfl(srl, from), sik = CPLX ? __shfl(sil, from) : 0.0;
+        turn(ck, srk, sik, cl, srl, sil);
+        apply_rot<CPLX>(u0, v0, cl, 1.0, srl, sil);
+      }
+      if (s + 2 < b) {
+        if (k < 8 && l < 8) {
+          s_G[w ^ 1][0][k][l] = A;
+          s_G[w ^ 1][0][k][l + 8] = C;
+          s_G[w ^ 1][0][k + 8][l] = D;
+          s_G[w ^ 1][0][k + 8][l + 8] = B;
+        }
+        __syncthreads();
+      }
+      const T un = row_prev(u0), vp = row_prev(v0), vn = row_next(v0);  // of lanes l - 1, l - 1, l + 1
+      const T u = u0;
+      u0 = l8 == 0 ? u : l8 == 1 ? vp : un;
+      v0 = l8 == 7 ? u : vn;
+    }
+    if (any) {
+      const T zero = N::make(0.0, 0.0);
+      s_Q[l * nq + k] = zero;
+      s_Q[l * nq + k + 16] = zero;
+      s_Q[(l + 16) * nq + k] = zero;
+      s_Q[(l + 16) * nq + k + 16] = zero;
+      __syncthreads();
+      if (l < 8) {
+        s_Q[l * nq + k] = u0;
+        s_Q[(l + 8) * nq + k] = v0;
+      }
+    }
+  }
+  if (!any) return;  // uniform: nothing rotated, W and V of the pair are unchanged
+  if (tid == 0 && blockIdx.y == 0) state[kStateHead + sweep] = 1;
+  __syncthreads();
+  // ---- the pair's columns of this workgroup's stripes <- (.) Q in place, as Q^T X^T (a lane's four results run down
+  // a column, so a store covers 16 consecutive rows); Q's fragments stay in registers
+  double qr[2][KS], qi[2][KS];
+#pragma unroll
+  for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const T q = s_Q[(tj * 16 + (lane & 15)) * nq + 4 * i + (lane >> 4)];
+      qr[tj][i] = N::re(q);
+      qi[tj][i] = N::im(q);
+    }
+  const int tiles = intra ? 1 : 2;
+  for (; st < s1; st += kPairThreads / 64) {
+    auto col = stripe_col(st);
+    const int rows = stripe_rows(st), row = stripe_idx(st) * 16 + (lane & 15);
+    T y[KS];
+#pragma unroll
+    for (int i = 0; i < KS; ++i) y[i] = x[i];
+    const int nx = st + kPairThreads / 64;
+    if (nx < s1) stripe_load<CPLX, KS>(x, stripe_col(nx), stripe_rows(nx), stripe_idx(nx), nc, lane);
+#pragma unroll
+    for (int tj = 0; tj < 2; ++tj) {
+      if (tj < tiles) {
+        d4 accR = {0.0, 0.0, 0.0, 0.0}, accI = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+          accR = __builtin_amdgcn_mfma_f64_16x16x4f64(qr[tj][i], N::re(y[i]), accR, 0, 0, 0);
+          if constexpr (CPLX) {
+            accI = __builtin_amdgcn_mfma_f64_16x16x4f64(qi[tj][i], N::re(y[i]), accI, 0, 0, 0);
+            accR = __builtin_amdgcn_mfma_f64_16x16x4f64(-qi[tj][i], N::im(y[i]), accR, 0, 0, 0);
+            accI = __builtin_amdgcn_mfma_f64_16x16x4f64(qr[tj][i], N::im(y[i]), accI, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int c = tj * 16 + (lane >> 4) + 4 * v;
+          if (row < rows && c < nc) col(c)[row] = N::make(accR[v], accI[v]);
+        }
+      }
+    }
   }
 }
 
@@ -1923,7 +2214,10 @@ extern "C" int yastn_hip_svd_panel_sweep(void* work, const double* floors, int d
       else
         hipLaunchKernelGGL((panel_gram_kernel<true, 8>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
                            jobs, (const double2*)work, (double*)part, b, gch, d_state, sweep);
-      if (wide)
+      if (b == 16)
+        hipLaunchKernelGGL((panel_pair_kernel<true>), gi, dim3(kPairThreads), 0, stream, d_blocks, jobs, (double2*)work,
+                           floors, (const double*)part, d_state, sweep, gch);
+      else if (wide)
         hipLaunchKernelGGL((panel_inner_kernel<true, 16>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
                            d_blocks, jobs, (double2*)work, floors, (const double*)part, d_state, sweep, b, gch,
                            lds_inner);
@@ -1938,7 +2232,10 @@ extern "C" int yastn_hip_svd_panel_sweep(void* work, const double* floors, int d
       else
         hipLaunchKernelGGL((panel_gram_kernel<false, 8>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
                            jobs, (const double*)work, (double*)part, b, gch, d_state, sweep);
-      if (wide)
+      if (b == 16)
+        hipLaunchKernelGGL((panel_pair_kernel<false>), gi, dim3(kPairThreads), 0, stream, d_blocks, jobs, (double*)work,
+                           floors, (const double*)part, d_state, sweep, gch);
+      else if (wide)
         hipLaunchKernelGGL((panel_inner_kernel<false, 16>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
                            d_blocks, jobs, (double*)work, floors, (const double*)part, d_state, sweep, b, gch,
                            lds_inner);

@@ -712,8 +712,30 @@ SVD_LDS_MAX_Q = int(os.environ.get('YASTN_HIP_SVD_LDS_MAX_Q', '16'))
 # workgroups per round but more rounds per sweep.  Tuning knob; the LDS limit may lower it further.
 PANEL_WIDTH = int(os.environ.get('YASTN_HIP_PANEL_WIDTH', '16'))
 PANEL_CHUNK_ROWS = 64  # rows per workgroup of the panel Gram kernel
-# workgroups per panel pair in the inner kernel (0: about one 16-row stripe of W and V per wave); tuning knob
+# workgroups per panel pair in the inner kernel (0: panel_slices below); tuning knob
 PANEL_SLICES = max(0, min(64, int(os.environ.get('YASTN_HIP_PANEL_SLICES', '0'))))
+
+
+def panel_slices(cross, stripes, cplx, width):
+    """Workgroups per panel pair in the inner kernel of a round of ``cross`` pairs: each sums the Gram partials
+    and repeats the inner sweep, then updates its slice of the pair's 16-row stripes of W and V.
+
+    With 16-column panels a workgroup has 4 waves, so more slices than a quarter of the stripes are idle.  The
+    round lasts as long as the fullest CU, which holds g = ceil(cross slices / CUs) workgroups: g / slices of a
+    pair's update (0.3 us per stripe of 4 waves, complex 0.6) plus the sweep, 6 us (complex 9) and about 0.8 of that
+    again per further workgroup; the fewest slices of least cost are taken.  Measured (whole SVD): 14 pairs
+    of 56 stripes 11.2 ms with 1 slice, 7.6 with 14; 84 pairs 13.5 with 1, 11.0 with 3, 12.1 with 7; 140 pairs 13.7 with
+    1, 12.9 with 3, 16.5 with 10; 138 complex pairs of 138 stripes 135 with 1, 114 with 3, 128 with 4, 161 with 14.
+    Other widths: 16 waves and a longer sweep, so at most about one workgroup per CU and one stripe per wave."""
+    cu = L.device_cu_count()
+    if width != 16:
+        return max(1, min(64, -(-stripes // 16), cu // cross))
+    stripe, sweep = (0.6, 9.0) if cplx else (0.3, 6.0)
+
+    def cost(s):
+        g = -(-cross * s // cu)
+        return g * stripes * stripe / s + sweep * (1 + 0.8 * (g - 1))
+    return min(range(1, max(1, min(64, -(-stripes // 4))) + 1), key=lambda s: (cost(s), s))
 
 
 class SvdPlan:
@@ -819,16 +841,10 @@ class SvdPlan:
                 offs.append((len(jobs), len(per_round[r])))
                 jobs.extend(per_round[r])
             self.rounds = offs
-            # workgroups per panel pair in the inner kernel: each sums the Gram partials and repeats the
-            # inner sweep, then updates its slice of the 16-row stripes of W and V.  At most about one
-            # stripe per wave (16 waves); and about one workgroup per CU over the largest round of cross
-            # pairs, since every further slice repeats the sequential inner sweep (measured: rounds of
-            # ~260 pairs of up to 1134-row complex blocks run 2x faster with 1 slice than with 9, rounds
-            # of ~75 pairs of up to 440-row blocks fastest with 3).
-            per_wave = -(-(-(-pmax // 16) - (-qmax // 16)) // 16)
+            stripes = -(-pmax // 16) - (-qmax // 16)
             maxn = max(n for _, n in offs)
             cross = max((n for _, n in offs[1:]), default=maxn)
-            self.panel_slices = PANEL_SLICES or max(1, min(64, per_wave, L.device_cu_count() // cross))
+            self.panel_slices = PANEL_SLICES or panel_slices(cross, stripes, itemsize == 16, width)
             self.h_rounds = np.ascontiguousarray(np.array(offs, dtype=np.int64).reshape(-1, 2))
             self.d_rounds = torch.from_numpy(self.h_rounds).to(device)
             self.max_round_jobs = maxn
