@@ -35,7 +35,7 @@ extern "C" {
 #define YH_F64 0
 #define YH_C128 1
 
-#define YH_ABI_VERSION 13
+#define YH_ABI_VERSION 14
 
 /* ---- box-gather plan (one job per copied or zero-filled box) -------------
  * int64 words per job (YH_JOB_WORDS):
@@ -209,6 +209,16 @@ int yastn_hip_eigh(void* S, void* U, const void* A, int dtype, const int64_t* d_
  * at the rounding-noise level of the block.  maxch_p = ceil(max p / 64); part holds >= (max jobs per
  * round) maxch_p T (T + 1) / 2 256 (x2 complex) doubles, T = ceil(2b / 16).  b <= 32.
  * yastn_hip_check_panel_jobs validates a job list against the blocks on the host. */
+/* Blocks of A4 / A5 with min(m, n) <= 32: the listed blocks (order[0 ... n-1]; SVD words as for yastn_hip_svd) are each
+ * decomposed by one workgroup in one launch, with the outputs and info words of yastn_hip_svd (mode 0) or
+ * yastn_hip_eigh (mode 1).  lds_bytes holds (p|1) q + (q|1) q + 2 h (h+1) elements of every block, p = max(m, n),
+ * q = min(m, n), h = 16 for q <= 16, else 32 (checked on the host by yastn_hip_check_small_plan). */
+#define YH_SMALL_Q 32
+int yastn_hip_check_small_plan(const int64_t* h_blocks, int64_t nblocks, const int32_t* h_order, int64_t n, int mode,
+                               int dtype, int64_t lds_bytes);
+int yastn_hip_jacobi_small(void* U, void* S, void* Vh, const void* A, int dtype, int mode, const int64_t* d_blocks,
+                           const int32_t* d_order, int64_t n, int64_t lds_bytes, int32_t* d_info, int max_sweeps,
+                           hipStream_t stream);
 int yastn_hip_device_info(int* lds_per_block, int* num_cu);
 int yastn_hip_svd_panel_init(const void* A, void* work, double* mu, double* floors, int dtype, int mode,
                              const int64_t* d_blocks, const int32_t* d_ids, int64_t nb, hipStream_t stream);

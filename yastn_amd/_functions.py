@@ -594,25 +594,27 @@ def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
     st = stream_of(data)
     work = torch.empty(max(plan.work_numel, 1), dtype=data.dtype, device=data.device)
     info = torch.empty(max(plan.nblocks, 1), dtype=torch.int32, device=data.device)
-    joined = None
-    if plan.n_lds:
-        # the LDS-resident kernel (one workgroup per small block) runs on a side stream, overlapping
-        # the panel path of the large blocks, which occupies only part of the GPU; joined below
-        lds_st = st
-        if plan.n_big and not torch.cuda.is_current_stream_capturing():
-            cur = torch.cuda.current_stream(data.device)
-            side = _side_stream(data.device)
-            side.wait_stream(cur)
-            lds_st = side.cuda_stream
-            joined = (cur, side)
-        if mode == 0:
-            L.call('yastn_hip_svd', ptr(out_a), ptr(out_s), ptr(out_b), ptr(data), dt, plan.d_blocks.data_ptr(),
-                   plan.n_lds, plan.d_order.data_ptr(), plan.n_lds, plan.lds_bytes, ptr(work), ptr(info),
-                   MAX_SWEEPS, lds_st)
-        else:
-            L.call('yastn_hip_eigh', ptr(out_s), ptr(out_a), ptr(data), dt, plan.d_blocks.data_ptr(), plan.n_lds,
-                   plan.d_order.data_ptr(), plan.n_lds, plan.lds_bytes, ptr(work), ptr(info), MAX_SWEEPS, lds_st)
+    joined, lds_st = None, st
+    if plan.n_big and (plan.n_small or plan.n_lds) and not torch.cuda.is_current_stream_capturing():
+        # the one-workgroup kernels (small blocks) run on a side stream, overlapping the panel path of the
+        # large blocks, which occupies only part of the GPU; joined below
+        cur = torch.cuda.current_stream(data.device)
+        side = _side_stream(data.device)
+        side.wait_stream(cur)
+        lds_st = side.cuda_stream
+        joined = (cur, side)
     try:
+        order = plan.d_order.data_ptr()
+        if plan.n_small:
+            L.call('yastn_hip_jacobi_small', ptr(out_a), ptr(out_s), ptr(out_b), ptr(data), dt, mode,
+                   plan.d_blocks.data_ptr(), order, plan.n_small, plan.small_bytes, ptr(info), MAX_SWEEPS, lds_st)
+        order += plan.n_small * plan.d_order.element_size()
+        if plan.n_lds and mode == 0:
+            L.call('yastn_hip_svd', ptr(out_a), ptr(out_s), ptr(out_b), ptr(data), dt, plan.d_blocks.data_ptr(),
+                   plan.n_lds, order, plan.n_lds, plan.lds_bytes, ptr(work), ptr(info), MAX_SWEEPS, lds_st)
+        elif plan.n_lds:
+            L.call('yastn_hip_eigh', ptr(out_s), ptr(out_a), ptr(data), dt, plan.d_blocks.data_ptr(), plan.n_lds,
+                   order, plan.n_lds, plan.lds_bytes, ptr(work), ptr(info), MAX_SWEEPS, lds_st)
         if plan.n_big:
             mu = torch.empty(plan.nblocks, dtype=torch.float64, device=data.device)
             floors = torch.empty(plan.nblocks, dtype=torch.float64, device=data.device)

@@ -12,7 +12,7 @@ LIB_PATH = os.environ.get('YASTN_HIP_LIB', os.path.join(HERE, 'libyastn_hip.so')
 # constants mirrored from include/yastn_hip.h
 YH_OK, YH_ERR_ARG, YH_ERR_HIP, YH_ERR_NUMERIC = 0, -1, -2, -3
 YH_F64, YH_C128 = 0, 1
-YH_ABI_VERSION = 13
+YH_ABI_VERSION = 14
 YH_MAXR = 8
 YH_JOB_WORDS = 32
 YH_JOB_BUFFER_WORD = 30
@@ -29,6 +29,7 @@ TILE_DIMS = {YH_TILE_32x32: (32, 32), YH_TILE_64x64: (64, 64), YH_TILE_128x64: (
              YH_TILE_SMALLM: (16, 256), YH_TILE_RD32: (32, 32)}
 YH_SVD_WORDS = 8
 YH_SVD_MAX_Q = 2048
+YH_SMALL_Q = 32
 YH_QR_WORDS = 8
 YH_SPLITK_WORDS = 8
 YH_QR_NB = 32
@@ -70,6 +71,8 @@ _SIGS = {
     'yastn_hip_check_svd_plan': [_p, _i64, _p, _i64, _i64, _i32, _i32, _i64, _i64, _i64, _i64, _i64],
     'yastn_hip_svd': [_p, _p, _p, _p, _i32, _p, _i64, _p, _i64, _i64, _p, _p, _i32, _p],
     'yastn_hip_eigh': [_p, _p, _p, _i32, _p, _i64, _p, _i64, _i64, _p, _p, _i32, _p],
+    'yastn_hip_check_small_plan': [_p, _i64, _p, _i64, _i32, _i32, _i64],
+    'yastn_hip_jacobi_small': [_p, _p, _p, _p, _i32, _i32, _p, _p, _i64, _i64, _p, _i32, _p],
     'yastn_hip_fix_svd_signs': [_p, _p, _i32, _p, _i64, _p],
     'yastn_hip_device_info': [_p, _p],
     'yastn_hip_svd_panel_init': [_p, _p, _p, _p, _i32, _i32, _p, _p, _i64, _p],

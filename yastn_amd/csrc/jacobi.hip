@@ -55,6 +55,12 @@ struct Num<true> {
   static __device__ inline double abs2(double2 x) { return x.x * x.x + x.y * x.y; }
 };
 
+// c ? a : b by components (the conditional operator on two double2 objects selects between their addresses).
+__device__ __attribute__((always_inline)) inline double pick(bool c, double a, double b) { return c ? a : b; }
+__device__ __attribute__((always_inline)) inline double2 pick(bool c, double2 a, double2 b) {
+  return make_double2(c ? a.x : b.x, c ? a.y : b.y);
+}
+
 // Wave-wide reductions: DPP moves within each row of 16 lanes (quad_perm [1,0,3,2], quad_perm
 // [2,3,0,1], row_half_mirror, row_mirror: after the four steps every lane holds its row's value),
 // then the four row values are read into scalar registers, so the result is wave-uniform.
@@ -1193,8 +1199,8 @@ __global__ void __launch_bounds__(kPairThreads)
       }
       const T un = row_prev(u0), vp = row_prev(v0), vn = row_next(v0);  // of lanes l - 1, l - 1, l + 1
       const T u = u0;
-      u0 = l8 == 0 ? u : l8 == 1 ? vp : un;
-      v0 = l8 == 7 ? u : vn;
+      u0 = pick(l8 == 0, u, pick(l8 == 1, vp, un));
+      v0 = pick(l8 == 7, u, vn);
     }
     if (any) {
       const T zero = N::make(0.0, 0.0);
@@ -1253,6 +1259,279 @@ __global__ void __launch_bounds__(kPairThreads)
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Small blocks (q <= 32): the whole decomposition of a block in one workgroup of 256 threads and one launch.  W (p x q)
+// and V (q x q) stay in LDS, column-major with odd leading dimensions.  A sweep forms the Gram matrix of all q columns
+// on the matrix cores, runs one sweep of rotations on it (the circle order of 2 E = 16 or 32 columns, thread (k, l)
+// owning the 2 x 2 block of slots k and l as in panel_pair_kernel), and multiplies W and V by the accumulated
+// rotation on the matrix cores; it stops when a sweep rotates nothing.  Like the panel path and unlike jacobi_kernel,
+// a rotation costs no pass over the columns: a sweep of 32 columns takes 31 sub-rounds of about 0.4 us.
+// Kernel time, one block (jacobi_kernel in brackets): 16 x 16 64 us (91), 32 x 32 161 us (440).
+// sweeps each wait for the host; past 32 columns the panel path's several workgroups win.
+constexpr int kSmallQ = YH_SMALL_Q, kSmallThreads = 256;
+
+// LDS elements of a block: W, V and the two exchange buffers (the accumulated rotation overlays them).
+__host__ __device__ inline int64_t small_elems(int64_t p, int64_t q) {
+  const int64_t h = q <= 16 ? 16 : 32;
+  return (p | 1) * q + (q | 1) * q + 2 * h * (h + 1);
+}
+
+template <bool CPLX, int MODE, int E>
+__device__ __attribute__((always_inline)) inline void small_block(
+    const BlockDesc& d, const typename Num<CPLX>::T* __restrict__ A_, typename Num<CPLX>::T* __restrict__ U,
+    double* __restrict__ S, typename Num<CPLX>::T* __restrict__ Vh, int32_t* __restrict__ info, int max_sweeps) {
+  typedef Num<CPLX> N;
+  typedef typename N::T T;
+  constexpr int H = 2 * E, nq = H + 1, kWavesS = kSmallThreads / 64, TT = H / 16;
+  extern __shared__ double smem_raw[];
+  __shared__ double s_red[kWavesS], s_sig[kSmallQ];
+  __shared__ int s_col[kSmallQ];  // column of rank r
+  const bool tr = (MODE == 0) && (d.m < d.n);
+  const int p = (int)(tr ? d.n : d.m), q = (int)(tr ? d.m : d.n);
+  const int ldw = p | 1, ldv = q | 1;
+  T* W = reinterpret_cast<T*>(smem_raw);
+  T* V = W + ldw * q;
+  typedef T Plane[H][nq];
+  Plane* X = reinterpret_cast<Plane*>(V + ldv * q);
+  T* Q = reinterpret_cast<T*>(X);  // column c at Q + c nq
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int k = tid >> 4, l = tid & 15, ke = k & (E - 1), le = l & (E - 1);
+  const T zero = N::make(0.0, 0.0), one = N::make(1.0, 0.0);
+  auto total = [&](double v) {  // sum over the workgroup, in wave order
+    v = wave_sum(v);
+    __syncthreads();
+    if (lane == 0) s_red[wave] = v;
+    __syncthreads();
+    double t = 0.0;
+    for (int w = 0; w < kWavesS; ++w) t += s_red[w];
+    return t;
+  };
+  // ---- W = A (or A^H when m < n), read in A's order, and V = I
+  for (int e = tid; e < p * q; e += kSmallThreads) {
+    if (tr) {
+      const int c = e / p, r = e - c * p;
+      W[c * ldw + r] = N::conj(A_[d.a_off + e]);
+    } else {
+      const int r = e / q, c = e - r * q;
+      W[c * ldw + r] = A_[d.a_off + e];
+    }
+  }
+  for (int e = tid; e < ldv * q; e += kSmallThreads) V[e] = N::make(e % (ldv + 1) == 0 ? 1.0 : 0.0, 0.0);
+  __syncthreads();
+  double mu = 0.0;
+  if (MODE == 1) {  // Gershgorin bound, added to the diagonal
+    double row = 0.0;
+    if (tid < q)
+      for (int c = 0; c < q; ++c) row += sqrt(N::abs2(W[c * ldw + tid]));
+    row = wave_max(row);  // q <= 64: all rows in wave 0
+    if (tid == 0) s_red[0] = row;
+    __syncthreads();
+    mu = s_red[0];
+    if (tid < q) {
+      const T x = W[tid * ldw + tid];
+      W[tid * ldw + tid] = N::make(N::re(x) + mu, N::im(x));
+    }
+    __syncthreads();
+  }
+  const double tol = DBL_EPSILON * sqrt((double)(p > 1 ? p : 1)), tol2 = tol * tol;
+  double f = 0.0;
+  for (int c = wave; c < q; c += kWavesS)
+    for (int r = lane; r < p; r += 64) f += N::abs2(W[c * ldw + r]);
+  const double floor2 = DBL_EPSILON * DBL_EPSILON * total(f);
+  auto from_top = [](int i) { return i == 0 ? 0 : i == 1 ? E : i - 1; };
+  auto from_bot = [](int i) { return i == E - 1 ? E - 1 : E + 1 + i; };
+  int sweeps = 0;
+  bool converged = q <= 1;
+  while (!converged && sweeps < max_sweeps) {
+    // ---- G = W^H W, upper 16 x 16 tiles, one per wave; columns past q are zero
+    {
+      const int ti = wave == 2 ? 1 : 0, tj = wave == 0 ? 0 : 1;
+      if (wave < TT * (TT + 1) / 2) {
+        const int ca = 16 * ti + (lane & 15), cb = 16 * tj + (lane & 15);
+        const bool oka = ca < q, okb = cb < q;
+        const T* wa = W + (oka ? ca : 0) * ldw;
+        const T* wb = W + (okb ? cb : 0) * ldw;
+        d4 accR = {0.0, 0.0, 0.0, 0.0}, accI = {0.0, 0.0, 0.0, 0.0};
+        for (int r0 = 0; r0 < p; r0 += 4) {
+          const int r = r0 + (lane >> 4), rc = r < p ? r : 0;
+          const T xa = wa[rc], xb = wb[rc];
+          const T a = pick(oka & (r < p), xa, zero), b = pick(okb & (r < p), xb, zero);
+          accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(a), N::re(b), accR, 0, 0, 0);
+          if constexpr (CPLX) {  // conj(a) b
+            accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::im(a), N::im(b), accR, 0, 0, 0);
+            accI = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(a), N::im(b), accI, 0, 0, 0);
+            accI = __builtin_amdgcn_mfma_f64_16x16x4f64(-N::im(a), N::re(b), accI, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = 16 * ti + (lane >> 4) + 4 * v, j = 16 * tj + (lane & 15);
+          X[0][i][j] = N::make(accR[v], accI[v]);
+          if (ti != tj) X[0][j][i] = N::make(accR[v], -accI[v]);
+        }
+      }
+    }
+    __syncthreads();
+    // ---- one sweep of rotations on G: a ring of H - 1 places, E slots
+    T u0 = pick(k == le, one, zero), v0 = pick(k == le + E, one, zero);   // Q(k, top le), Q(k, bottom le)
+    T u1 = zero, v1 = pick(E == 16 && k == le, one, zero);                // rows k + 16 (E = 16)
+    bool any = false;
+#pragma unroll 1
+    for (int s = 0; s < H - 1; ++s) {
+      const int w = s & 1;
+      const int rt = s ? from_top(ke) : ke, rb = s ? from_bot(ke) : ke + E;
+      const int ct = s ? from_top(le) : le, cb = s ? from_bot(le) : le + E;
+      const T gl = X[w][ct][cb];
+      const double al = N::re(X[w][ct][ct]), bl = N::re(X[w][cb][cb]);
+      T A = X[w][rt][ct], C = X[w][rt][cb], D = X[w][rb][ct], B = X[w][rb][cb];
+      double cl, srl, sil;
+      const bool go = rotation_short<CPLX>(al, bl, N::re(gl), N::im(gl), tol2, floor2, cl, srl, sil);
+      if (__any(go)) {
+        any = true;
+        const int src = (lane & 48) + ke;
+        const double ck = __shfl(cl, src), srk = __shfl(srl, src), sik = CPLX ? __shfl(sil, src) : 0.0;
+        apply_rot<CPLX>(A, D, ck, 1.0, srk, -sik);
+        apply_rot<CPLX>(C, B, ck, 1.0, srk, -sik);
+        apply_rot<CPLX>(A, C, cl, 1.0, srl, sil);
+        apply_rot<CPLX>(D, B, cl, 1.0, srl, sil);
+        apply_rot<CPLX>(u0, v0, cl, 1.0, srl, sil);
+        if (E == 16) apply_rot<CPLX>(u1, v1, cl, 1.0, srl, sil);
+      }
+      if (s + 2 < H) {
+        if (k < E && l < E) {
+          X[w ^ 1][k][l] = A;
+          X[w ^ 1][k][l + E] = C;
+          X[w ^ 1][k + E][l] = D;
+          X[w ^ 1][k + E][l + E] = B;
+        }
+        __syncthreads();
+      }
+      {
+        const T up = row_prev(u0), vp = row_prev(v0), vn = row_next(v0);
+        v0 = pick(le == E - 1, u0, vn);
+        u0 = pick(le == 0, u0, pick(le == 1, vp, up));
+      }
+      if (E == 16) {
+        const T up = row_prev(u1), vp = row_prev(v1), vn = row_next(v1);
+        v1 = pick(le == E - 1, u1, vn);
+        u1 = pick(le == 0, u1, pick(le == 1, vp, up));
+      }
+    }
+    ++sweeps;
+    if (!any) {  // the same in every wave
+      converged = true;
+      break;
+    }
+    __syncthreads();
+    if (l < E) {
+      Q[l * nq + k] = u0;
+      Q[(l + E) * nq + k] = v0;
+      if (E == 16) {
+        Q[l * nq + k + 16] = u1;
+        Q[(l + E) * nq + k + 16] = v1;
+      }
+    }
+    __syncthreads();
+    // ---- W <- W Q, V <- V Q: 16-row stripes, as Q^T X^T (a wave reads its whole stripe before writing it)
+    const int sw = (p + 15) / 16, sv = (q + 15) / 16;
+    for (int st = wave; st < sw + sv; st += kWavesS) {
+      T* M = st >= sw ? V : W;
+      const int ld = st >= sw ? ldv : ldw, rows = st >= sw ? q : p;
+      const int row = (st >= sw ? st - sw : st) * 16 + (lane & 15);
+      constexpr int KS = H / 4;
+      T x[KS];
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const int c = 4 * i + (lane >> 4);
+        const bool ok = (c < q) & (row < rows);
+        const T v = M[ok ? c * ld + row : 0];
+        x[i] = pick(ok, v, zero);
+      }
+#pragma unroll
+      for (int tj = 0; tj < TT; ++tj) {
+        d4 accR = {0.0, 0.0, 0.0, 0.0}, accI = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+          const T b = Q[(tj * 16 + (lane & 15)) * nq + 4 * i + (lane >> 4)];
+          accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(b), N::re(x[i]), accR, 0, 0, 0);
+          if constexpr (CPLX) {
+            accI = __builtin_amdgcn_mfma_f64_16x16x4f64(N::im(b), N::re(x[i]), accI, 0, 0, 0);
+            accR = __builtin_amdgcn_mfma_f64_16x16x4f64(-N::im(b), N::im(x[i]), accR, 0, 0, 0);
+            accI = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(b), N::im(x[i]), accI, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int c = tj * 16 + (lane >> 4) + 4 * v;
+          if (row < rows && c < q) M[c * ld + row] = N::make(accR[v], accI[v]);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  // ---- sigma_j = ||w_j||, ranks (descending, ties by index), vectors in the outputs' order
+  for (int c = wave; c < q; c += kWavesS) {
+    double a = 0.0;
+    for (int r = lane; r < p; r += 64) a += N::abs2(W[c * ldw + r]);
+    a = wave_sum(a);
+    if (lane == 0) s_sig[c] = sqrt(a);
+  }
+  __syncthreads();
+  if (tid < q) {
+    const double sj = s_sig[tid];
+    int rk = 0;
+    for (int i = 0; i < q; ++i) rk += (s_sig[i] > sj) || (s_sig[i] == sj && i < tid);
+    const int pos = MODE == 1 ? q - 1 - rk : rk;
+    s_col[pos] = tid;
+    S[d.s_off + pos] = MODE == 1 ? sj - mu : sj;
+  }
+  __syncthreads();
+  if (MODE == 1) {
+    for (int e = tid; e < q * q; e += kSmallThreads) {
+      const int r = e / q, pos = e - r * q;
+      U[d.u_off + e] = V[s_col[pos] * ldv + r];
+    }
+  } else {
+    // m >= n: U = W Sigma^-1 (p x q), Vh = V^H (q x q); m < n: U = V (q x q), Vh = (W Sigma^-1)^H (q x p)
+    for (int e = tid; e < (tr ? q : p) * q; e += kSmallThreads) {
+      const int r = e / q, pos = e - r * q, j = s_col[pos];
+      if (tr) {
+        U[d.u_off + e] = V[j * ldv + r];
+      } else {
+        const double sj = s_sig[j], inv = sj > 0.0 ? 1.0 / sj : 0.0;
+        const T w = W[j * ldw + r];
+        U[d.u_off + e] = N::make(N::re(w) * inv, N::im(w) * inv);
+      }
+    }
+    const int len = tr ? p : q;
+    for (int e = tid; e < q * len; e += kSmallThreads) {
+      const int pos = e / len, c = e - pos * len, j = s_col[pos];
+      if (tr) {
+        const double sj = s_sig[j], inv = sj > 0.0 ? 1.0 / sj : 0.0;
+        const T w = W[j * ldw + c];
+        Vh[d.v_off + e] = N::make(N::re(w) * inv, -N::im(w) * inv);
+      } else {
+        Vh[d.v_off + e] = N::conj(V[j * ldv + c]);
+      }
+    }
+  }
+  if (tid == 0) *info = converged ? sweeps : -1;
+}
+
+template <bool CPLX, int MODE>
+__global__ void __launch_bounds__(kSmallThreads)
+    small_kernel(const int64_t* __restrict__ blocks, const int32_t* __restrict__ order,
+                 const typename Num<CPLX>::T* __restrict__ A, typename Num<CPLX>::T* __restrict__ U,
+                 double* __restrict__ S, typename Num<CPLX>::T* __restrict__ Vh, int32_t* __restrict__ info,
+                 int max_sweeps) {
+  const int bidx = order[blockIdx.x];
+  const BlockDesc d = load_desc(blocks + (int64_t)bidx * YH_SVD_WORDS);
+  if (min(d.m, d.n) <= 16)
+    small_block<CPLX, MODE, 8>(d, A, U, S, Vh, info + bidx, max_sweeps);
+  else
+    small_block<CPLX, MODE, 16>(d, A, U, S, Vh, info + bidx, max_sweeps);
 }
 
 // Sweep count from the per-sweep rotation flags: the first sweep that rotated nothing ends the
@@ -2128,6 +2407,58 @@ extern "C" int yastn_hip_eigh(void* S, void* U, const void* A, int dtype, const 
                                                    work, d_info, max_sweeps, stream)
                          : launch_jacobi<true, 1>(d_blocks, d_order, n_lds, lds_bytes, nblocks, A, U, S, nullptr,
                                                   work, d_info, max_sweeps, stream);
+}
+
+extern "C" int yastn_hip_check_small_plan(const int64_t* h_blocks, int64_t nblocks, const int32_t* h_order, int64_t n,
+                                          int mode, int dtype, int64_t lds_bytes) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  YH_CHECK_ARG(mode == 0 || mode == 1, "mode %d", mode);
+  YH_CHECK_ARG(n >= 0 && n <= nblocks, "small blocks %lld of %lld", (long long)n, (long long)nblocks);
+  for (int64_t o = 0; o < n; ++o) {
+    const int32_t b = h_order[o];
+    YH_CHECK_ARG(b >= 0 && b < nblocks, "order[%lld] = %d", (long long)o, b);
+    const int64_t bm = h_blocks[b * YH_SVD_WORDS + 1], bn = h_blocks[b * YH_SVD_WORDS + 2];
+    const int64_t p = bm < bn ? bn : bm, q = bm < bn ? bm : bn;
+    YH_CHECK_ARG(q >= 1 && q <= kSmallQ && p <= ((int64_t)1 << 20), "small block %d: %lld x %lld", b, (long long)bm,
+                 (long long)bn);
+    YH_CHECK_ARG(small_elems(p, q) * yh::itemsize_of(dtype) <= lds_bytes, "small block %d exceeds the LDS of %lld bytes",
+                 b, (long long)lds_bytes);
+  }
+  return YH_OK;
+}
+
+namespace {
+
+template <bool CPLX, int MODE>
+int launch_small(const int64_t* d_blocks, const int32_t* d_order, int64_t n, int64_t lds_bytes, const void* A, void* U,
+                 void* S, void* Vh, int32_t* info, int max_sweeps, hipStream_t stream) {
+  typedef typename Num<CPLX>::T T;
+  int st = yh::hip_status(hipFuncSetAttribute((const void*)small_kernel<CPLX, MODE>,
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes),
+                          "small block LDS size");
+  if (st) return st;
+  hipLaunchKernelGGL((small_kernel<CPLX, MODE>), dim3((unsigned)n), dim3(kSmallThreads), (size_t)lds_bytes, stream,
+                     d_blocks, d_order, (const T*)A, (T*)U, (double*)S, (T*)Vh, info, max_sweeps);
+  st = yh::hip_status(hipGetLastError(), "small block launch");
+  if (st || MODE == 1) return st;
+  return launch_complete<CPLX>(d_blocks, d_order, n, U, S, Vh, stream);
+}
+
+}  // namespace
+
+extern "C" int yastn_hip_jacobi_small(void* U, void* S, void* Vh, const void* A, int dtype, int mode,
+                                      const int64_t* d_blocks, const int32_t* d_order, int64_t n, int64_t lds_bytes,
+                                      int32_t* d_info, int max_sweeps, hipStream_t stream) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  YH_CHECK_ARG(mode == 0 || mode == 1, "mode %d", mode);
+  YH_CHECK_ARG(n >= 0 && n <= INT32_MAX && lds_bytes >= 0 && lds_bytes <= 160 * 1024, "small blocks %lld, LDS %lld",
+               (long long)n, (long long)lds_bytes);
+  if (n == 0) return YH_OK;
+  if (dtype == YH_F64)
+    return mode == 0 ? launch_small<false, 0>(d_blocks, d_order, n, lds_bytes, A, U, S, Vh, d_info, max_sweeps, stream)
+                     : launch_small<false, 1>(d_blocks, d_order, n, lds_bytes, A, U, S, Vh, d_info, max_sweeps, stream);
+  return mode == 0 ? launch_small<true, 0>(d_blocks, d_order, n, lds_bytes, A, U, S, Vh, d_info, max_sweeps, stream)
+                   : launch_small<true, 1>(d_blocks, d_order, n, lds_bytes, A, U, S, Vh, d_info, max_sweeps, stream);
 }
 
 extern "C" int yastn_hip_device_info(int* lds_per_block, int* num_cu) {

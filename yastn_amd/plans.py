@@ -705,9 +705,12 @@ def _circle_pair(ne, r, k):
 
 
 PRECOND = True  # QR-precondition the panel path of SVD blocks (off: plain one-sided Jacobi on W0)
-# SVD blocks with more columns than this take the QR-preconditioned panel path even where they fit the
-# LDS kernel, whose unpreconditioned sweeps on one workgroup outlast the panel rounds past this size.
-SVD_LDS_MAX_Q = int(os.environ.get('YASTN_HIP_SVD_LDS_MAX_Q', '16'))
+# Blocks with more columns than this take the panel path (SVD blocks QR-preconditioned) even where they fit one
+# workgroup, whose sweeps outlast the panel rounds past this size.  Up to 32 columns the one-workgroup kernel is
+# yastn_hip_jacobi_small; larger caps send blocks of more columns to yastn_hip_svd / yastn_hip_eigh.
+# Measured, 25 Hermitian blocks of 1 ... 106 columns (eigh): cap 128 4.94 ms, 48 2.73, 32 2.12, 16 2.22.
+SVD_LDS_MAX_Q = int(os.environ.get('YASTN_HIP_SVD_LDS_MAX_Q', '32'))
+EIGH_LDS_MAX_Q = int(os.environ.get('YASTN_HIP_EIGH_LDS_MAX_Q', '32'))
 # Panel width b of the panel Jacobi (a workgroup rotates 2b columns per round): smaller panels give more
 # workgroups per round but more rounds per sweep.  Tuning knob; the LDS limit may lower it further.
 PANEL_WIDTH = int(os.environ.get('YASTN_HIP_PANEL_WIDTH', '16'))
@@ -741,8 +744,8 @@ def panel_slices(cross, stripes, cplx, width):
 class SvdPlan:
     """Block list of the batched Jacobi SVD / eigh.
 
-    Blocks whose working matrices (W and V, (p q + q^2) elements) fit the LDS limit run in the
-    LDS-resident kernel, one workgroup per block, all in one launch.  Larger blocks use the panel
+    Blocks of few columns whose working matrices (W and V, (p q + q^2) elements) fit the LDS limit run in
+    an LDS-resident kernel, one workgroup per block, all in one launch.  Larger blocks use the panel
     path: W and V in a workspace, panels of width b, one launch per round of panel pairs.  For SVD
     blocks the panel path first factors W0 = Q R (blocked Householder QR: a panel kernel plus three
     grouped GEMMs per step; the p x YH_QR_NB panel is staged in LDS when every block's fits, else
@@ -753,9 +756,9 @@ class SvdPlan:
     def __init__(self, blocks, itemsize, mode, a_numel, u_numel, s_numel, v_numel, device):
         # blocks: list of (a_off, m, n, u_off, s_off, v_off)
         NB = L.YH_QR_NB
-        words, small, big, pre = [], [], [], []
+        words, small, lds, big, pre = [], [], [], [], []
         work = 0
-        lds_bytes = 0
+        lds_bytes = small_bytes = 0
         dev_lds = L.device_lds_per_block()
         # the LDS kernel also holds ~8 KiB of static shared memory
         lds_limit = min(L.YH_SVD_LDS_BYTES, dev_lds - 9 * 1024)
@@ -766,8 +769,16 @@ class SvdPlan:
             p, q = (n, m) if tr else (m, n)
             need = p * q + q * q
             jw = None
-            if need * itemsize <= lds_limit and not (mode == 0 and PRECOND and q > SVD_LDS_MAX_Q):
+            cap = EIGH_LDS_MAX_Q if mode == 1 else SVD_LDS_MAX_Q if PRECOND else q
+            h = 16 if q <= 16 else 32
+            need_small = ((p | 1) * q + (q | 1) * q + 2 * h * (h + 1)) * itemsize
+            if q <= min(cap, L.YH_SMALL_Q) and need_small <= dev_lds - 2048 and need * itemsize <= lds_limit:
                 small.append(b)
+                small_bytes = max(small_bytes, need_small)
+                lds_bytes = max(lds_bytes, need * itemsize)
+                w_off = 0
+            elif L.YH_SMALL_Q < q <= cap and need * itemsize <= lds_limit:
+                lds.append(b)
                 lds_bytes = max(lds_bytes, need * itemsize)
                 w_off = 0
             elif mode == 0 and PRECOND:
@@ -790,15 +801,19 @@ class SvdPlan:
             jwords.append(jw if jw is not None else words[-1])
         size = lambda b: blocks[b][1] * blocks[b][2] * min(blocks[b][1], blocks[b][2])
         small.sort(key=lambda b: -size(b))
+        lds.sort(key=lambda b: -size(b))
         big.sort(key=lambda b: -size(b))
         self.h_blocks = np.ascontiguousarray(np.array(words, dtype=np.int64).reshape(-1, L.YH_SVD_WORDS))
-        self.h_order = np.ascontiguousarray(np.array(small + big, dtype=np.int32))
-        self.nblocks, self.n_lds, self.lds_bytes, self.work_numel = len(words), len(small), lds_bytes, work
+        self.h_order = np.ascontiguousarray(np.array(small + lds + big, dtype=np.int32))
+        self.n_small, self.small_bytes, self.n_lds = len(small), small_bytes, len(lds)
+        self.nblocks, self.lds_bytes, self.work_numel = len(words), lds_bytes, work
         self.flops = sum(4 * m * n * min(m, n) + 8 * min(m, n) ** 3 for (_, m, n, *_r) in blocks)
         dt = L.YH_C128 if itemsize == 16 else L.YH_F64
         self.dt = dt
         L.call('yastn_hip_check_svd_plan', self.h_blocks.ctypes.data, self.nblocks, self.h_order.ctypes.data,
-               self.n_lds, self.lds_bytes, mode, dt, a_numel, u_numel, s_numel, v_numel, max(work, 0))
+               self.n_small + self.n_lds, self.lds_bytes, mode, dt, a_numel, u_numel, s_numel, v_numel, max(work, 0))
+        L.call('yastn_hip_check_small_plan', self.h_blocks.ctypes.data, self.nblocks, self.h_order.ctypes.data,
+               self.n_small, mode, dt, self.small_bytes)
         self.d_blocks = torch.from_numpy(self.h_blocks).to(device)
         self.d_order = torch.from_numpy(self.h_order).to(device)
         # panel path
@@ -810,7 +825,8 @@ class SvdPlan:
             if pre:
                 # the Jacobi stage of the preconditioned blocks works on X (q x q) in its own workspace
                 L.call('yastn_hip_check_svd_plan', self.h_jblocks.ctypes.data, self.nblocks,
-                       self.h_order.ctypes.data, 0, 0, mode, dt, a_numel, u_numel, s_numel, v_numel, max(work, 0))
+                       self.h_order.ctypes.data, self.n_small + self.n_lds, self.lds_bytes, mode, dt, a_numel, u_numel,
+                       s_numel, v_numel, max(work, 0))
             self.d_jblocks = torch.from_numpy(self.h_jblocks).to(device)
             limit = dev_lds - 2048
             width = max(1, min(PANEL_WIDTH, 32))
