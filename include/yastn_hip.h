@@ -35,7 +35,7 @@ extern "C" {
 #define YH_F64 0
 #define YH_C128 1
 
-#define YH_ABI_VERSION 14
+#define YH_ABI_VERSION 15
 
 /* ---- box-gather plan (one job per copied or zero-filled box) -------------
  * int64 words per job (YH_JOB_WORDS):
@@ -278,13 +278,18 @@ int yastn_hip_check_qr_plan(const int64_t* h_qdesc, const int64_t* h_blocks, con
  * lds_bytes >= p*YH_QR_NB*itemsize for every block, in place in the workspace when lds_bytes == 0. */
 int yastn_hip_svd_qr_panel(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, int step,
                            int64_t lds_bytes, hipStream_t stream);
+/* W0 = A (or A^H when m < n) and floors[b] = eps^2 ||A||_F^2 of the preconditioned blocks (for them in place of
+ * yastn_hip_svd_panel_init; the scratch at y_off, at least 64 elements, is used and left undefined). */
+int yastn_hip_svd_precond_load(const void* A, void* work, double* floors, int dtype, const int64_t* d_blocks,
+                               const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, hipStream_t stream);
 /* X = R^H, V_J = I. */
 int yastn_hip_svd_precond_init(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n,
                                hipStream_t stream);
 /* sigma, sorted; q-side vectors x_j / sigma_j (completed where sigma is at the noise level); p-side
  * vectors initialised to [V_J; 0] (U for m >= n, conjugated rows of Vh for m < n), to be multiplied
- * by Q.  d_blocks are the block's SVD words (original m, n and output offsets). */
-int yastn_hip_svd_precond_finalize(void* U, void* S, void* Vh, const void* work, int dtype, const int64_t* d_blocks,
+ * by Q.  d_blocks are the block's SVD words (original m, n and output offsets).  Overwrites the scratch at
+ * y_off. */
+int yastn_hip_svd_precond_finalize(void* U, void* S, void* Vh, void* work, int dtype, const int64_t* d_blocks,
                                    const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, int32_t* d_info,
                                    int sweeps, const int32_t* d_sweeps, hipStream_t stream);
 

@@ -618,9 +618,12 @@ def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
         if plan.n_big:
             mu = torch.empty(plan.nblocks, dtype=torch.float64, device=data.device)
             floors = torch.empty(plan.nblocks, dtype=torch.float64, device=data.device)
-            L.call('yastn_hip_svd_panel_init', ptr(data), ptr(work), ptr(mu), ptr(floors), dt, mode,
-                   plan.d_blocks.data_ptr(), plan.d_big.data_ptr(), plan.n_big, st)
+            if plan.n_plain:
+                L.call('yastn_hip_svd_panel_init', ptr(data), ptr(work), ptr(mu), ptr(floors), dt, mode,
+                       plan.d_blocks.data_ptr(), plan.d_plain.data_ptr(), plan.n_plain, st)
             if plan.n_pre:
+                L.call('yastn_hip_svd_precond_load', ptr(data), ptr(work), ptr(floors), dt, plan.d_blocks.data_ptr(),
+                       plan.d_qdesc.data_ptr(), plan.d_pre.data_ptr(), plan.n_pre, st)
                 # W0 = Q R (Householder, one panel kernel and three grouped GEMMs per step), then X = R^H
                 for step, (d_ids, n, trail) in enumerate(plan.qr_steps):
                     L.call('yastn_hip_svd_qr_panel', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step,

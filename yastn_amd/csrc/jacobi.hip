@@ -303,13 +303,10 @@ __device__ inline BlockDesc load_desc(const int64_t* w) {
 
 // Column norms -> singular values (descending, ties by index), vectors written by whole waves.
 // sigma_j is staged in the block's S slice; the ranks are kept in LDS.
-// MODE 2 is the QR-preconditioned SVD: W = X (q x q, p == q here), V = V_J, and pf is the long
-// dimension of the block; the q-side vectors x_j / sigma_j go to Vh (m >= n) or U (m < n) and the
-// p-side vectors start as [v_j; 0] in the other output, to be multiplied by Q afterwards.
 template <bool CPLX, int MODE>
 __device__ void finalize_block(const BlockDesc& d, const typename Num<CPLX>::T* W, const typename Num<CPLX>::T* V,
                                int64_t p, int64_t q, bool tr, double mu, typename Num<CPLX>::T* __restrict__ U,
-                               double* __restrict__ S, typename Num<CPLX>::T* __restrict__ Vh, int64_t pf = 0) {
+                               double* __restrict__ S, typename Num<CPLX>::T* __restrict__ Vh) {
   typedef Num<CPLX> N;
   typedef typename N::T T;
   __shared__ int s_rank_of[YH_SVD_MAX_Q];
@@ -353,21 +350,6 @@ __device__ void finalize_block(const BlockDesc& d, const typename Num<CPLX>::T* 
     if (MODE == 1) {
       const int64_t pos = q - 1 - rkj;
       for (int64_t x = lane; x < q; x += 64) U[d.u_off + x * q + pos] = vj[x];
-    } else if (MODE == 2) {
-      const double inv = sj > 0.0 ? 1.0 / sj : 0.0;
-      if (!tr) {  // W0 = A = (Q V_J) Sigma U_J^H: Vh (q x q) row rkj = u_j^H, U (pf x q) column rkj = [v_j; 0]
-        for (int64_t x = lane; x < q; x += 64) {
-          const T w = wj[x];
-          Vh[d.v_off + rkj * q + x] = N::make(N::re(w) * inv, -N::im(w) * inv);
-        }
-        for (int64_t x = lane; x < pf; x += 64) U[d.u_off + x * q + rkj] = x < q ? vj[x] : N::make(0.0, 0.0);
-      } else {  // W0 = A^H: U (q x q) column rkj = u_j, Vh (q x pf) row rkj = [v_j; 0]^H
-        for (int64_t x = lane; x < q; x += 64) {
-          const T w = wj[x];
-          U[d.u_off + x * q + rkj] = N::make(N::re(w) * inv, N::im(w) * inv);
-        }
-        for (int64_t x = lane; x < pf; x += 64) Vh[d.v_off + rkj * pf + x] = x < q ? N::conj(vj[x]) : N::make(0.0, 0.0);
-      }
     } else if (!tr) {
       // A V = W: U (m x k) column rkj = w_j / sigma_j, Vh (k x n) row rkj = v_j^H
       const double inv = sj > 0.0 ? 1.0 / sj : 0.0;
@@ -2193,40 +2175,226 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// The copies around the preconditioning (A -> W0, R^H -> X, the sorted vectors -> U, Vh) are bound by memory, so each
+// block is spread over `slices` workgroups (grid.y), which take its 32 x 32 tiles in turn; a copy between row- and
+// column-major goes through an LDS tile so that both sides are coalesced.  With one workgroup per block the three
+// took 3.7, 1.1 and 3.7 ms on 19 complex blocks of up to 1134 columns (now 0.07, 0.08 and 0.25 ms) and 49, 24 and 75 us
+// on 27 real blocks of up to 198 columns (the vectors now 7 us).
+constexpr int kTile = 32, kTileThreads = 256;
+
+// At most 64: a block's GEMM scratch holds at least 64 elements for the slices' partial sums.
+inline unsigned tile_slices(int64_t n) { return (unsigned)std::min<int64_t>(64, std::max<int64_t>(1, 2048 / n)); }
+
+// dst(j, i) = f(src(i, j)) over the tiles of an R x C matrix, src(i, j) at src + i * sld + j and dst(j, i) at
+// dst + j * dld + i: both coalesced.  f(value, i, j) may also accumulate.
+template <typename T, typename F>
+__device__ __attribute__((always_inline)) inline void transpose_tiles(T (&tile)[kTile][kTile + 1], const T* src,
+                                                                      int64_t sld, T* dst, int64_t dld, int64_t R,
+                                                                      int64_t C, F f) {
+  const int a = threadIdx.x & (kTile - 1), b = threadIdx.x / kTile;  // b: 0 .. 7
+  const int64_t nr = (R + kTile - 1) / kTile, ncl = (C + kTile - 1) / kTile;
+  for (int64_t t = blockIdx.y; t < nr * ncl; t += gridDim.y) {
+    const int64_t i0 = (t / ncl) * kTile, j0 = (t % ncl) * kTile;
+    T v[kTile / 8];
+#pragma unroll
+    for (int u = 0; u < kTile / 8; ++u) {  // all loads first; elements past the matrix read its last row / column
+      const int64_t i = i0 + b + 8 * u, j = j0 + a;
+      v[u] = src[(i < R ? i : R - 1) * sld + (j < C ? j : C - 1)];
+    }
+    __syncthreads();  // the previous tile has been written out
+#pragma unroll
+    for (int u = 0; u < kTile / 8; ++u) {
+      const int64_t i = i0 + b + 8 * u, j = j0 + a;
+      if (i < R && j < C) tile[b + 8 * u][a] = f(v[u], i, j);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kTile / 8; ++u) {
+      const int64_t j = j0 + b + 8 * u, i = i0 + a;
+      if (i < R && j < C) dst[j * dld + i] = tile[a][b + 8 * u];
+    }
+  }
+}
+
+// W0 = A (or A^H when m < n), column-major; the slice's part of ||A||_F^2 goes to element `slice` of the block's GEMM
+// scratch (y_off), which is free here.
+template <bool CPLX>
+__global__ void __launch_bounds__(kTileThreads)
+    precond_load_kernel(const int64_t* __restrict__ blocks, const int64_t* __restrict__ qdesc,
+                        const int32_t* __restrict__ ids, const typename Num<CPLX>::T* __restrict__ A,
+                        typename Num<CPLX>::T* __restrict__ work) {
+  typedef Num<CPLX> N;
+  typedef typename N::T T;
+  __shared__ T tile[kTile][kTile + 1];
+  __shared__ double s_red[kTileThreads / 64];
+  const int bidx = ids[blockIdx.x];
+  const BlockDesc d = load_desc(blocks + (int64_t)bidx * YH_SVD_WORDS);
+  const QrDesc qd = load_qr(qdesc + (int64_t)bidx * YH_QR_WORDS);
+  const T* a = A + d.a_off;
+  T* W0 = work + qd.w_off;
+  double sum = 0.0;
+  if (d.m < d.n) {  // A^H column-major is conj(A) as it lies
+    const int64_t n = d.m * d.n;
+    for (int64_t e = (int64_t)blockIdx.y * kTileThreads + threadIdx.x; e < n; e += (int64_t)gridDim.y * kTileThreads) {
+      const T v = a[e];
+      sum += N::abs2(v);
+      W0[e] = N::conj(v);
+    }
+  } else {
+    transpose_tiles(tile, a, d.n, W0, qd.p, d.m, d.n, [&](T v, int64_t, int64_t) {
+      sum += N::abs2(v);
+      return v;
+    });
+  }
+  sum = wave_sum(sum);
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < kTileThreads / 64; ++w) t += s_red[w];
+    reinterpret_cast<double*>(work + qd.y_off)[blockIdx.y] = t;
+  }
+}
+
+// floors[b] = eps^2 ||A||_F^2 from the slices' parts, summed in slice order.
+template <bool CPLX>
+__global__ void __launch_bounds__(64)
+    precond_floor_kernel(const int64_t* __restrict__ qdesc, const int32_t* __restrict__ ids, int64_t n, int slices,
+                         const typename Num<CPLX>::T* __restrict__ work, double* __restrict__ floors) {
+  const int64_t x = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (x >= n) return;
+  const QrDesc qd = load_qr(qdesc + (int64_t)ids[x] * YH_QR_WORDS);
+  const double* part = reinterpret_cast<const double*>(work + qd.y_off);
+  double t = 0.0;
+  for (int i = 0; i < slices; ++i) t += part[i];
+  floors[ids[x]] = DBL_EPSILON * DBL_EPSILON * t;
+}
+
 // X = R^H (R is the q x q upper triangle of W0) and V_J = I.
 template <bool CPLX>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kTileThreads)
     precond_init_kernel(const int64_t* __restrict__ qdesc, const int32_t* __restrict__ ids,
                         typename Num<CPLX>::T* __restrict__ work) {
   typedef Num<CPLX> N;
   typedef typename N::T T;
+  __shared__ T tile[kTile][kTile + 1];
   const QrDesc d = load_qr(qdesc + (int64_t)ids[blockIdx.x] * YH_QR_WORDS);
-  const T* W0 = work + d.w_off;
   T* X = work + d.x_off;
   T* VJ = X + d.q * d.q;
-  for (int64_t e = threadIdx.x; e < d.q * d.q; e += kThreads) {
-    const int64_t c = e / d.q, r = e - c * d.q;
-    X[e] = r >= c ? N::conj(W0[c + r * d.p]) : N::make(0.0, 0.0);
-    VJ[e] = N::make(r == c ? 1.0 : 0.0, 0.0);
+  // W0 column-major: element (r, c) of the transposed view lies at c p + r; row i of the source is column i of R
+  transpose_tiles(tile, work + d.w_off, d.p, X, d.q, d.q, d.q, [](T v, int64_t i, int64_t j) {
+    return j <= i ? N::conj(v) : N::make(0.0, 0.0);  // R(j, i), j <= i
+  });
+  const int64_t n = d.q * d.q;
+  for (int64_t e = (int64_t)blockIdx.y * kTileThreads + threadIdx.x; e < n; e += (int64_t)gridDim.y * kTileThreads)
+    VJ[e] = N::make(e % (d.q + 1) == 0 ? 1.0 : 0.0, 0.0);
+}
+
+// Finalize of the preconditioned blocks, three launches: the column norms of X (one wave per column; staged in the
+// block's GEMM scratch, which is free here), their ranks (descending, ties by index: the sorted values go to S, the
+// column of each rank to the scratch), and the vectors: with column j = col(r), x_j / sigma_j conjugated is row r of
+// Vh (m >= n) or x_j / sigma_j column r of U (m < n), and [v_j; 0] starts column r of U (m >= n) or, conjugated,
+// row r of Vh, to be multiplied by Q afterwards.
+template <bool CPLX>
+__global__ void __launch_bounds__(kTileThreads)
+    precond_norms_kernel(const int64_t* __restrict__ qdesc, const int32_t* __restrict__ ids,
+                         typename Num<CPLX>::T* __restrict__ work) {
+  typedef Num<CPLX> N;
+  typedef typename N::T T;
+  const QrDesc d = load_qr(qdesc + (int64_t)ids[blockIdx.x] * YH_QR_WORDS);
+  const T* X = work + d.x_off;
+  double* sig = reinterpret_cast<double*>(work + d.y_off);
+  const int lane = threadIdx.x & 63;
+  constexpr int kW = kTileThreads / 64;
+  for (int64_t j = (int64_t)blockIdx.y * kW + (threadIdx.x >> 6); j < d.q; j += (int64_t)gridDim.y * kW) {
+    double a = 0.0;
+    for (int64_t x = lane; x < d.q; x += 64) a += N::abs2(X[j * d.q + x]);
+    a = wave_sum(a);
+    if (lane == 0) sig[j] = sqrt(a);
   }
 }
 
-// Finalize of the preconditioned blocks: sigma, ranks, q-side vectors and the [V_J; 0] start of
-// the p-side vectors (jblocks: the Jacobi-stage descriptors, work_off = x_off, m = n = q).
 template <bool CPLX>
-__global__ void __launch_bounds__(kThreads)
-    precond_finalize_kernel(const int64_t* __restrict__ blocks, const int64_t* __restrict__ qdesc,
-                            const int32_t* __restrict__ ids, const typename Num<CPLX>::T* __restrict__ work,
-                            typename Num<CPLX>::T* __restrict__ U, double* __restrict__ S,
-                            typename Num<CPLX>::T* __restrict__ Vh, int32_t* __restrict__ info, int sweeps,
-                            const int32_t* __restrict__ d_sweeps) {
+__global__ void __launch_bounds__(kTileThreads)
+    precond_ranks_kernel(const int64_t* __restrict__ blocks, const int64_t* __restrict__ qdesc,
+                         const int32_t* __restrict__ ids, typename Num<CPLX>::T* __restrict__ work,
+                         double* __restrict__ S, int32_t* __restrict__ info, int sweeps,
+                         const int32_t* __restrict__ d_sweeps) {
+  const int bidx = ids[blockIdx.x];
+  const BlockDesc d = load_desc(blocks + (int64_t)bidx * YH_SVD_WORDS);
+  const QrDesc qd = load_qr(qdesc + (int64_t)bidx * YH_QR_WORDS);
+  const double* sig = reinterpret_cast<const double*>(work + qd.y_off);
+  int32_t* col = reinterpret_cast<int32_t*>(work + qd.y_off + qd.q);  // past the q norms
+  const int lane = threadIdx.x & 63;
+  constexpr int kW = kTileThreads / 64;
+  for (int64_t j = (int64_t)blockIdx.y * kW + (threadIdx.x >> 6); j < qd.q; j += (int64_t)gridDim.y * kW) {
+    const double sj = sig[j];
+    double cnt = 0.0;
+    for (int64_t i = lane; i < qd.q; i += 64) {
+      const double si = sig[i];
+      cnt += (si > sj) || (si == sj && i < j) ? 1.0 : 0.0;
+    }
+    const int64_t r = (int64_t)wave_sum(cnt);
+    if (lane == 0) {
+      S[d.s_off + r] = sj;
+      col[r] = (int32_t)j;
+    }
+  }
+  if (blockIdx.y == 0 && threadIdx.x == 0) info[bidx] = d_sweeps ? *d_sweeps : sweeps;
+}
+
+template <bool CPLX>
+__global__ void __launch_bounds__(kTileThreads)
+    precond_vectors_kernel(const int64_t* __restrict__ blocks, const int64_t* __restrict__ qdesc,
+                           const int32_t* __restrict__ ids, const typename Num<CPLX>::T* __restrict__ work,
+                           typename Num<CPLX>::T* __restrict__ U, const double* __restrict__ S,
+                           typename Num<CPLX>::T* __restrict__ Vh) {
+  typedef Num<CPLX> N;
+  typedef typename N::T T;
+  __shared__ T tile[kTile][kTile + 1];
   const int bidx = ids[blockIdx.x];
   const BlockDesc d = load_desc(blocks + (int64_t)bidx * YH_SVD_WORDS);
   const QrDesc qd = load_qr(qdesc + (int64_t)bidx * YH_QR_WORDS);
   const bool tr = d.m < d.n;
-  const typename Num<CPLX>::T* X = work + qd.x_off;
-  finalize_block<CPLX, 2>(d, X, X + qd.q * qd.q, qd.q, qd.q, tr, 0.0, U, S, Vh, qd.p);
-  if (threadIdx.x == 0) info[bidx] = d_sweeps ? *d_sweeps : sweeps;
+  const int64_t q = qd.q, p = qd.p;
+  const T* X = work + qd.x_off;
+  const T* VJ = X + q * q;
+  const int32_t* col = reinterpret_cast<const int32_t*>(work + qd.y_off + q);
+  const double* s = S + d.s_off;
+  // rows of Vh: m >= n the normalised columns of X (length q), m < n the columns of V_J, zero past q (length p)
+  T* rows = Vh + d.v_off;
+  const int64_t len = tr ? p : q;
+  for (int64_t e = (int64_t)blockIdx.y * kTileThreads + threadIdx.x; e < q * len;
+       e += (int64_t)gridDim.y * kTileThreads) {
+    const int64_t r = e / len, x = e - r * len, j = col[r];
+    const T v = (tr ? VJ : X)[j * q + (x < q ? x : 0)];
+    const double f = tr ? (x < q ? 1.0 : 0.0) : (s[r] > 0.0 ? 1.0 / s[r] : 0.0);
+    rows[e] = N::make(N::re(v) * f, -N::im(v) * f);
+  }
+  // columns of U: m >= n those of V_J, zero past q (p rows), m < n the normalised columns of X (q rows)
+  T* cols = U + d.u_off;
+  const int64_t R = tr ? q : p, nr = (R + kTile - 1) / kTile, ncl = (q + kTile - 1) / kTile;
+  const int a = threadIdx.x & (kTile - 1), b = threadIdx.x / kTile;
+  for (int64_t t = blockIdx.y; t < nr * ncl; t += gridDim.y) {
+    const int64_t x0 = (t / ncl) * kTile, r0 = (t % ncl) * kTile;
+    T v[kTile / 8];
+    double f[kTile / 8];
+#pragma unroll
+    for (int u = 0; u < kTile / 8; ++u) {  // a column per 32 lanes
+      const int64_t r = r0 + b + 8 * u, x = x0 + a, rc = r < q ? r : q - 1;
+      v[u] = (tr ? X : VJ)[col[rc] * q + (x < q ? x : 0)];
+      f[u] = tr ? (s[rc] > 0.0 ? 1.0 / s[rc] : 0.0) : (x < q ? 1.0 : 0.0);
+    }
+    __syncthreads();  // the previous tile has been written out
+#pragma unroll
+    for (int u = 0; u < kTile / 8; ++u) tile[b + 8 * u][a] = N::make(N::re(v[u]) * f[u], N::im(v[u]) * f[u]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kTile / 8; ++u) {
+      const int64_t x = x0 + b + 8 * u, r = r0 + a;
+      if (x < R && r < q) cols[x * q + r] = tile[a][b + 8 * u];
+    }
+  }
 }
 
 // ---- batched QR (the backend's qr): A = Q R per block, economic, diag(R) real and >= 0.
@@ -2690,36 +2858,70 @@ extern "C" int yastn_hip_svd_qr_panel(void* work, int dtype, const int64_t* d_qd
   return yh::hip_status(hipGetLastError(), "svd qr panel launch");
 }
 
+extern "C" int yastn_hip_svd_precond_load(const void* A, void* work, double* floors, int dtype,
+                                          const int64_t* d_blocks, const int64_t* d_qdesc, const int32_t* d_ids,
+                                          int64_t n, hipStream_t stream) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  YH_CHECK_ARG(n >= 0 && n <= INT32_MAX, "blocks %lld", (long long)n);
+  if (n == 0) return YH_OK;
+  const unsigned slices = tile_slices(n);
+  const dim3 g((unsigned)n, slices), gf((unsigned)yh::cdiv(n, 64));
+  if (dtype == YH_F64) {
+    hipLaunchKernelGGL(precond_load_kernel<false>, g, dim3(kTileThreads), 0, stream, d_blocks, d_qdesc, d_ids,
+                       (const double*)A, (double*)work);
+    hipLaunchKernelGGL(precond_floor_kernel<false>, gf, dim3(64), 0, stream, d_qdesc, d_ids, n, (int)slices,
+                       (const double*)work, floors);
+  } else {
+    hipLaunchKernelGGL(precond_load_kernel<true>, g, dim3(kTileThreads), 0, stream, d_blocks, d_qdesc, d_ids,
+                       (const double2*)A, (double2*)work);
+    hipLaunchKernelGGL(precond_floor_kernel<true>, gf, dim3(64), 0, stream, d_qdesc, d_ids, n, (int)slices,
+                       (const double2*)work, floors);
+  }
+  return yh::hip_status(hipGetLastError(), "svd precond load launch");
+}
+
 extern "C" int yastn_hip_svd_precond_init(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids,
                                           int64_t n, hipStream_t stream) {
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
   if (n == 0) return YH_OK;
+  const dim3 g((unsigned)n, tile_slices(n));
   if (dtype == YH_F64)
-    hipLaunchKernelGGL(precond_init_kernel<false>, dim3((unsigned)n), dim3(kThreads), 0, stream, d_qdesc, d_ids,
-                       (double*)work);
+    hipLaunchKernelGGL(precond_init_kernel<false>, g, dim3(kTileThreads), 0, stream, d_qdesc, d_ids, (double*)work);
   else
-    hipLaunchKernelGGL(precond_init_kernel<true>, dim3((unsigned)n), dim3(kThreads), 0, stream, d_qdesc, d_ids,
-                       (double2*)work);
+    hipLaunchKernelGGL(precond_init_kernel<true>, g, dim3(kTileThreads), 0, stream, d_qdesc, d_ids, (double2*)work);
   return yh::hip_status(hipGetLastError(), "svd precond init launch");
 }
 
-extern "C" int yastn_hip_svd_precond_finalize(void* U, void* S, void* Vh, const void* work, int dtype,
+namespace {
+
+template <bool CPLX>
+int launch_precond_finalize(void* U, void* S, void* Vh, void* work, const int64_t* d_blocks, const int64_t* d_qdesc,
+                            const int32_t* d_ids, int64_t n, int32_t* d_info, int sweeps, const int32_t* d_sweeps,
+                            hipStream_t stream) {
+  typedef typename Num<CPLX>::T T;
+  const dim3 g((unsigned)n, tile_slices(n)), t(kTileThreads);
+  hipLaunchKernelGGL(precond_norms_kernel<CPLX>, g, t, 0, stream, d_qdesc, d_ids, (T*)work);
+  hipLaunchKernelGGL(precond_ranks_kernel<CPLX>, g, t, 0, stream, d_blocks, d_qdesc, d_ids, (T*)work, (double*)S,
+                     d_info, sweeps, d_sweeps);
+  hipLaunchKernelGGL(precond_vectors_kernel<CPLX>, g, t, 0, stream, d_blocks, d_qdesc, d_ids, (const T*)work, (T*)U,
+                     (const double*)S, (T*)Vh);
+  const int st = yh::hip_status(hipGetLastError(), "svd precond finalize launch");
+  if (st) return st;
+  return launch_complete<CPLX>(d_blocks, d_ids, n, U, S, Vh, stream, 1);
+}
+
+}  // namespace
+
+extern "C" int yastn_hip_svd_precond_finalize(void* U, void* S, void* Vh, void* work, int dtype,
                                               const int64_t* d_blocks, const int64_t* d_qdesc, const int32_t* d_ids,
                                               int64_t n, int32_t* d_info, int sweeps, const int32_t* d_sweeps,
                                               hipStream_t stream) {
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
   if (n == 0) return YH_OK;
-  const dim3 g((unsigned)n), t(kThreads);
-  if (dtype == YH_F64)
-    hipLaunchKernelGGL(precond_finalize_kernel<false>, g, t, 0, stream, d_blocks, d_qdesc, d_ids,
-                       (const double*)work, (double*)U, (double*)S, (double*)Vh, d_info, sweeps, d_sweeps);
-  else
-    hipLaunchKernelGGL(precond_finalize_kernel<true>, g, t, 0, stream, d_blocks, d_qdesc, d_ids,
-                       (const double2*)work, (double2*)U, (double*)S, (double2*)Vh, d_info, sweeps, d_sweeps);
-  const int st = yh::hip_status(hipGetLastError(), "svd precond finalize launch");
-  if (st) return st;
-  return dtype == YH_F64 ? launch_complete<false>(d_blocks, d_ids, n, U, S, Vh, stream, 1)
-                         : launch_complete<true>(d_blocks, d_ids, n, U, S, Vh, stream, 1);
+  return dtype == YH_F64 ? launch_precond_finalize<false>(U, S, Vh, work, d_blocks, d_qdesc, d_ids, n, d_info, sweeps,
+                                                          d_sweeps, stream)
+                         : launch_precond_finalize<true>(U, S, Vh, work, d_blocks, d_qdesc, d_ids, n, d_info, sweeps,
+                                                         d_sweeps, stream);
 }
 
 extern "C" int yastn_hip_check_qr_op_plan(const int64_t* h_qdesc, const int64_t* h_qblocks, int64_t nblocks,

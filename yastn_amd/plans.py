@@ -725,10 +725,11 @@ def panel_slices(cross, stripes, cplx, width):
 
     With 16-column panels a workgroup has 4 waves, so more slices than a quarter of the stripes are idle.  The
     round lasts as long as the fullest CU, which holds g = ceil(cross slices / CUs) workgroups: g / slices of a
-    pair's update (0.3 us per stripe of 4 waves, complex 0.6) plus the sweep, 6 us (complex 9) and about 0.8 of that
-    again per further workgroup; the fewest slices of least cost are taken.  Measured (whole SVD): 14 pairs
-    of 56 stripes 11.2 ms with 1 slice, 7.6 with 14; 84 pairs 13.5 with 1, 11.0 with 3, 12.1 with 7; 140 pairs 13.7 with
-    1, 12.9 with 3, 16.5 with 10; 138 complex pairs of 138 stripes 135 with 1, 114 with 3, 128 with 4, 161 with 14.
+    pair's update (0.3 us per stripe, complex 0.6; 1.35, 1.55 and 1.65 times as fast with two, three and more workgroups
+    to hide each other's loads) plus the sweep, 6 us (complex 9) and about 0.8 of that again per further workgroup;
+    the fewest slices of least cost are taken.  Measured, whole calls: 14 pairs of 56 stripes 11.2 ms with 1 slice,
+    7.6 with 14; 84 pairs 13.5 with 1, 11.0 with 3, 12.1 with 7; 140 pairs 13.7 with 1, 12.9 with 3, 16.5 with 10; 138 complex
+    pairs of 138 stripes 135 with 1, 114 with 3, 128 with 4, 161 with 14; 255 of them 187 with 1, 169 with 3, 177 with 5.
     Other widths: 16 waves and a longer sweep, so at most about one workgroup per CU and one stripe per wave."""
     cu = L.device_cu_count()
     if width != 16:
@@ -737,7 +738,7 @@ def panel_slices(cross, stripes, cplx, width):
 
     def cost(s):
         g = -(-cross * s // cu)
-        return g * stripes * stripe / s + sweep * (1 + 0.8 * (g - 1))
+        return g * stripes * stripe / s / (1.0, 1.35, 1.55, 1.65)[min(g, 4) - 1] + sweep * (1 + 0.8 * (g - 1))
     return min(range(1, max(1, min(64, -(-stripes // 4))) + 1), key=lambda s: (cost(s), s))
 
 
@@ -871,7 +872,6 @@ class SvdPlan:
             self.part_numel = maxn * self.maxch_p * (t16 * (t16 + 1) // 2) * 256 * (itemsize // 8)
             self.d_jobs = torch.from_numpy(self.h_jobs).to(device)
             self.h_big = np.ascontiguousarray(np.array(big, dtype=np.int32))
-            self.d_big = torch.from_numpy(self.h_big).to(device)
             plain = [b for b in big if b not in set(pre)]
             self.n_plain = len(plain)
             self.d_plain = torch.from_numpy(np.array(plain or [0], dtype=np.int32)).to(device)
