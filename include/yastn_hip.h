@@ -318,7 +318,7 @@ int yastn_hip_qr_finalize(void* Q, void* R, const void* work, int dtype, const i
  * the products run as grouped GEMMs of the host's plan, these two entry points do the rest.
  * Words (YH_QRADJ_WORDS int64 per block): 0 m, 1 n, 2 k, 3 m_off (M1, M2, C: k x k row-major), 4 b_off
  * (B, m x k row-major), 5 ga_off (block of gA, m x n row-major), 6 r_off (R, k x n row-major), 7 unused.
- * trsm: one 64-thread workgroup per (row, block), k <= 65536 / itemsize. */
+ * trsm: one workgroup per 16 rows of a block, k <= 65536 / itemsize. */
 #define YH_QRADJ_WORDS 8
 int yastn_hip_check_qr_adjoint_plan(const int64_t* h_words, int64_t nblocks, int dtype, int64_t m_numel,
                                     int64_t b_numel, int64_t ga_numel, int64_t r_numel);
