@@ -35,7 +35,7 @@ extern "C" {
 #define YH_F64 0
 #define YH_C128 1
 
-#define YH_ABI_VERSION 15
+#define YH_ABI_VERSION 16
 
 /* ---- box-gather plan (one job per copied or zero-filled box) -------------
  * int64 words per job (YH_JOB_WORDS):
@@ -278,6 +278,16 @@ int yastn_hip_check_qr_plan(const int64_t* h_qdesc, const int64_t* h_blocks, con
  * lds_bytes >= p*YH_QR_NB*itemsize for every block, in place in the workspace when lds_bytes == 0. */
 int yastn_hip_svd_qr_panel(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, int step,
                            int64_t lds_bytes, hipStream_t stream);
+/* Block reflectors applied in one launch, 16 columns per workgroup, in place of three grouped GEMMs per panel:
+ * trailing: the columns of W0 right of panel `step` (after yastn_hip_svd_qr_panel of that step), of the listed blocks;
+ * svd_reflect: the p-side vectors that yastn_hip_svd_precond_finalize started, by all panels, last first;
+ * qr_reflect: E of the batched QR, by all panels, last first.  max_cols: the most columns of any block. */
+int yastn_hip_reflect_trailing(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, int step,
+                               int64_t max_cols, hipStream_t stream);
+int yastn_hip_svd_reflect(void* U, void* Vh, void* work, int dtype, const int64_t* d_blocks, const int64_t* d_qdesc,
+                          const int32_t* d_ids, int64_t n, int64_t max_cols, hipStream_t stream);
+int yastn_hip_qr_reflect(void* work, int dtype, const int64_t* d_qdesc, int64_t nblocks, int64_t max_cols,
+                         hipStream_t stream);
 /* W0 = A (or A^H when m < n) and floors[b] = eps^2 ||A||_F^2 of the preconditioned blocks (for them in place of
  * yastn_hip_svd_panel_init; the scratch at y_off, at least 64 elements, is used and left undefined). */
 int yastn_hip_svd_precond_load(const void* A, void* work, double* floors, int dtype, const int64_t* d_blocks,

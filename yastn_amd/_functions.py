@@ -587,6 +587,16 @@ def _side_stream(device):
     return _SIDE[key]
 
 
+def _householder_steps(plan, work, dt, st):
+    """The panel steps of a batched Householder QR (plans.SvdPlan / QrPlan): the panels of all blocks in one launch,
+    then their reflectors on the columns to their right in another."""
+    for step, (d_ids, n, rest) in enumerate(plan.panel_steps):
+        L.call('yastn_hip_svd_qr_panel', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step, plan.qr_lds, st)
+        if rest:
+            L.call('yastn_hip_reflect_trailing', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step, rest,
+                   st)
+
+
 def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
     """LDS-resident blocks in one launch; larger blocks through the panel path (one launch per round of
     panel pairs, one host check per sweep).  mode 0: SVD (U, S, Vh); mode 1: eigh (S, U)."""
@@ -624,13 +634,8 @@ def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
             if plan.n_pre:
                 L.call('yastn_hip_svd_precond_load', ptr(data), ptr(work), ptr(floors), dt, plan.d_blocks.data_ptr(),
                        plan.d_qdesc.data_ptr(), plan.d_pre.data_ptr(), plan.n_pre, st)
-                # W0 = Q R (Householder, one panel kernel and three grouped GEMMs per step), then X = R^H
-                for step, (d_ids, n, trail) in enumerate(plan.qr_steps):
-                    L.call('yastn_hip_svd_qr_panel', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step,
-                           plan.qr_lds, st)
-                    if trail is not None:
-                        for gp in trail:
-                            run_gemm(gp, (work,), (work,), dt, tune=False)
+                # W0 = Q R (Householder), then X = R^H
+                _householder_steps(plan, work, dt, st)
                 L.call('yastn_hip_svd_precond_init', ptr(work), dt, plan.d_qdesc.data_ptr(), plan.d_pre.data_ptr(),
                        plan.n_pre, st)
             # two launches per round (Gram partials, then inner sweep + update); a round of a sweep after one
@@ -664,10 +669,8 @@ def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
                        plan.d_blocks.data_ptr(), plan.d_qdesc.data_ptr(), plan.d_pre.data_ptr(), plan.n_pre, ptr(info),
                        done, d_sweeps, st)
                 # p-side vectors: [V_J; 0] -> Q [V_J; 0], panels in reverse order
-                for h1, h2, h3 in plan.q_apply:
-                    run_gemm(h1, (work,), (work, out_a, out_b), dt, tune=False)
-                    run_gemm(h2, (work,), (work,), dt, tune=False)
-                    run_gemm(h3, (work, out_a, out_b), (work,), dt, tune=False)
+                L.call('yastn_hip_svd_reflect', ptr(out_a), ptr(out_b), ptr(work), dt, plan.d_blocks.data_ptr(),
+                       plan.d_qdesc.data_ptr(), plan.d_pre.data_ptr(), plan.n_pre, plan.qr_cols, st)
     finally:
         # the side-stream launch reads data and writes the outputs: joined even when the panel path raises
         if joined is not None:
@@ -930,16 +933,8 @@ def qr_forward(data, meta, sizes, plan=None):
     work = torch.empty(plan.work_numel, dtype=data.dtype, device=data.device)
     L.call('yastn_hip_qr_init', ptr(data), ptr(work), dt, plan.d_qdesc.data_ptr(), plan.d_qblocks.data_ptr(),
            plan.nblocks, st)
-    for step, (d_ids, n, trail) in enumerate(plan.steps):
-        L.call('yastn_hip_svd_qr_panel', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step,
-               plan.lds, st)
-        if trail is not None:
-            for gp in trail:
-                run_gemm(gp, (work,), (work,), dt, tune=False)
-    for h1, h2, h3 in plan.q_apply:
-        run_gemm(h1, (work,), (work,), dt, tune=False)
-        run_gemm(h2, (work,), (work,), dt, tune=False)
-        run_gemm(h3, (work,), (work,), dt, tune=False)
+    _householder_steps(plan, work, dt, st)
+    L.call('yastn_hip_qr_reflect', ptr(work), dt, plan.d_qdesc.data_ptr(), plan.nblocks, plan.max_k, st)
     L.call('yastn_hip_qr_finalize', ptr(Q), ptr(R), ptr(work), dt, plan.d_qdesc.data_ptr(),
            plan.d_qblocks.data_ptr(), plan.nblocks, st)
     return Q, R

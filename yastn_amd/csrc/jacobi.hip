@@ -2175,6 +2175,201 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Block reflectors applied in one launch: C <- (I + V Tm' V^H) C for 16 columns of a block's C per workgroup, Tm = -T as
+// the panel kernel left it (Tm' = Tm^H for the trailing columns, Tm for the multiplication by Q).
+//   MODE 0: the columns of W0 right of panel `step` by that panel's reflectors;
+//   MODE 1: the p-side vectors of the preconditioned SVD (U, or Vh holding their conjugates) by all panels, last first;
+//   MODE 2: E of the batched QR by all panels, last first.
+// The columns are independent, so the three products of a panel (Y = V^H C, Y2 = Tm' Y, C += V Y2) need no other
+// workgroup: 8 waves split the rows, meet in LDS three times per panel, and all panels of a multiplication by Q run in
+// one launch.  Bound by the chain of those phases (~8 us a panel at 440 rows) and, on large blocks, by reading V once per
+// 16 columns.  As three grouped GEMMs per panel (84 launches of 7-19 us for seven blocks of up to 440 x 440, 700 us) the
+// launches and their ramps ruled: 290 us now (1.77 -> 1.47 ms for that QR with its adjoint); the QR of one 3000 x 3000
+// complex block 86 -> 75 ms, of 40 x 40 0.168 -> 0.124: faster at every size, so there is no other path.
+constexpr int kReflCols = 16, kReflWaves = 8, kReflThreads = 64 * kReflWaves;
+
+template <bool CPLX>
+constexpr size_t reflect_lds() {  // the waves' parts of Y (32 x 16 each), Y and Y2
+  return sizeof(double) * (CPLX ? 2 : 1) * (kReflWaves * 512 + 2 * 32 * 17);
+}
+
+template <bool CPLX, int MODE>
+__global__ void __launch_bounds__(kReflThreads)
+    reflect_kernel(const int64_t* __restrict__ blocks, const int64_t* __restrict__ qdesc,
+                   const int32_t* __restrict__ ids, typename Num<CPLX>::T* work, typename Num<CPLX>::T* U,
+                   typename Num<CPLX>::T* Vh, int step) {
+  typedef Num<CPLX> N;
+  typedef typename N::T T;
+  constexpr int NB = YH_QR_NB, NPL = CPLX ? 2 : 1;
+  extern __shared__ double smem_raw[];
+  double* s_part = smem_raw;  // [wave][plane][tile 0 / 1][item][lane]
+  T(*s_Y)[17] = reinterpret_cast<T(*)[17]>(smem_raw + kReflWaves * NPL * 512);
+  T(*s_Y2)[17] = s_Y + 32;
+  const int bidx = ids ? ids[blockIdx.x] : blockIdx.x;
+  const QrDesc d = load_qr(qdesc + (int64_t)bidx * YH_QR_WORDS);
+  const int64_t p = d.p, K = d.k;
+  T* C;
+  int64_t rs = 1, cs, ncol;
+  bool cj = false;
+  int shi = (int)((K + NB - 1) / NB) - 1, slo = 0;
+  if (MODE == 0) {
+    shi = slo = step;
+    const int64_t c0 = (int64_t)step * NB + min((int64_t)NB, K - (int64_t)step * NB);
+    ncol = d.q - c0;
+    C = work + d.w_off + c0 * p;
+    cs = p;
+  } else if (MODE == 1) {
+    const BlockDesc bd = load_desc(blocks + (int64_t)bidx * YH_SVD_WORDS);
+    ncol = d.q;
+    if (bd.m < bd.n) {
+      C = Vh + bd.v_off;
+      cs = p;
+      cj = true;
+    } else {
+      C = U + bd.u_off;
+      rs = d.q;
+      cs = 1;
+    }
+  } else {
+    C = work + d.x_off;
+    cs = p;
+    ncol = K;
+  }
+  const int64_t j0 = (int64_t)blockIdx.y * kReflCols;
+  if (j0 >= ncol) return;  // uniform
+  if (MODE == 2) shi = min(shi, (int)((j0 + kReflCols - 1) / NB));  // column j of E is e_j, zero below, until panel j / NB
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const T zero = N::make(0.0, 0.0);
+  const bool jok = j0 + r16 < ncol;
+  const int64_t jc = jok ? j0 + r16 : j0;  // columns past the block read its first one here and are not written
+  const double cv = cj ? -1.0 : 1.0;       // the sign of V's imaginary part
+  for (int s = shi; s >= slo; --s) {
+    const int64_t k0 = (int64_t)s * NB, L = p - k0;
+    const int nb = (int)min((int64_t)NB, K - k0);
+    const T* V = work + d.vall_off + k0 + k0 * p;
+    const T* Tm = work + d.tm_off + (int64_t)s * NB * NB;
+    T* Cs = C + k0 * rs;
+    // ---- Y = V^H C: wave w takes rows 4 w .. 4 w + 3 of every 32; lane: V(row kq, column r16 and 16 + r16), C(row kq, r16)
+    d4 accR[2], accI[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) accR[t] = accI[t] = d4{0.0, 0.0, 0.0, 0.0};
+    const int64_t i0 = min(r16, nb - 1) * p, i1 = min(16 + r16, nb - 1) * p;
+    constexpr int UN = CPLX ? 4 : 8;
+    for (int64_t rb = 4 * wave + kq; rb - kq < L; rb += 4 * kReflWaves * UN) {
+      T a0[UN], a1[UN], c[UN];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {  // all loads of a group first; rows past the block read its first one
+        const int64_t r = rb + 4 * kReflWaves * u, rc = r < L ? r : 0;
+        a0[u] = V[rc + i0];
+        a1[u] = V[rc + i1];
+        c[u] = Cs[rc * rs + jc * cs];
+      }
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        const bool ok = rb + 4 * kReflWaves * u < L;
+        const T b = pick(ok & jok, c[u], zero);
+        const T x0 = pick(ok & (r16 < nb), a0[u], zero), x1 = pick(ok & (16 + r16 < nb), a1[u], zero);
+        accR[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(x0), N::re(b), accR[0], 0, 0, 0);
+        accR[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(x1), N::re(b), accR[1], 0, 0, 0);
+        if constexpr (CPLX) {  // conj(x) b
+          const double y0 = cv * N::im(x0), y1 = cv * N::im(x1);
+          accI[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(x0), N::im(b), accI[0], 0, 0, 0);
+          accI[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(x1), N::im(b), accI[1], 0, 0, 0);
+          accR[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(y0, N::im(b), accR[0], 0, 0, 0);
+          accR[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(y1, N::im(b), accR[1], 0, 0, 0);
+          accI[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(-y0, N::re(b), accI[0], 0, 0, 0);
+          accI[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(-y1, N::re(b), accI[1], 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s_part[(wave * NPL) * 512 + t * 256 + v * 64 + lane] = accR[t][v];
+        if constexpr (CPLX) s_part[(wave * NPL + 1) * 512 + t * 256 + v * 64 + lane] = accI[t][v];
+      }
+    __syncthreads();
+    {  // thread: element (i, j) of Y, i = 16 tile + lane / 16 + 4 item, summed over the waves in order
+      double yr = 0.0, yi = 0.0;
+#pragma unroll
+      for (int w = 0; w < kReflWaves; ++w) {
+        yr += s_part[(w * NPL) * 512 + tid];
+        if constexpr (CPLX) yi += s_part[(w * NPL + 1) * 512 + tid];
+      }
+      s_Y[tid >> 4][tid & 15] = N::make(yr, yi);  // tid = 256 tile + 64 item + lane: row tid / 16, column tid % 16
+    }
+    __syncthreads();
+    // ---- Y2 = Tm' Y (Tm is zero outside its nb x nb upper triangle), one 16 x 16 tile per wave 0 / 1
+    if (wave < 2) {
+      d4 tR = {0.0, 0.0, 0.0, 0.0}, tI = {0.0, 0.0, 0.0, 0.0};
+      const int i = 16 * wave + r16;
+#pragma unroll
+      for (int ks = 0; ks < NB / 4; ++ks) {
+        const int kk = 4 * ks + kq;
+        const T tv = MODE == 0 ? Tm[kk + i * NB] : Tm[i + kk * NB];
+        const double tr = N::re(tv), ti = MODE == 0 ? -N::im(tv) : cv * N::im(tv);
+        const T y = s_Y[kk][r16];
+        tR = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, N::re(y), tR, 0, 0, 0);
+        if constexpr (CPLX) {
+          tI = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, N::im(y), tI, 0, 0, 0);
+          tR = __builtin_amdgcn_mfma_f64_16x16x4f64(-ti, N::im(y), tR, 0, 0, 0);
+          tI = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, N::re(y), tI, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s_Y2[16 * wave + kq + 4 * v][r16] = N::make(tR[v], tI[v]);
+    }
+    __syncthreads();
+    // ---- C += V Y2, one 16-row tile per wave at a time; with unit row stride as its transpose, so that a lane's items
+    // run along a row and every access covers 16 consecutive elements
+    T y2[NB / 4];
+#pragma unroll
+    for (int ks = 0; ks < NB / 4; ++ks) y2[ks] = s_Y2[4 * ks + kq][r16];
+    for (int64_t t0 = 16 * wave; t0 < L; t0 += 16 * kReflWaves) {
+      const int64_t row = t0 + r16, rc = row < L ? row : 0;
+      T v[NB / 4], o[4];
+#pragma unroll
+      for (int ks = 0; ks < NB / 4; ++ks) v[ks] = V[rc + min(4 * ks + kq, nb - 1) * p];
+      const bool unit = rs == 1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t rr = unit ? row : t0 + kq + 4 * u, jj = j0 + (unit ? kq + 4 * u : r16);
+        o[u] = Cs[(rr < L ? rr : 0) * rs + (jj < ncol ? jj : j0) * cs];
+      }
+      d4 aR = {0.0, 0.0, 0.0, 0.0}, aI = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int ks = 0; ks < NB / 4; ++ks) {
+        const T x = pick(4 * ks + kq < nb, v[ks], zero);
+        const double xr = N::re(x), xi = cv * N::im(x), yr = N::re(y2[ks]), yi = N::im(y2[ks]);
+        if (unit) {
+          aR = __builtin_amdgcn_mfma_f64_16x16x4f64(yr, xr, aR, 0, 0, 0);
+          if constexpr (CPLX) {
+            aI = __builtin_amdgcn_mfma_f64_16x16x4f64(yr, xi, aI, 0, 0, 0);
+            aR = __builtin_amdgcn_mfma_f64_16x16x4f64(-yi, xi, aR, 0, 0, 0);
+            aI = __builtin_amdgcn_mfma_f64_16x16x4f64(yi, xr, aI, 0, 0, 0);
+          }
+        } else {
+          aR = __builtin_amdgcn_mfma_f64_16x16x4f64(xr, yr, aR, 0, 0, 0);
+          if constexpr (CPLX) {
+            aI = __builtin_amdgcn_mfma_f64_16x16x4f64(xr, yi, aI, 0, 0, 0);
+            aR = __builtin_amdgcn_mfma_f64_16x16x4f64(-xi, yi, aR, 0, 0, 0);
+            aI = __builtin_amdgcn_mfma_f64_16x16x4f64(xi, yr, aI, 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t rr = unit ? row : t0 + kq + 4 * u, jj = j0 + (unit ? kq + 4 * u : r16);
+        if (rr < L && jj < ncol) Cs[rr * rs + jj * cs] = N::make(N::re(o[u]) + aR[u], N::im(o[u]) + aI[u]);
+      }
+    }
+    __syncthreads();  // C visible to the other waves for the next panel; the LDS buffers free
+  }
+}
+
 // The copies around the preconditioning (A -> W0, R^H -> X, the sorted vectors -> U, Vh) are bound by memory, so each
 // block is spread over `slices` workgroups (grid.y), which take its 32 x 32 tiles in turn; a copy between row- and
 // column-major goes through an LDS tile so that both sides are coalesced.  With one workgroup per block the three
@@ -2957,6 +3152,54 @@ extern "C" int yastn_hip_svd_qr_panel(void* work, int dtype, const int64_t* d_qd
                        (double2*)work, step);
   }
   return yh::hip_status(hipGetLastError(), "svd qr panel launch");
+}
+
+namespace {
+
+// MODE as reflect_kernel's; max_cols: the most columns of C of any block.
+template <bool CPLX, int MODE>
+int launch_reflect(const int64_t* d_blocks, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, void* work, void* U,
+                   void* Vh, int step, int64_t max_cols, hipStream_t stream) {
+  typedef typename Num<CPLX>::T T;
+  const int64_t slabs = yh::cdiv(max_cols, kReflCols);
+  YH_CHECK_ARG(n >= 0 && n <= INT32_MAX && max_cols >= 0 && slabs <= 65535, "reflector grid %lld x %lld", (long long)n,
+               (long long)slabs);
+  if (n == 0 || slabs == 0) return YH_OK;
+  const int st = yh::hip_status(hipFuncSetAttribute((const void*)reflect_kernel<CPLX, MODE>,
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    (int)reflect_lds<CPLX>()),
+                                "reflector LDS size");
+  if (st) return st;
+  hipLaunchKernelGGL((reflect_kernel<CPLX, MODE>), dim3((unsigned)n, (unsigned)slabs), dim3(kReflThreads),
+                     reflect_lds<CPLX>(), stream, d_blocks, d_qdesc, d_ids, (T*)work, (T*)U, (T*)Vh, step);
+  return yh::hip_status(hipGetLastError(), "reflector launch");
+}
+
+}  // namespace
+
+extern "C" int yastn_hip_reflect_trailing(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n,
+                                          int step, int64_t max_cols, hipStream_t stream) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  YH_CHECK_ARG(step >= 0, "step %d", step);
+  return dtype == YH_F64
+             ? launch_reflect<false, 0>(nullptr, d_qdesc, d_ids, n, work, nullptr, nullptr, step, max_cols, stream)
+             : launch_reflect<true, 0>(nullptr, d_qdesc, d_ids, n, work, nullptr, nullptr, step, max_cols, stream);
+}
+
+extern "C" int yastn_hip_svd_reflect(void* U, void* Vh, void* work, int dtype, const int64_t* d_blocks,
+                                     const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, int64_t max_cols,
+                                     hipStream_t stream) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  return dtype == YH_F64 ? launch_reflect<false, 1>(d_blocks, d_qdesc, d_ids, n, work, U, Vh, 0, max_cols, stream)
+                         : launch_reflect<true, 1>(d_blocks, d_qdesc, d_ids, n, work, U, Vh, 0, max_cols, stream);
+}
+
+extern "C" int yastn_hip_qr_reflect(void* work, int dtype, const int64_t* d_qdesc, int64_t nblocks, int64_t max_cols,
+                                    hipStream_t stream) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  return dtype == YH_F64
+             ? launch_reflect<false, 2>(nullptr, d_qdesc, nullptr, nblocks, work, nullptr, nullptr, 0, max_cols, stream)
+             : launch_reflect<true, 2>(nullptr, d_qdesc, nullptr, nblocks, work, nullptr, nullptr, 0, max_cols, stream);
 }
 
 extern "C" int yastn_hip_svd_precond_load(const void* A, void* work, double* floors, int dtype,

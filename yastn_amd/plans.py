@@ -9,6 +9,7 @@ scalar arguments.  Each plan is validated once on the host by the library's
 with an out-of-bounds work list.
 """
 import ctypes
+import functools
 from collections import OrderedDict
 import os
 import math
@@ -742,16 +743,27 @@ def panel_slices(cross, stripes, cplx, width):
     return min(range(1, max(1, min(64, -(-stripes // 4))) + 1), key=lambda s: (cost(s), s))
 
 
+def _panel_steps(blocks, device):
+    """Per step of a batched Householder QR of blocks (id, columns, reflectors): (device ids of the blocks that have a
+    panel there, their number, the most columns right of that panel)."""
+    NB, steps = L.YH_QR_NB, []
+    for k0 in range(0, max((k for _, _, k in blocks), default=0), NB):
+        act = [(b, n - min(k0 + NB, k)) for b, n, k in blocks if k > k0]
+        ids = torch.from_numpy(np.array([b for b, _ in act], dtype=np.int32)).to(device)
+        steps.append((ids, len(act), max(rest for _, rest in act)))
+    return steps
+
+
 class SvdPlan:
     """Block list of the batched Jacobi SVD / eigh.
 
     Blocks of few columns whose working matrices (W and V, (p q + q^2) elements) fit the LDS limit run in
     an LDS-resident kernel, one workgroup per block, all in one launch.  Larger blocks use the panel
     path: W and V in a workspace, panels of width b, one launch per round of panel pairs.  For SVD
-    blocks the panel path first factors W0 = Q R (blocked Householder QR: a panel kernel plus three
-    grouped GEMMs per step; the p x YH_QR_NB panel is staged in LDS when every block's fits, else
+    blocks the panel path first factors W0 = Q R (blocked Householder QR: a panel kernel and a launch of block
+    reflectors per step; the p x YH_QR_NB panel is staged in LDS when every block's fits, else
     factored in place in the workspace) and iterates on X = R^H; the p-side vectors are multiplied
-    by Q at the end (three grouped GEMMs per step).
+    by Q at the end (one launch).
     """
 
     def __init__(self, blocks, itemsize, mode, a_numel, u_numel, s_numel, v_numel, device):
@@ -880,8 +892,7 @@ class SvdPlan:
             self._qr_plans(blocks, pre, qd, itemsize, work, u_numel, v_numel, device)
 
     def _qr_plans(self, blocks, pre, qd, itemsize, work, u_numel, v_numel, device):
-        """Panel lists and grouped-GEMM plans of the Householder QR (trailing updates) and of the
-        final multiplication of the p-side vectors by Q (buffers: 0 workspace, 1 U, 2 Vh)."""
+        """Panel lists of the Householder QR."""
         NB = L.YH_QR_NB
         self.h_qdesc = np.ascontiguousarray(qd)
         pmax = max(int(qd[b, 0]) for b in pre)
@@ -895,60 +906,71 @@ class SvdPlan:
                len(ids), self.dt, max(work, 0), self.qr_lds)
         self.d_qdesc = torch.from_numpy(self.h_qdesc).to(device)
         self.d_pre = torch.from_numpy(ids).to(device)
-        nsteps = max(-(-int(qd[b, 1]) // NB) for b in pre)
-        bufs = (max(work, 1), max(u_numel, 1), max(v_numel, 1))
-        self.qr_steps = []   # (d_ids, n, trailing plans)
-        self.q_apply = []    # per step (reverse order): plans H1, H2, H3
-        for s in range(nsteps):
+        self.qr_cols = max(int(qd[b, 1]) for b in pre)
+        self.panel_steps = _panel_steps([(b, int(qd[b, 1]), int(qd[b, 1])) for b in pre], device)
+        self._gemm_args = (pre, (max(work, 1), max(u_numel, 1), max(v_numel, 1)), device)
+
+    @functools.cached_property
+    def qr_steps(self):
+        """What the reflector launches of the panel steps compute, written as grouped GEMMs (their reference in tests; not
+        run by the decompositions): per step (block ids, their number, the products for the columns right of the panel
+        or None): Y = V^H C; Y2 = Tm^H Y; C += V Y2   (Tm = -T: C <- (I - V T^H V^H) C)."""
+        pre, bufs, device = self._gemm_args
+        NB, steps = L.YH_QR_NB, []
+        for s, (d_ids, n, rest_max) in enumerate(self.panel_steps):
             k0 = s * NB
-            act = [b for b in pre if int(qd[b, 1]) > k0]
             g1, t1, g2, t2, g3, t3 = [], [], [], [], [], []
-            h1, u1, h2, u2, h3, u3 = [], [], [], [], [], []
-            for b in act:
-                p, q, w_off, vall_off, tm_off, x_off, y_off, _ = (int(x) for x in qd[b])
-                m, n = blocks[b][1], blocks[b][2]
-                tr = m < n
+            for b in pre:
+                p, q, w_off, vall_off, tm_off, x_off, y_off, _ = (int(x) for x in self.h_qdesc[b])
                 nbs = min(NB, q - k0)
-                Lr = p - k0
-                tm = tm_off + s * NB * NB
-                y2 = y_off + NB * q
                 rest = q - k0 - nbs
-                v0 = vall_off + k0 + k0 * p
-                if rest > 0:
-                    # Y = V^H C ; Y2 = Tm^H Y ; C += V Y2   (Tm = -T: C <- (I - V T^H V^H) C)
-                    g1.append((nbs, rest, y_off, q, 1, len(t1), 1, 0))
-                    t1.append((v0, p, 1, w_off + k0 + (k0 + nbs) * p, 1, p, Lr, 1))
-                    g2.append((nbs, rest, y2, q, 1, len(t2), 1, 0))
-                    t2.append((tm, NB, 1, y_off, q, 1, nbs, 1))
-                    g3.append((Lr, rest, w_off + k0 + (k0 + nbs) * p, 1, p, len(t3), 1, 1))
-                    t3.append((v0, 1, p, y2, q, 1, nbs, 0))
-                # Q application on the p-side vectors M (U for m >= n; conj(M) stored in Vh rows for m < n)
-                if not tr:
-                    mb, m_off, m_rs, m_cs, cj = 1, blocks[b][3], q, 1, 0
-                else:
-                    mb, m_off, m_rs, m_cs, cj = 2, blocks[b][5], 1, p, 1
-                h1.append((nbs, q, y_off, q, 1, len(u1), 1, 0))
-                u1.append((v0, p, 1, m_off + k0 * m_rs, m_rs, m_cs, Lr, (1 - cj) | (0 << 8) | (mb << 16)))
-                h2.append((nbs, q, y2, q, 1, len(u2), 1, 0))
-                u2.append((tm, 1, NB, y_off, q, 1, nbs, cj))
-                h3.append((Lr, q, m_off + k0 * m_rs, m_rs, m_cs, len(u3), 1, 1 | (mb << 8)))
-                u3.append((v0, 1, p, y2, q, 1, nbs, cj))
-            d_ids = torch.from_numpy(np.array(act, dtype=np.int32)).to(device)
+                if nbs <= 0 or rest <= 0:
+                    continue
+                c_off, y2, v0 = w_off + k0 + (k0 + nbs) * p, y_off + NB * q, vall_off + k0 + k0 * p
+                g1.append((nbs, rest, y_off, q, 1, len(t1), 1, 0))
+                t1.append((v0, p, 1, c_off, 1, p, p - k0, 1))
+                g2.append((nbs, rest, y2, q, 1, len(t2), 1, 0))
+                t2.append((tm_off + s * NB * NB, NB, 1, y_off, q, 1, nbs, 1))
+                g3.append((p - k0, rest, c_off, 1, p, len(t3), 1, 1))
+                t3.append((v0, 1, p, y2, q, 1, nbs, 0))
             trail = None
             if g1:
-                trail = (GemmPlan(g1, t1, bufs[:1], bufs[:1], device), GemmPlan(g2, t2, bufs[:1], bufs[:1], device),
-                         GemmPlan(g3, t3, bufs[:1], bufs[:1], device))
-            self.qr_steps.append((d_ids, len(act), trail))
-            self.q_apply.append((GemmPlan(h1, u1, bufs, bufs[:1], device), GemmPlan(h2, u2, bufs[:1], bufs[:1], device),
-                                 GemmPlan(h3, u3, bufs[:1], bufs, device)))
-        self.q_apply.reverse()
+                trail = tuple(GemmPlan(g, t, bufs[:1], bufs[:1], device) for g, t in ((g1, t1), (g2, t2), (g3, t3)))
+            steps.append((d_ids, n, trail))
+        return steps
+
+    @functools.cached_property
+    def q_apply(self):
+        """As ``qr_steps`` for the multiplication of the p-side vectors M (U for m >= n; conj(M) stored in Vh rows for
+        m < n) by Q, per panel in reverse order (buffers: 0 workspace, 1 U, 2 Vh)."""
+        pre, bufs, device = self._gemm_args
+        NB, out = L.YH_QR_NB, []
+        for s in reversed(range(len(self.panel_steps))):
+            k0 = s * NB
+            h1, u1, h2, u2, h3, u3 = [], [], [], [], [], []
+            for b in pre:
+                p, q, w_off, vall_off, tm_off, x_off, y_off, _ = (int(x) for x in self.h_qdesc[b])
+                nbs, y2, v0 = min(NB, q - k0), y_off + NB * q, vall_off + k0 + k0 * p
+                if nbs <= 0:
+                    continue
+                _, m, n, u_off, _, v_off = (int(x) for x in self.h_blocks[b][:6])
+                mb, m_off, m_rs, m_cs, cj = (2, v_off, 1, p, 1) if m < n else (1, u_off, q, 1, 0)
+                h1.append((nbs, q, y_off, q, 1, len(u1), 1, 0))
+                u1.append((v0, p, 1, m_off + k0 * m_rs, m_rs, m_cs, p - k0, (1 - cj) | (0 << 8) | (mb << 16)))
+                h2.append((nbs, q, y2, q, 1, len(u2), 1, 0))
+                u2.append((tm_off + s * NB * NB, 1, NB, y_off, q, 1, nbs, cj))
+                h3.append((p - k0, q, m_off + k0 * m_rs, m_rs, m_cs, len(u3), 1, 1 | (mb << 8)))
+                u3.append((v0, 1, p, y2, q, 1, nbs, cj))
+            out.append((GemmPlan(h1, u1, bufs, bufs[:1], device), GemmPlan(h2, u2, bufs[:1], bufs[:1], device),
+                        GemmPlan(h3, u3, bufs[:1], bufs, device)))
+        return out
 
 
 class QrPlan:
     """Batched Householder QR of the blocks of backend.qr (meta rows (sl, (m, n), slQ, (m, k), slR,
     (k, n))): per block the workspace holds W0 (m x n), the reflectors (m x k), -T per panel, E (m x k)
-    and the GEMM scratch; the panel steps and the GEMM plans follow the preconditioning of the SVD
-    (trailing updates of W0 after each panel, then E <- H_s E for the panels in reverse).  The
+    and scratch; the panel steps follow the preconditioning of the SVD (the columns of W0 right of each
+    panel after it, then E <- H_s E for the panels in reverse).  The
     32-column Householder panels are staged in LDS when every block's fits (``lds`` > 0), else
     factored in place in the workspace (``lds`` = 0)."""
 
@@ -973,52 +995,16 @@ class QrPlan:
         self.h_qdesc = np.ascontiguousarray(np.array(qd, dtype=np.int64).reshape(-1, L.YH_QR_WORDS))
         self.h_qblocks = np.ascontiguousarray(np.array(qb, dtype=np.int64).reshape(-1, L.YH_QROP_WORDS))
         pmax = max((r[0] for r in qd), default=1)
-        self.lds = pmax * NB * itemsize
-        if self.lds > L.device_lds_per_block() - 20 * 1024:  # static LDS of the panel kernel: ~17.5 KiB
-            self.lds = 0
+        self.max_k = max((r[7] for r in qd), default=0)
+        self.qr_lds = pmax * NB * itemsize
+        if self.qr_lds > L.device_lds_per_block() - 20 * 1024:  # static LDS of the panel kernel: ~17.5 KiB
+            self.qr_lds = 0
         self.native = True
         L.call('yastn_hip_check_qr_op_plan', self.h_qdesc.ctypes.data, self.h_qblocks.ctypes.data, self.nblocks,
-               self.dt, a_numel, sizes[0], sizes[1], self.work_numel, self.lds)
+               self.dt, a_numel, sizes[0], sizes[1], self.work_numel, self.qr_lds)
         self.d_qdesc = torch.from_numpy(self.h_qdesc).to(device)
         self.d_qblocks = torch.from_numpy(self.h_qblocks).to(device)
-        nsteps = max((-(-r[7] // NB) for r in qd), default=0)
-        bufs = (self.work_numel,)
-        self.steps, self.q_apply = [], []
-        for s in range(nsteps):
-            k0 = s * NB
-            act = [b for b in range(self.nblocks) if qd[b][7] > k0]
-            g1, t1, g2, t2, g3, t3 = [], [], [], [], [], []
-            h1, u1, h2, u2, h3, u3 = [], [], [], [], [], []
-            for b in act:
-                m, n, w_off, vall_off, tm_off, e_off, y_off, k = qd[b]
-                nbs = min(NB, k - k0)
-                Lr = m - k0
-                tm = tm_off + s * NB * NB
-                y2 = y_off + NB * n
-                rest = n - k0 - nbs
-                v0 = vall_off + k0 + k0 * m  # reflectors: m x k column-major
-                if rest > 0:  # W0(:, right of the panel) <- (I - V T^H V^H) W0(...), Tm = -T
-                    g1.append((nbs, rest, y_off, n, 1, len(t1), 1, 0))
-                    t1.append((v0, m, 1, w_off + k0 + (k0 + nbs) * m, 1, m, Lr, 1))
-                    g2.append((nbs, rest, y2, n, 1, len(t2), 1, 0))
-                    t2.append((tm, NB, 1, y_off, n, 1, nbs, 1))
-                    g3.append((Lr, rest, w_off + k0 + (k0 + nbs) * m, 1, m, len(t3), 1, 1))
-                    t3.append((v0, 1, m, y2, n, 1, nbs, 0))
-                # E(k0:, :) <- (I - V T V^H) E(k0:, :)
-                h1.append((nbs, k, y_off, n, 1, len(u1), 1, 0))
-                u1.append((v0, m, 1, e_off + k0, 1, m, Lr, 1))
-                h2.append((nbs, k, y2, n, 1, len(u2), 1, 0))
-                u2.append((tm, 1, NB, y_off, n, 1, nbs, 0))
-                h3.append((Lr, k, e_off + k0, 1, m, len(u3), 1, 1))
-                u3.append((v0, 1, m, y2, n, 1, nbs, 0))
-            d_ids = torch.from_numpy(np.array(act, dtype=np.int32)).to(device)
-            trail = None
-            if g1:
-                trail = tuple(GemmPlan(g, tt, bufs, bufs, device) for g, tt in ((g1, t1), (g2, t2), (g3, t3)))
-            self.steps.append((d_ids, len(act), trail))
-            self.q_apply.append(tuple(GemmPlan(g, tt, bufs, bufs, device) for g, tt in ((h1, u1), (h2, u2),
-                                                                                           (h3, u3))))
-        self.q_apply.reverse()
+        self.panel_steps = _panel_steps([(b, r[1], r[7]) for b, r in enumerate(qd)], device)
 
 
 class QrAdjointPlan:
