@@ -200,9 +200,9 @@ int yastn_hip_eigh(void* S, void* U, const void* A, int dtype, const int64_t* d_
  * d_jobs); per round, two launches: partial Gram matrices of each job's 2b columns over chunks of 64
  * rows (part), then per job `slices` workgroups that each run the job's inner sweep of rotations on
  * its Gram matrix and update their share of the pair's rows of W and V in place.  d_state (int32,
- * state_numel >= 4 + max_sweeps, ZERO before sweep 0): word 4 + sweep is set when a pair rotated in
- * that sweep, word 1 when the LDS cannot hold a pair; a round of sweep s > 0 whose previous sweep
- * rotated nothing exits at once, so sweeps can be issued without a host read in between (HIP graph
+ * state_numel >= 4 + max_sweeps, ZERO before sweep 0): word 4 + sweep is set when that
+ * sweep needs another one after it, word 1 when the LDS cannot hold a pair; a round of sweep s > 0 whose previous sweep
+ * was the last exits at once, so sweeps can be issued without a host read in between (HIP graph
  * capture).  yastn_hip_svd_panel_result turns the words into the sweep count (word 3: -3 for an LDS
  * plan too small); finalize writes U, S, Vh (or S, U) like yastn_hip_svd.  Columns whose squared norm
  * is below (eps ||A||_F)^2 (floors[b], set by init) are not rotated, here and in yastn_hip_svd: they are
@@ -228,8 +228,8 @@ int yastn_hip_svd_panel_sweep(void* work, const double* floors, int dtype, const
                               int32_t* d_state, int64_t state_numel, hipStream_t stream);
 int yastn_hip_check_panel_jobs(const int64_t* h_blocks, int64_t nblocks, const int32_t* h_jobs, int64_t njobs, int b,
                                int mode, int maxch_p);
-/* Sweep count of the panel rounds: word 3 of the state <- the first of the `launched` sweeps that rotated
- * nothing, + 1; -1 if every launched sweep rotated; -3 if a round found an LDS plan too small for a pair. */
+/* Sweep count of the panel rounds: word 3 of the state <- the first of the `launched` sweeps that needs
+ * none after it, + 1; -1 if every launched sweep does; -3 if a round found an LDS plan too small for a pair. */
 int yastn_hip_svd_panel_result(int32_t* d_state, int64_t state_numel, int launched, hipStream_t stream);
 /* d_sweeps (nullable): a device word holding the sweep count written to info (then `sweeps` is
  * ignored), e.g. word 3 of the panel sweep state. */
@@ -288,8 +288,9 @@ int yastn_hip_svd_reflect(void* U, void* Vh, void* work, int dtype, const int64_
                           const int32_t* d_ids, int64_t n, int64_t max_cols, hipStream_t stream);
 int yastn_hip_qr_reflect(void* work, int dtype, const int64_t* d_qdesc, int64_t nblocks, int64_t max_cols,
                          hipStream_t stream);
-/* W0 = A (or A^H when m < n) and floors[b] = eps^2 ||A||_F^2 of the preconditioned blocks (for them in place of
- * yastn_hip_svd_panel_init; the scratch at y_off, at least 64 elements, is used and left undefined). */
+/* W0 = A (or A^H when m < n), its columns in descending order of their norms, and floors[b] = eps^2 ||A||_F^2 of the
+ * preconditioned blocks (for them in place of yastn_hip_svd_panel_init).  The scratch at y_off holds the columns' ranks
+ * from its element 2 q on (q int32), which yastn_hip_svd_precond_finalize reads; the rest of it is undefined. */
 int yastn_hip_svd_precond_load(const void* A, void* work, double* floors, int dtype, const int64_t* d_blocks,
                                const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, hipStream_t stream);
 /* X = R^H, V_J = I. */
