@@ -52,7 +52,15 @@ def raw(t):
 def stream_of(t):
     if t.device.type != 'cuda':
         raise RuntimeError(f"yastn_amd backend needs GPU tensors, got a tensor on {t.device}")
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
+
+
+def _stream_object(index):
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# the raw handle of the current stream without a Stream object (a tenth of its cost), where torch has the call
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', _stream_object)
 
 
 def ptr(t):
@@ -319,6 +327,8 @@ def _mask_host(mask):
         key = tuple(k) if isinstance(k, (list, tuple)) else k
         if isinstance(v, slice):
             vals[key] = v
+        elif torch.is_tensor(v) and v.device.type == 'cpu' and not _is_wrapped(v):
+            vals[key] = as_index(v.detach().numpy())
         elif torch.is_tensor(v):
             vals[key] = None
             groups.setdefault((v.dtype, v.device), []).append((key, v))
@@ -402,19 +412,18 @@ class EmbedMask(_Fn):
 
 # ------------------------------------------------------------------ grouped GEMM
 
+_Pointers = L.ctypes.c_void_p * L.YH_MAX_BUFS
+
+
 def launch_plan(plan, outs, ins, dtype, stream):
     """One launch of a grouped-GEMM plan, followed by its split-K reduction when it has one (the
     partial products then live in a scratch buffer appended to the outputs)."""
-    outs = list(outs)
     part = None
     if plan.part_numel:
         dev = next(t for t in outs if t is not None)
         part = torch.empty(plan.part_numel, dtype=dev.dtype, device=dev.device)
-        outs = outs + [None] * (plan.part_buf - len(outs)) + [part]
-    outs = outs + [None] * (L.YH_MAX_BUFS - len(outs))
-    ins = list(ins) + [None] * (L.YH_MAX_BUFS - len(ins))
-    po = (L.ctypes.c_void_p * L.YH_MAX_BUFS)(*[ptr(t) for t in outs])
-    pi = (L.ctypes.c_void_p * L.YH_MAX_BUFS)(*[ptr(t) for t in ins])
+        outs = [*outs, *[None] * (plan.part_buf - len(outs)), part]
+    po, pi = _Pointers(*map(ptr, outs)), _Pointers(*map(ptr, ins))  # the rest are null
     L.call('yastn_hip_grouped_gemm', po, pi, dtype, *plan.args(), stream)
     if part is not None:
         L.call('yastn_hip_splitk_reduce', po, ptr(part), dtype, plan.d_red.data_ptr(), len(plan.h_red), stream)

@@ -269,7 +269,8 @@ def to_tensor(val, Ds=None, dtype='float64', device='cpu'):
 @torch.no_grad()
 def to_mask(val):
     """Index list of a boolean mask; kept on the host (the mask plans are built there)."""
-    return torch.from_numpy(np.nonzero(F.host_array(torch.as_tensor(val)).reshape(-1))[0].astype(np.int64))
+    host = val if isinstance(val, np.ndarray) else F.host_array(torch.as_tensor(val))
+    return torch.from_numpy(np.nonzero(host.reshape(-1))[0].astype(np.int64, copy=False))
 
 
 def square_matrix_from_dict(H, D=None, **kwargs):

@@ -46,13 +46,35 @@ class BlockSparseError(Exception):
 
 # ------------------------------------------------------------------ data model
 
-class Struct(NamedTuple):
+# The planners below are cached by the structures of their operands.  Hashing the charges, sizes and slices of a few
+# hundred blocks takes longer than anything else that a small contraction does on the host (75 of 160 us at 300 blocks),
+# so Struct and Slices compute their hash once.
+class _KeepHash:
+    def __hash__(self):
+        h = self.__dict__.get('_hash')
+        if h is None:
+            h = self.__dict__['_hash'] = tuple.__hash__(self)
+        return h
+
+    def __getstate__(self):  # pickles and copies carry the tuple alone
+        return None
+
+
+class _StructFields(NamedTuple):
     s: tuple = ()
     n: tuple = ()
     diag: bool = False
     t: tuple = ()
     D: tuple = ()
     size: int = 0
+
+
+class Struct(_KeepHash, _StructFields):
+    pass
+
+
+class Slices(_KeepHash, tuple):
+    """The Slc of every block, in the order of the blocks."""
 
 
 class Slc(NamedTuple):
@@ -146,7 +168,12 @@ def leg(config, s, t, D):
 
 
 def _slices_of(Dps, Ds):
-    return tuple(Slc(((stop - dp, stop),), ds, dp) for stop, dp, ds in zip(accumulate(Dps), Dps, Ds))
+    return Slices(Slc(((stop - dp, stop),), ds, dp) for stop, dp, ds in zip(accumulate(Dps), Dps, Ds))
+
+
+@lru_cache(maxsize=1024)
+def _conj_struct(sym, struct):
+    return struct._replace(s=tuple(-x for x in struct.s), n=sym.add_charges(struct.n, new_signature=-1))
 
 
 # ------------------------------------------------------------------ tensor
@@ -216,10 +243,7 @@ class Tensor:
 
     # -- algebra
     def conj(self):
-        sym = self.config.sym
-        n = sym.add_charges(self.struct.n, new_signature=-1)
-        struct = self.struct._replace(s=tuple(-x for x in self.struct.s), n=n)
-        return self._replace(struct=struct, hfs=tuple(h.conj() for h in self.hfs),
+        return self._replace(struct=_conj_struct(self.config.sym, self.struct), hfs=tuple(h.conj() for h in self.hfs),
                              data=self.config.backend.conj(self._data))
 
     def transpose(self, axes):
@@ -313,7 +337,7 @@ class Tensor:
             sd = d['struct']
             struct = Struct(s=tup(sd['s']), n=tup(sd['n']), diag=bool(sd['diag']), t=tup(sd['t']), D=tup(sd['D']),
                             size=int(sd['size']))
-            slices = tuple(Slc(tup(x[0]), tup(x[1]), int(x[2])) for x in d['slices'])
+            slices = Slices(Slc(tup(x[0]), tup(x[1]), int(x[2])) for x in d['slices'])
             hfs = tuple(Fusion(**{k: (tup(v) if k != 'op' else v) for k, v in h.items()}) for h in d['hfs'])
             data = d['data']
             if isinstance(data, np.ndarray):
@@ -495,6 +519,7 @@ def _get_tD_legs(struct):
     return [tuple(d.keys()) for d in dicts], [tuple(d.values()) for d in dicts], dicts
 
 
+@lru_cache(maxsize=1024)
 def _leg_struct_trivial(struct, axis=0):
     nsym = len(struct.n)
     tD = sorted((tt[nsym * axis: nsym * (axis + 1)], DD[axis]) for tt, DD in zip(struct.t, struct.D))
@@ -545,7 +570,7 @@ def _meta_merge_to_matrix(config, struct, slices, axes, inds):
                 meta_mrg.append((tn, grp[k][4], grp[k][5], (d0.Dslc, d1.Dslc), (d0.Dprod, d1.Dprod)))
                 k += 1
     struct_new = struct._replace(t=tuple(t_new), D=tuple(D_new), s=s_eff, size=lo)
-    return struct_new, tuple(sl_new), tuple(meta_mrg), ls[0], ls[1]
+    return struct_new, Slices(sl_new), tuple(meta_mrg), ls[0], ls[1]
 
 
 def _no_change_in_transpose_and_merge(meta_mrg, meta_new, Dsize):
@@ -571,27 +596,30 @@ def _no_change_in_transpose_and_merge(meta_mrg, meta_new, Dsize):
 
 
 def _transpose_and_merge(config, data, order, struct, slices, meta_mrg, inds=None):
+    args = _merge_args(order, struct, slices, meta_mrg, inds, config.backend.get_size(data))
+    return data if args is None else config.backend.transpose_and_merge(data, *args)
+
+
+def _merge_args(order, struct, slices, meta_mrg, inds, size):
+    """The arguments of the backend's transpose_and_merge after the data (of ``size`` elements), or None where the data
+    is already in place."""
     meta_new = tuple((x, y, z.slcs[0]) for x, y, z in zip(struct.t, struct.D, slices))
-    if inds is None and tuple(range(len(order))) == tuple(order) and struct.size == config.backend.get_size(data) \
+    if inds is None and tuple(range(len(order))) == tuple(order) and struct.size == size \
             and _no_change_in_transpose_and_merge(meta_mrg, meta_new, struct.size):
-        return data
-    return config.backend.transpose_and_merge(data, order, meta_new, meta_mrg, struct.size)
+        return None
+    return order, meta_new, meta_mrg, struct.size
 
 
-def _transpose_and_merge_pair(config, ops):
-    """_transpose_and_merge of two operands ((data, order, struct, slices, meta_mrg, inds) each); one backend
-    call for both when both need a merge and the backend fuses such pairs (transpose_and_merge_pair)."""
-    todo = []
-    for data, order, struct, slices, meta_mrg, inds in ops:
-        meta_new = tuple((x, y, z.slcs[0]) for x, y, z in zip(struct.t, struct.D, slices))
-        noop = inds is None and tuple(range(len(order))) == tuple(order) \
-            and struct.size == config.backend.get_size(data) \
-            and _no_change_in_transpose_and_merge(meta_mrg, meta_new, struct.size)
-        todo.append(None if noop else (data, order, meta_new, meta_mrg, struct.size))
-    pair = getattr(config.backend, 'transpose_and_merge_pair', None)
-    if pair is not None and todo[0] is not None and todo[1] is not None:
-        return pair(*todo[0], *todo[1])
-    return tuple(op[0] if t is None else config.backend.transpose_and_merge(*t) for op, t in zip(ops, todo))
+def _transpose_and_merge_pair(config, data_a, args_a, data_b, args_b):
+    """transpose_and_merge of two operands (args: _merge_args); one backend call for both when both need a merge and the
+    backend fuses such pairs (transpose_and_merge_pair)."""
+    backend = config.backend
+    if args_a is not None and args_b is not None:
+        pair = getattr(backend, 'transpose_and_merge_pair', None)
+        if pair is not None:
+            return pair(data_a, *args_a, data_b, *args_b)
+    return (data_a if args_a is None else backend.transpose_and_merge(data_a, *args_a),
+            data_b if args_b is None else backend.transpose_and_merge(data_b, *args_b))
 
 
 def _merge_to_matrix(a, axes, inds=None):
@@ -845,7 +873,6 @@ def consume_transpose(a):
 
 # ------------------------------------------------------------------ tensordot
 
-@lru_cache(maxsize=1024)
 def _common_inds(t_a, t_b, nin_a, nin_b, ndim_a, ndim_b, nsym):
     """reference _contractions.py:250-278."""
     ta = np.array(t_a, dtype=np.int64).reshape((len(t_a), ndim_a, nsym))
@@ -858,7 +885,6 @@ def _common_inds(t_a, t_b, nin_a, nin_b, ndim_a, ndim_b, nsym):
     return (None if len(ia) == len(la) else ia), (None if len(ib) == len(lb) else ib)
 
 
-@lru_cache(maxsize=1024)
 def _meta_tensordot_f2m(struct_a, slices_a, struct_b, slices_b):
     """reference _contractions.py:281-298."""
     nsym = len(struct_a.n)
@@ -878,7 +904,6 @@ def _meta_tensordot_f2m(struct_a, slices_a, struct_b, slices_b):
     return meta, Struct(s=(struct_a.s[0], struct_b.s[1]), t=t_c, D=D_c, size=sum(Dp)), slices_c
 
 
-@lru_cache(maxsize=1024)
 def _meta_tensordot_fc(struct_a, slices_a, struct_b, slices_b):
     """reference _contractions.py:301-346."""
     nsym = len(struct_a.n)
@@ -909,7 +934,6 @@ def _meta_tensordot_fc(struct_a, slices_a, struct_b, slices_b):
     return meta, Struct(s=struct_a.s[:-1] + struct_b.s[1:], t=t_c, D=D_c, size=sum(Dp)), slices_c
 
 
-@lru_cache(maxsize=1024)
 def _meta_tensordot_nf(struct_a, slices_a, struct_b, slices_b, ind_a, ind_b, nout_a, nin_a, nin_b, nout_b):
     """No-fusion policy (reference _contractions.py:349-450).  Returns (meta_dot, reshape_a, reshape_b,
     struct_c, slices_c): reshape_* = (slice, block shape, rows, cols) of each participating block as the
@@ -958,7 +982,7 @@ def _meta_tensordot_nf(struct_a, slices_a, struct_b, slices_b, ind_a, ind_b, nou
     Dp = [r * c for r, c in Dp2]
     offs = tuple(accumulate(Dp, initial=0))
     slc_c = tuple(zip(offs, offs[1:]))
-    slices_c = tuple(Slc((sl,), D, dp) for sl, D, dp in zip(slc_c, D_c, Dp))
+    slices_c = Slices(Slc((sl,), D, dp) for sl, D, dp in zip(slc_c, D_c, Dp))
     pairs = np.column_stack([pa, pb])[np.argsort(inv)].tolist()
     bounds = tuple(accumulate(cnt.tolist(), initial=0))
     meta_dot = [(sl, d2, pairs[i:j]) for sl, d2, i, j in zip(slc_c, Dp2, bounds, bounds[1:])]
@@ -993,62 +1017,85 @@ def tensordot(a, b, axes, conj=(0, 0)):
             raise BlockSparseError('hard-fusion structures of contracted legs differ')
     nout_a = tuple(i for i in a.trans if i not in nin_a)
     nout_b = tuple(i for i in b.trans if i not in nin_b)
-    n_c = a.config.sym.add_charges(a.struct.n, b.struct.n)
-    s_c = tuple(a.struct.s[i] for i in nout_a) + tuple(b.struct.s[i] for i in nout_b)
     hfs_c = tuple(a.hfs[i] for i in nout_a) + tuple(b.hfs[i] for i in nout_b)
-    if a.config.tensordot_policy == 'fuse_to_matrix':
-        data, struct_c, slices_c = _tensordot_f2m(a, b, nout_a, nin_a, nin_b, nout_b, s_c)
-    elif a.config.tensordot_policy == 'fuse_contracted':
-        data, struct_c, slices_c = _tensordot_fc(a, b, nout_a, nin_a, nin_b, nout_b)
-    elif a.config.tensordot_policy == 'no_fusion':
-        data, struct_c, slices_c = _tensordot_nf(a, b, nout_a, nin_a, nin_b, nout_b)
-    else:
+    if a.config.tensordot_policy not in _TENSORDOT:
         raise BlockSparseError(f"tensordot policy {a.config.tensordot_policy} not restated")
-    return Tensor(a.config, struct_c._replace(n=n_c), slices_c, data, hfs=hfs_c, trans=None)
+    data, struct_c, slices_c = _TENSORDOT[a.config.tensordot_policy](a, b, nout_a, nin_a, nin_b, nout_b)
+    return Tensor(a.config, struct_c, slices_c, data, hfs=hfs_c, trans=None)
 
 
-def _tensordot_f2m(a, b, nout_a, nin_a, nin_b, nout_b, s_c):
-    nsym = a.config.sym.NSYM
-    ind_a, ind_b = _common_inds(a.struct.t, b.struct.t, nin_a, nin_b, a.ndim_n, b.ndim_n, nsym)
-    struct_a, slices_a, mrg_a, ls_l, ls_ac = _meta_merge_to_matrix(a.config, a.struct, a.slices, (nout_a, nin_a), ind_a)
-    struct_b, slices_b, mrg_b, ls_bc, ls_r = _meta_merge_to_matrix(b.config, b.struct, b.slices, (nin_b, nout_b), ind_b)
-    data_a, data_b = _transpose_and_merge_pair(
-        a.config, ((a._data, nout_a + nin_a, struct_a, slices_a, mrg_a, ind_a),
-                   (b._data, nin_b + nout_b, struct_b, slices_b, mrg_b, ind_b)))
+@lru_cache(maxsize=1024)
+def _plan_tensordot_f2m(config, struct_a, slices_a, size_a, struct_b, slices_b, size_b, nout_a, nin_a, nin_b, nout_b):
+    nsym = config.sym.NSYM
+    ind_a, ind_b = _common_inds(struct_a.t, struct_b.t, nin_a, nin_b, len(struct_a.s), len(struct_b.s), nsym)
+    n_c = config.sym.add_charges(struct_a.n, struct_b.n)
+    s_c = tuple(struct_a.s[i] for i in nout_a) + tuple(struct_b.s[i] for i in nout_b)
+    struct_a, slices_a, mrg_a, ls_l, ls_ac = _meta_merge_to_matrix(config, struct_a, slices_a, (nout_a, nin_a), ind_a)
+    struct_b, slices_b, mrg_b, ls_bc, ls_r = _meta_merge_to_matrix(config, struct_b, slices_b, (nin_b, nout_b), ind_b)
     if ls_ac != ls_bc:
         raise BlockSparseError('Bond dimensions do not match.')
+    args_a = _merge_args(nout_a + nin_a, struct_a, slices_a, mrg_a, ind_a, size_a)
+    args_b = _merge_args(nin_b + nout_b, struct_b, slices_b, mrg_b, ind_b, size_b)
     meta_dot, struct_c, slices_c = _meta_tensordot_f2m(struct_a, slices_a, struct_b, slices_b)
-    data = a.config.backend.dot(data_a, data_b, meta_dot, struct_c.size)
-    meta_un, struct_c, slices_c = _meta_unmerge_matrix(a.config, struct_c, slices_c, ls_l, ls_r, s_c)
+    size_dot = struct_c.size
+    meta_un, struct_c, slices_c = _meta_unmerge_matrix(config, struct_c, slices_c, ls_l, ls_r, s_c)
+    return args_a, args_b, meta_dot, size_dot, meta_un, struct_c._replace(n=n_c), slices_c
+
+
+def _tensordot_f2m(a, b, nout_a, nin_a, nin_b, nout_b):
+    size = a.config.backend.get_size
+    args_a, args_b, meta_dot, size_dot, meta_un, struct_c, slices_c = _plan_tensordot_f2m(
+        a.config, a.struct, a.slices, size(a._data), b.struct, b.slices, size(b._data), nout_a, nin_a, nin_b, nout_b)
+    data_a, data_b = _transpose_and_merge_pair(a.config, a._data, args_a, b._data, args_b)
+    data = a.config.backend.dot(data_a, data_b, meta_dot, size_dot)
     return _unmerge(a.config, data, meta_un), struct_c, slices_c
 
 
-def _tensordot_fc(a, b, nout_a, nin_a, nin_b, nout_b):
-    nsym = a.config.sym.NSYM
-    ind_a, ind_b = _common_inds(a.struct.t, b.struct.t, nin_a, nin_b, a.ndim_n, b.ndim_n, nsym)
+@lru_cache(maxsize=1024)
+def _plan_tensordot_fc(config, struct_a, slices_a, size_a, struct_b, slices_b, size_b, nout_a, nin_a, nin_b, nout_b):
+    nsym = config.sym.NSYM
+    ind_a, ind_b = _common_inds(struct_a.t, struct_b.t, nin_a, nin_b, len(struct_a.s), len(struct_b.s), nsym)
+    n_c = config.sym.add_charges(struct_a.n, struct_b.n)
     axes_a = tuple((x,) for x in nout_a) + (nin_a,)
-    order_a = nout_a + nin_a
-    struct_a, slices_a, mrg_a, t_a, D_a = _meta_fuse_hard(a.config, a.struct, a.slices, axes_a, ind_a)
+    struct_a, slices_a, mrg_a, t_a, D_a = _meta_fuse_hard(config, struct_a, slices_a, axes_a, ind_a)
     axes_b = (nin_b,) + tuple((x,) for x in nout_b)
-    order_b = nin_b + nout_b
-    struct_b, slices_b, mrg_b, t_b, D_b = _meta_fuse_hard(b.config, b.struct, b.slices, axes_b, ind_b)
-    data_a, data_b = _transpose_and_merge_pair(a.config, ((a._data, order_a, struct_a, slices_a, mrg_a, None),
-                                                          (b._data, order_b, struct_b, slices_b, mrg_b, None)))
+    struct_b, slices_b, mrg_b, t_b, D_b = _meta_fuse_hard(config, struct_b, slices_b, axes_b, ind_b)
     if not all(D_a[i] == D_b[j] for i, j in zip(nin_a, nin_b)):
         raise BlockSparseError('Bond dimensions do not match.')
+    args_a = _merge_args(nout_a + nin_a, struct_a, slices_a, mrg_a, None, size_a)
+    args_b = _merge_args(nin_b + nout_b, struct_b, slices_b, mrg_b, None, size_b)
     meta_dot, struct_c, slices_c = _meta_tensordot_fc(struct_a, slices_a, struct_b, slices_b)
-    data = a.config.backend.dot(data_a, data_b, meta_dot, struct_c.size)
-    return data, struct_c, slices_c
+    return args_a, args_b, meta_dot, struct_c._replace(n=n_c), slices_c
+
+
+def _tensordot_fc(a, b, nout_a, nin_a, nin_b, nout_b):
+    size = a.config.backend.get_size
+    args_a, args_b, meta_dot, struct_c, slices_c = _plan_tensordot_fc(
+        a.config, a.struct, a.slices, size(a._data), b.struct, b.slices, size(b._data), nout_a, nin_a, nin_b, nout_b)
+    data_a, data_b = _transpose_and_merge_pair(a.config, a._data, args_a, b._data, args_b)
+    return a.config.backend.dot(data_a, data_b, meta_dot, struct_c.size), struct_c, slices_c
+
+
+@lru_cache(maxsize=1024)
+def _plan_tensordot_nf(config, struct_a, slices_a, struct_b, slices_b, nout_a, nin_a, nin_b, nout_b):
+    ind_a, ind_b = _common_inds(struct_a.t, struct_b.t, nin_a, nin_b, len(struct_a.s), len(struct_b.s),
+                                config.sym.NSYM)
+    meta_dot, reshape_a, reshape_b, struct_c, slices_c = _meta_tensordot_nf(
+        struct_a, slices_a, struct_b, slices_b, ind_a, ind_b, nout_a, nin_a, nin_b, nout_b)
+    n_c = config.sym.add_charges(struct_a.n, struct_b.n)
+    return meta_dot, reshape_a, reshape_b, struct_c._replace(n=n_c), slices_c
 
 
 def _tensordot_nf(a, b, nout_a, nin_a, nin_b, nout_b):
     """reference _contractions.py:186-246 (the transpose_dot_sum branch)."""
-    ind_a, ind_b = _common_inds(a.struct.t, b.struct.t, nin_a, nin_b, a.ndim_n, b.ndim_n, a.config.sym.NSYM)
-    meta_dot, reshape_a, reshape_b, struct_c, slices_c = _meta_tensordot_nf(
-        a.struct, a.slices, b.struct, b.slices, ind_a, ind_b, nout_a, nin_a, nin_b, nout_b)
+    meta_dot, reshape_a, reshape_b, struct_c, slices_c = _plan_tensordot_nf(
+        a.config, a.struct, a.slices, b.struct, b.slices, nout_a, nin_a, nin_b, nout_b)
     data = a.config.backend.transpose_dot_sum(a._data, b._data, meta_dot, reshape_a, reshape_b, nout_a + nin_a,
                                               nin_b + nout_b, struct_c.size)
     return data, struct_c, slices_c
+
+
+_TENSORDOT = {'fuse_to_matrix': _tensordot_f2m, 'fuse_contracted': _tensordot_fc, 'no_fusion': _tensordot_nf}
 
 
 @lru_cache(maxsize=1024)
@@ -1140,14 +1187,15 @@ def apply_mask(mask, *args, axes=0):
 
 # ------------------------------------------------------------------ decompositions
 
+@lru_cache(maxsize=1024)
 def _meta_svd(config, struct, slices, minD, sU, nU):
-    """reference linalg.py:323-380 (not cached there either: the backend caches plans by content)."""
+    """reference linalg.py:323-380."""
     sym, nsym = config.sym, config.sym.NSYM
     n0 = sym.zero()
     if any(D == 0 for D in minD):
         keep = [i for i, d in enumerate(minD) if d > 0]
         struct = struct._replace(t=tuple(struct.t[i] for i in keep), D=tuple(struct.D[i] for i in keep))
-        slices = tuple(slices[i] for i in keep)
+        slices = Slices(slices[i] for i in keep)
         minD = tuple(minD[i] for i in keep)
     if nU and sU == struct.s[1]:
         t_con = tuple(x[nsym:] for x in struct.t)
@@ -1209,6 +1257,7 @@ def svd(a, axes=(0, 1), sU=1, nU=True, Uaxis=-1, Vaxis=0, fix_signs=False, **kwa
     return U.moveaxis(-1, Uaxis), S, V.moveaxis(0, Vaxis)
 
 
+@lru_cache(maxsize=1024)
 def _meta_qr(config, struct, slices, sQ):
     """Sector layout of Q and R for a = Q R (reference linalg.py:795-830): Q(s0, sQ) keeps the charge of a,
     R(-sQ, s1) has zero charge; the connecting leg of a sector carries the charge that lets R be charge-free.
@@ -1342,7 +1391,7 @@ def truncation_mask(S, tol=0, tol_block=0, D_block=float('inf'), D_total=float('
         lo, hi = sl.slcs[0]
         tol_rel = tol_block[t] if isinstance(tol_block, dict) and t in tol_block else tol_null
         blk = Sh[lo:hi]
-        D_tol = int(np.sum(blk > tol_rel * np.max(np.abs(blk)))) if hi > lo else 0
+        D_tol = np.count_nonzero(blk > tol_rel * np.abs(blk).max()) if hi > lo else 0
         D_bl = D_block[t] if isinstance(D_block, dict) and t in D_block else D_null
         D_bl = min(D_bl, D_tol)
         if 0 < D_bl < sl.Dp:
@@ -1351,7 +1400,7 @@ def truncation_mask(S, tol=0, tol_block=0, D_block=float('inf'), D_total=float('
         elif D_bl == 0:
             keep[lo:hi] = False
     tmp = Sh * keep
-    D_tol = int(np.sum(tmp > tol * np.max(np.abs(tmp)))) if tmp.size else 0
+    D_tol = np.count_nonzero(tmp > tol * np.abs(tmp).max()) if tmp.size else 0
     D_total = min(D_total, D_tol)
     if D_total == 0:
         keep[:] = False
@@ -1468,6 +1517,7 @@ def svd_with_truncation(a, axes=(0, 1), sU=1, nU=True, Uaxis=-1, Vaxis=0, fix_si
     return U.moveaxis(-1, Uaxis), S, V.moveaxis(0, Vaxis)
 
 
+@lru_cache(maxsize=1024)
 def _meta_eigh(config, struct, slices, sU, minD):
     """reference linalg.py:963-1010."""
     sym, nsym = config.sym, config.sym.NSYM
