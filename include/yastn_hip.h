@@ -35,7 +35,7 @@ extern "C" {
 #define YH_F64 0
 #define YH_C128 1
 
-#define YH_ABI_VERSION 16
+#define YH_ABI_VERSION 17
 
 /* ---- box-gather plan (one job per copied or zero-filled box) -------------
  * int64 words per job (YH_JOB_WORDS):
@@ -348,6 +348,11 @@ int yastn_hip_fix_svd_signs(void* U, void* Vh, int dtype, const int64_t* d_block
  *      that entry with differentiable tensor ops; the binding does the same with the pivots). */
 int yastn_hip_svd_sign_pivots(const void* U, int64_t* piv, int dtype, const int64_t* d_blocks, int64_t nblocks,
                               hipStream_t stream);
+/* What the host reads after a decomposition, in one place: out[0] = min(info), out[1] = negative info words, out[2] = 1 if
+ * `data` (numel elements) holds an inf or NaN.  out: int32, out_numel >= 3 + YH_CHECK_SCRATCH. */
+#define YH_CHECK_SCRATCH 256
+int yastn_hip_check_result(int32_t* out, int64_t out_numel, const int32_t* info, int64_t nblocks, const void* data,
+                           int64_t numel, int dtype, hipStream_t stream);
 
 /* A9 core: the k x k middle factor of kernel_svd.backward / SVDGESDD.backward
  *     (_backend_torch_backwards.py:53-66, linalg/torch_svd_gesdd.py:296-428) for every block:

@@ -558,16 +558,13 @@ class deferred_checks:
         return False
 
     def check(self):
-        for what, info, nonfinite in self.flags:
-            _raise_on_info(info, what, nonfinite)
+        for what, flags in self.flags:
+            _raise_on_flags(flags, what)
 
 
-def _raise_on_info(info, what, nonfinite=None):
-    if info.numel() == 0:
-        return
-    flags = [info.min(), (info < 0).sum()] + ([nonfinite.to(info.dtype)] if nonfinite is not None else [])
-    lo, bad, *nf = torch.stack(flags).tolist()
-    if nf and nf[0]:
+def _raise_on_flags(flags, what):
+    lo, bad, nonfinite = flags.tolist()
+    if nonfinite:
         # as the reference, whose scipy SVD / eigh check the input (backend_np.py:281-286)
         raise ValueError(f"{what}: the input contains infs or NaNs")
     if lo == -3:
@@ -576,13 +573,19 @@ def _raise_on_info(info, what, nonfinite=None):
         raise L.HipBackendError(f"{what}: Jacobi did not converge in {MAX_SWEEPS} sweeps for {bad} block(s)")
 
 
-def _check_info(info, what, nonfinite=None):
-    if _DEFERRED:
-        _DEFERRED[-1].append((what, info, nonfinite))
-    elif torch.cuda.is_current_stream_capturing():
+def _check_info(info, what, data, dt, st):
+    """Convergence words of a decomposition of ``data`` and whether that is finite, checked now or deferred."""
+    capturing = torch.cuda.is_current_stream_capturing()
+    if not _DEFERRED and capturing:
         raise RuntimeError("yastn_amd: SVD/eigh captured in a HIP graph needs deferred_checks() around the capture")
-    elif SYNC_CHECKS:
-        _raise_on_info(info, what, nonfinite)
+    if info.numel() == 0 or not (_DEFERRED or SYNC_CHECKS):
+        return
+    out = torch.empty(3 + L.YH_CHECK_SCRATCH, dtype=torch.int32, device=info.device)
+    L.call('yastn_hip_check_result', ptr(out), out.numel(), ptr(info), info.numel(), ptr(data), data.numel(), dt, st)
+    if _DEFERRED:
+        _DEFERRED[-1].append((what, out[:3]))
+    else:
+        _raise_on_flags(out[:3], what)
 
 
 _SIDE = {}
@@ -684,8 +687,7 @@ def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
         # the side-stream launch reads data and writes the outputs: joined even when the panel path raises
         if joined is not None:
             joined[0].wait_stream(joined[1])
-    nonfinite = torch.isfinite(data).logical_not().any() if data.numel() else None
-    _check_info(info[:plan.nblocks], 'svd' if mode == 0 else 'eigh', nonfinite)
+    _check_info(info[:plan.nblocks], 'svd' if mode == 0 else 'eigh', data, dt, st)
 
 
 def svd_forward(data, meta, sizes):

@@ -12,7 +12,7 @@ LIB_PATH = os.environ.get('YASTN_HIP_LIB', os.path.join(HERE, 'libyastn_hip.so')
 # constants mirrored from include/yastn_hip.h
 YH_OK, YH_ERR_ARG, YH_ERR_HIP, YH_ERR_NUMERIC = 0, -1, -2, -3
 YH_F64, YH_C128 = 0, 1
-YH_ABI_VERSION = 16
+YH_ABI_VERSION = 17
 YH_MAXR = 8
 YH_JOB_WORDS = 32
 YH_JOB_BUFFER_WORD = 30
@@ -33,6 +33,7 @@ YH_SMALL_Q = 32
 YH_QR_WORDS = 8
 YH_SPLITK_WORDS = 8
 YH_QR_NB = 32
+YH_CHECK_SCRATCH = 256
 YH_QROP_WORDS = 3
 YH_QRADJ_WORDS = 8
 YH_SVD_LDS_BYTES = 131072
@@ -73,6 +74,7 @@ _SIGS = {
     'yastn_hip_eigh': [_p, _p, _p, _i32, _p, _i64, _p, _i64, _i64, _p, _p, _i32, _p],
     'yastn_hip_check_small_plan': [_p, _i64, _p, _i64, _i32, _i32, _i64],
     'yastn_hip_jacobi_small': [_p, _p, _p, _p, _i32, _i32, _p, _p, _i64, _i64, _p, _i32, _p],
+    'yastn_hip_check_result': [_p, _i64, _p, _i64, _p, _i64, _i32, _p],
     'yastn_hip_fix_svd_signs': [_p, _p, _i32, _p, _i64, _p],
     'yastn_hip_device_info': [_p, _p],
     'yastn_hip_svd_panel_init': [_p, _p, _p, _p, _i32, _i32, _p, _p, _i64, _p],

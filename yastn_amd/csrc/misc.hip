@@ -35,11 +35,14 @@ struct Z<true> {
 constexpr int kSplit = 16;
 
 // fix_svd_signs.  Blocks given as SVD plan words (0 a_off, 1 m, 2 n, 3 u_off, 4 s_off, 5 v_off);
-// U block m x k, Vh block k x n.  A workgroup takes 64-column chunks of U: lane = column (coalesced
-// row reads), wave = stripe of rows; per column the argmax of int64(|U[r, j]| * 2^40) with ties to the
-// smallest row, then the phase is applied to U[:, j] and Vh[j, :].
+// U block m x k, Vh block k x n.  A workgroup takes 16 columns of U at a time, thread (tid / 16, tid % 16) every 16th
+// row of one of them, four loads in flight: per column the argmax of int64(|U[r, j]| * 2^40) with ties to the
+// smallest row, then the phase is applied to U[:, j] and Vh[j, :].  Bound by memory once enough loads are in flight:
+// with 64 columns per workgroup and one load at a time it took 43 us on 27 real blocks of up to 198 columns and 616 on
+// 19 complex ones of up to 1134, now 12 and 129.
 // With piv != nullptr only the pivot positions are written: piv[s_off + j] = flat index of the pivot
 // of column j in U (the caller applies the phases with differentiable tensor ops).
+constexpr int kSignCols = 16, kSignRows = kThreads / kSignCols;
 template <bool CPLX>
 __global__ void __launch_bounds__(kThreads) fix_signs_kernel(typename Z<CPLX>::T* __restrict__ U,
                                                              typename Z<CPLX>::T* __restrict__ Vh,
@@ -47,33 +50,39 @@ __global__ void __launch_bounds__(kThreads) fix_signs_kernel(typename Z<CPLX>::T
                                                              int64_t* __restrict__ piv) {
   typedef Z<CPLX> N;
   typedef typename N::T T;
-  constexpr int kW = kThreads / 64;
-  __shared__ int64_t s_best[kW][64];
-  __shared__ int64_t s_row[kW][64];
-  __shared__ double s_ph[2][64];
-  const int64_t* w = blocks + (int64_t)(blockIdx.x / kSplit) * YH_SVD_WORDS;
-  const int split = blockIdx.x % kSplit;
+  constexpr int UN = 4;
+  __shared__ int64_t s_best[kSignRows][kSignCols];
+  __shared__ int64_t s_row[kSignRows][kSignCols];
+  __shared__ double s_ph[2][kSignCols];
+  const int64_t* w = blocks + (int64_t)blockIdx.x * YH_SVD_WORDS;
   const int64_t m = w[1], n = w[2], u_off = w[3], s_off = w[4], v_off = w[5];
   const int64_t k = m < n ? m : n;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t c0 = (int64_t)split * 64; c0 < k; c0 += (int64_t)kSplit * 64) {
-    const int64_t j = c0 + lane;
+  const int c = threadIdx.x % kSignCols, g = threadIdx.x / kSignCols;
+  for (int64_t c0 = (int64_t)blockIdx.y * kSignCols; c0 < k; c0 += (int64_t)gridDim.y * kSignCols) {
+    const int64_t j = c0 + c, jc = j < k ? j : k - 1;
     int64_t best = -1, brow = 0;
-    if (j < k) {
-      for (int64_t r = wave; r < m; r += kW) {
-        const int64_t qv = (int64_t)(N::absv(U[u_off + r * k + j]) * 1099511627776.0);
-        if (qv > best) {
+    for (int64_t r0 = g; r0 < m; r0 += kSignRows * UN) {
+      T u[UN];
+#pragma unroll
+      for (int x = 0; x < UN; ++x) {  // rows past the block read its last one
+        const int64_t r = r0 + kSignRows * x;
+        u[x] = U[u_off + (r < m ? r : m - 1) * k + jc];
+      }
+#pragma unroll
+      for (int x = 0; x < UN; ++x) {
+        const int64_t qv = (int64_t)(N::absv(u[x]) * 1099511627776.0), r = r0 + kSignRows * x;
+        if (qv > best && r < m) {
           best = qv;
           brow = r;
         }
       }
     }
-    s_best[wave][lane] = best;
-    s_row[wave][lane] = brow;
+    s_best[g][c] = best;
+    s_row[g][c] = brow;
     __syncthreads();
-    if (wave == 0) {
-      for (int x = 1; x < kW; ++x) {
-        const int64_t ob = s_best[x][lane], orow = s_row[x][lane];
+    if (g == 0) {
+      for (int x = 1; x < kSignRows; ++x) {
+        const int64_t ob = s_best[x][c], orow = s_row[x][c];
         if (ob > best || (ob == best && orow < brow)) {
           best = ob;
           brow = orow;
@@ -85,31 +94,105 @@ __global__ void __launch_bounds__(kThreads) fix_signs_kernel(typename Z<CPLX>::T
         } else {
           const T pv = U[u_off + brow * k + j];
           const double a = N::absv(pv);
-          s_ph[0][lane] = N::re(pv) / a;
-          s_ph[1][lane] = N::im(pv) / a;
+          s_ph[0][c] = N::re(pv) / a;
+          s_ph[1][c] = N::im(pv) / a;
         }
       }
     }
     __syncthreads();
     if (!piv) {
-      const int64_t nc = (k - c0) < 64 ? (k - c0) : 64;
-      if (lane < nc) {
-        const double pr = s_ph[0][lane], pi = s_ph[1][lane];
-        for (int64_t r = wave; r < m; r += kW) {  // u * conj(phase)
-          const T u = U[u_off + r * k + j];
-          U[u_off + r * k + j] = N::mk(N::re(u) * pr + N::im(u) * pi, N::im(u) * pr - N::re(u) * pi);
+      if (j < k) {
+        const double pr = s_ph[0][c], pi = s_ph[1][c];
+        for (int64_t r0 = g; r0 < m; r0 += kSignRows * UN) {  // u * conj(phase)
+          T u[UN];
+#pragma unroll
+          for (int x = 0; x < UN; ++x) {
+            const int64_t r = r0 + kSignRows * x;
+            u[x] = U[u_off + (r < m ? r : m - 1) * k + j];
+          }
+#pragma unroll
+          for (int x = 0; x < UN; ++x) {
+            const int64_t r = r0 + kSignRows * x;
+            if (r < m)
+              U[u_off + r * k + j] =
+                  N::mk(N::re(u[x]) * pr + N::im(u[x]) * pi, N::im(u[x]) * pr - N::re(u[x]) * pi);
+          }
         }
       }
-      for (int64_t l = wave; l < nc; l += kW) {  // Vh row c0 + l times phase
-        const double pr = s_ph[0][l], pi = s_ph[1][l];
-        T* row = Vh + v_off + (c0 + l) * n;
-        for (int64_t c = lane; c < n; c += 64) {
-          const T v = row[c];
-          row[c] = N::mk(N::re(v) * pr - N::im(v) * pi, N::im(v) * pr + N::re(v) * pi);
+      const int64_t nv = ((k - c0) < kSignCols ? k - c0 : kSignCols) * n;  // Vh rows c0 + l times phase
+      T* rows = Vh + v_off + c0 * n;
+      for (int64_t e0 = threadIdx.x; e0 < nv; e0 += kThreads * UN) {
+        T v[UN];
+#pragma unroll
+        for (int x = 0; x < UN; ++x) {
+          const int64_t e = e0 + kThreads * x;
+          v[x] = rows[e < nv ? e : nv - 1];
+        }
+#pragma unroll
+        for (int x = 0; x < UN; ++x) {
+          const int64_t e = e0 + kThreads * x;
+          if (e >= nv) continue;
+          const int64_t l = e / n;
+          const double pr = s_ph[0][l], pi = s_ph[1][l];
+          rows[e] = N::mk(N::re(v[x]) * pr - N::im(v[x]) * pi, N::im(v[x]) * pr + N::re(v[x]) * pi);
         }
       }
     }
     __syncthreads();
+  }
+}
+
+// What the host reads after a decomposition: out[0] = min(info), out[1] = the number of negative info words, out[2] = 1
+// if an element of the input is inf or NaN.  part[i] is the finding of workgroup i of the first kernel.  Two launches of 3-5 us for
+// a bond of 78 or 1024 (bound by memory from some MB on: 32 us at 211 MB) in place of eight of tensor operations, whose
+// launches took 60 us of the host.
+constexpr int kCheckBlocks = YH_CHECK_SCRATCH;
+__global__ void __launch_bounds__(kThreads) finite_parts_kernel(const double* __restrict__ x, int64_t n,
+                                                                int32_t* __restrict__ part) {
+  __shared__ int s_bad;
+  if (threadIdx.x == 0) s_bad = 0;
+  __syncthreads();
+  bool bad = false;
+  constexpr int UN = 4;
+  const int64_t step = (int64_t)gridDim.x * kThreads;
+  for (int64_t e0 = (int64_t)blockIdx.x * kThreads + threadIdx.x; e0 < n; e0 += step * UN) {
+    double v[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) v[u] = x[e0 + u * step < n ? e0 + u * step : e0];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) bad |= !isfinite(v[u]);
+  }
+  if (__any(bad) && (threadIdx.x & 63) == 0) s_bad = 1;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = s_bad;
+}
+
+__global__ void __launch_bounds__(kThreads) check_info_kernel(const int32_t* __restrict__ info, int64_t n,
+                                                              const int32_t* __restrict__ part, int parts,
+                                                              int32_t* __restrict__ out) {
+  __shared__ int s_lo[kThreads], s_neg[kThreads], s_bad[kThreads];
+  int lo = INT32_MAX, neg = 0, bad = 0;
+  for (int64_t i = threadIdx.x; i < n; i += kThreads) {
+    lo = min(lo, info[i]);
+    neg += info[i] < 0;
+  }
+  for (int i = threadIdx.x; i < parts; i += kThreads) bad |= part[i];
+  s_lo[threadIdx.x] = lo;
+  s_neg[threadIdx.x] = neg;
+  s_bad[threadIdx.x] = bad;
+  __syncthreads();
+  for (int h = kThreads / 2; h > 0; h /= 2) {
+    if ((int)threadIdx.x < h) {
+      s_lo[threadIdx.x] = min(s_lo[threadIdx.x], s_lo[threadIdx.x + h]);
+      s_neg[threadIdx.x] += s_neg[threadIdx.x + h];
+      s_bad[threadIdx.x] |= s_bad[threadIdx.x + h];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    out[0] = s_lo[0];
+    out[1] = s_neg[0];
+    out[2] = s_bad[0];
   }
 }
 
@@ -338,17 +421,27 @@ extern "C" int yastn_hip_dot_diag_adjoint_a(void* gA, const void* g, const void*
   return yh::hip_status(hipGetLastError(), "dot_diag adjoint launch");
 }
 
+namespace {
+
+template <bool CPLX>
+int launch_fix_signs(void* U, void* Vh, const int64_t* d_blocks, int64_t nblocks, int64_t* piv, hipStream_t stream,
+                     const char* what) {
+  typedef typename Z<CPLX>::T T;
+  // workgroups per block: about 2048 in all, none with less than 16 columns of the largest blocks
+  const unsigned slices = (unsigned)std::min<int64_t>(128, std::max<int64_t>(4, 2048 / nblocks));
+  hipLaunchKernelGGL(fix_signs_kernel<CPLX>, dim3((unsigned)nblocks, slices), dim3(kThreads), 0, stream, (T*)U, (T*)Vh,
+                     d_blocks, piv);
+  return yh::hip_status(hipGetLastError(), what);
+}
+
+}  // namespace
+
 extern "C" int yastn_hip_fix_svd_signs(void* U, void* Vh, int dtype, const int64_t* d_blocks, int64_t nblocks,
                                        hipStream_t stream) {
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
   if (nblocks == 0) return YH_OK;
-  if (dtype == YH_F64)
-    hipLaunchKernelGGL(fix_signs_kernel<false>, dim3((unsigned)(nblocks * kSplit)), dim3(kThreads), 0, stream, (double*)U,
-                       (double*)Vh, d_blocks, (int64_t*)nullptr);
-  else
-    hipLaunchKernelGGL(fix_signs_kernel<true>, dim3((unsigned)(nblocks * kSplit)), dim3(kThreads), 0, stream, (double2*)U,
-                       (double2*)Vh, d_blocks, (int64_t*)nullptr);
-  return yh::hip_status(hipGetLastError(), "fix_svd_signs launch");
+  return dtype == YH_F64 ? launch_fix_signs<false>(U, Vh, d_blocks, nblocks, nullptr, stream, "fix_svd_signs launch")
+                         : launch_fix_signs<true>(U, Vh, d_blocks, nblocks, nullptr, stream, "fix_svd_signs launch");
 }
 
 extern "C" int yastn_hip_svd_sign_pivots(const void* U, int64_t* piv, int dtype, const int64_t* d_blocks,
@@ -356,13 +449,23 @@ extern "C" int yastn_hip_svd_sign_pivots(const void* U, int64_t* piv, int dtype,
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
   YH_CHECK_ARG(piv != nullptr, "null pivot buffer");
   if (nblocks == 0) return YH_OK;
-  if (dtype == YH_F64)
-    hipLaunchKernelGGL(fix_signs_kernel<false>, dim3((unsigned)(nblocks * kSplit)), dim3(kThreads), 0, stream,
-                       (double*)const_cast<void*>(U), (double*)nullptr, d_blocks, piv);
-  else
-    hipLaunchKernelGGL(fix_signs_kernel<true>, dim3((unsigned)(nblocks * kSplit)), dim3(kThreads), 0, stream,
-                       (double2*)const_cast<void*>(U), (double2*)nullptr, d_blocks, piv);
-  return yh::hip_status(hipGetLastError(), "svd_sign_pivots launch");
+  void* u = const_cast<void*>(U);
+  return dtype == YH_F64 ? launch_fix_signs<false>(u, nullptr, d_blocks, nblocks, piv, stream, "svd_sign_pivots launch")
+                         : launch_fix_signs<true>(u, nullptr, d_blocks, nblocks, piv, stream, "svd_sign_pivots launch");
+}
+
+extern "C" int yastn_hip_check_result(int32_t* out, int64_t out_numel, const int32_t* info, int64_t nblocks,
+                                      const void* data, int64_t numel, int dtype, hipStream_t stream) {
+  YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
+  YH_CHECK_ARG(nblocks >= 0 && numel >= 0 && out_numel >= 3 + kCheckBlocks, "sizes %lld, %lld, %lld",
+               (long long)nblocks, (long long)numel, (long long)out_numel);
+  const int64_t n = numel * (dtype == YH_C128 ? 2 : 1);
+  const int parts = (int)std::min<int64_t>(kCheckBlocks, yh::cdiv(n, kThreads));
+  if (parts > 0)
+    hipLaunchKernelGGL(finite_parts_kernel, dim3((unsigned)parts), dim3(kThreads), 0, stream, (const double*)data, n,
+                       out + 3);
+  hipLaunchKernelGGL(check_info_kernel, dim3(1), dim3(kThreads), 0, stream, info, nblocks, out + 3, parts, out);
+  return yh::hip_status(hipGetLastError(), "check result launch");
 }
 
 extern "C" int yastn_hip_svd_adjoint_core(void* J, void* T, const void* X, const void* Y, const void* S,
