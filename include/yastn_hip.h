@@ -35,7 +35,7 @@ extern "C" {
 #define YH_F64 0
 #define YH_C128 1
 
-#define YH_ABI_VERSION 17
+#define YH_ABI_VERSION 18
 
 /* ---- box-gather plan (one job per copied or zero-filled box) -------------
  * int64 words per job (YH_JOB_WORDS):
@@ -273,11 +273,10 @@ int yastn_hip_grouped_gemm_noalloc(void* const* outs, const void* const* ins, in
 #define YH_QR_WORDS 8
 #define YH_QR_NB 32
 int yastn_hip_check_qr_plan(const int64_t* h_qdesc, const int64_t* h_blocks, const int32_t* h_ids, int64_t n,
-                            int dtype, int64_t work_numel, int64_t lds_bytes);
-/* Factor panel `step` (columns step*YH_QR_NB ...) of every listed block: staged in LDS when
- * lds_bytes >= p*YH_QR_NB*itemsize for every block, in place in the workspace when lds_bytes == 0. */
+                            int dtype, int64_t work_numel);
+/* Factor panel `step` (columns step*YH_QR_NB ...) of every listed block, none of more than max_rows rows (p). */
 int yastn_hip_svd_qr_panel(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, int step,
-                           int64_t lds_bytes, hipStream_t stream);
+                           int64_t max_rows, hipStream_t stream);
 /* Block reflectors applied in one launch, 16 columns per workgroup, in place of three grouped GEMMs per panel:
  * trailing: the columns of W0 right of panel `step` (after yastn_hip_svd_qr_panel of that step), of the listed blocks;
  * svd_reflect: the p-side vectors that yastn_hip_svd_precond_finalize started, by all panels, last first;
@@ -312,8 +311,7 @@ int yastn_hip_svd_precond_finalize(void* U, void* S, void* Vh, void* work, int d
  * 0 a_off, 1 q_off, 2 r_off, element offsets of the row-major blocks. */
 #define YH_QROP_WORDS 3
 int yastn_hip_check_qr_op_plan(const int64_t* h_qdesc, const int64_t* h_qblocks, int64_t nblocks, int dtype,
-                               int64_t a_numel, int64_t q_numel, int64_t r_numel, int64_t work_numel,
-                               int64_t lds_bytes);
+                               int64_t a_numel, int64_t q_numel, int64_t r_numel, int64_t work_numel);
 /* W0 = A (column-major), E = [I_k; 0]. */
 int yastn_hip_qr_init(const void* A, void* work, int dtype, const int64_t* d_qdesc, const int64_t* d_qblocks,
                       int64_t nblocks, hipStream_t stream);

@@ -63,7 +63,7 @@ def test_svd_reflectors(shapes, cplx):
            plan.d_qdesc.data_ptr(), plan.d_pre.data_ptr(), plan.n_pre, st)
     for step, (d_ids, n, rest) in enumerate(plan.panel_steps):
         L.call('yastn_hip_svd_qr_panel', work.data_ptr(), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step,
-               plan.qr_lds, st)
+               plan.qr_rows, st)
         trail = plan.qr_steps[step][2]
         assert (trail is not None) == (rest > 0)
         if trail is None:

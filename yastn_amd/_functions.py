@@ -603,7 +603,7 @@ def _householder_steps(plan, work, dt, st):
     """The panel steps of a batched Householder QR (plans.SvdPlan / QrPlan): the panels of all blocks in one launch,
     then their reflectors on the columns to their right in another."""
     for step, (d_ids, n, rest) in enumerate(plan.panel_steps):
-        L.call('yastn_hip_svd_qr_panel', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step, plan.qr_lds, st)
+        L.call('yastn_hip_svd_qr_panel', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step, plan.qr_rows, st)
         if rest:
             L.call('yastn_hip_reflect_trailing', ptr(work), dt, plan.d_qdesc.data_ptr(), d_ids.data_ptr(), n, step, rest,
                    st)

@@ -63,11 +63,12 @@ __device__ __attribute__((always_inline)) inline double2 pick(bool c, double2 a,
 
 // Wave-wide reductions: DPP moves within each row of 16 lanes (quad_perm [1,0,3,2], quad_perm
 // [2,3,0,1], row_half_mirror, row_mirror: after the four steps every lane holds its row's value),
-// then the four row values are read into scalar registers, so the result is wave-uniform.
+// then the four row values are read into scalar registers, so the result is wave-uniform.  (Every lane of these moves
+// has a source; with bound_ctrl set the compiler need not clear the destination first.)
 template <int CTRL>
 __device__ __attribute__((always_inline)) inline double dpp_move(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
 
@@ -1880,13 +1881,12 @@ __device__ __attribute__((always_inline)) inline void scale_column(typename Num<
   if (tid == 0) xp[j - 1] = N::make(beta, 0.0);
 }
 
-// The column loop of the panel factorisation, one workgroup barrier per column.  Column j's reflector
+// The column loop of a panel factored in place, one workgroup barrier per column.  Column j's reflector
 // is applied to the later columns with v = [1; s x[j+1:]] formed on the fly from the unscaled column
 // (the same products as scaling first); the column itself is scaled during the next column's update,
 // which does not read it.  The wave that updates column j + 1 also sums the squares of its new tail,
 // the next reflector's norm, so that no block-wide reduction sits in the loop.
-// qr_columns_mem: every column update reads and writes the panel (LDS or, in place, global memory),
-// one wave per later column.
+// Every column update reads and writes the panel in global memory, one wave per later column.
 template <bool CPLX>
 __device__ __attribute__((always_inline)) inline void qr_columns_mem(typename Num<CPLX>::T* P, int64_t ld,
                                                                      int64_t L, int nb, double xn2, double* s_tr,
@@ -1942,199 +1942,362 @@ __device__ __attribute__((always_inline)) inline void qr_columns_mem(typename Nu
   scale_column<CPLX>(P + (int64_t)(nb - 1) * ld, nb, L, pscr, psci, pbeta, tid);
 }
 
-// Rows per lane of the register instance for the largest LDS-resident panels.
-template <bool CPLX>
-constexpr int kRegRows = CPLX ? 5 : 9;
+constexpr int64_t kQrMaxRows = (int64_t)1 << 27;  // rows x YH_QR_NB panel elements < 2^32 (32-bit indices)
 
-// qr_columns_reg (panel in LDS, L <= 64 RPL): column c stays in the registers of wave c % kWaves
-// (slot c / kWaves; lane l holds rows l + 64 u) until it becomes the reflector; its owner writes it
-// back to the LDS panel one iteration earlier, so every column is in the LDS when it is read as a
-// reflector and the LDS traffic of a column step is one read of the reflector per wave.
-template <bool CPLX, int RPL>
-__device__ __attribute__((always_inline)) inline void qr_columns_reg(typename Num<CPLX>::T* P, int64_t ld,
-                                                                     int64_t L, int nb, double xn2, double* s_tr,
-                                                                     double* s_ti, double* s_nrm, int tid, int lane,
-                                                                     int wave) {
+// house_coeffs in a shorter chain of dependent operations: 1 / beta and 1 / |alpha - beta|^2 from the hardware
+// approximations (2^-23) and two Newton-Raphson steps each, the norm corrected once more, all to rounding; squares near
+// the ends of the exponent range take house_coeffs itself.
+template <bool CPLX>
+__device__ __attribute__((always_inline)) inline void house_coeffs_short(typename Num<CPLX>::T alpha, double xn2,
+                                                                         double& beta, double& taur, double& taui,
+                                                                         double& scr, double& sci) {
+  typedef Num<CPLX> N;
+  const double t = N::abs2(alpha) + xn2;
+  if (!(xn2 > 0.0 && t > 1e-280 && t < 1e280)) {
+    house_coeffs<CPLX>(alpha, xn2, beta, taur, taui, scr, sci);
+    return;
+  }
+  double r = __builtin_amdgcn_rsq(t);
+  r = fma(0.5 * r, fma(-t * r, r, 1.0), r);
+  r = fma(0.5 * r, fma(-t * r, r, 1.0), r);
+  double nrm = t * r;
+  nrm = fma(0.5 * r, fma(-nrm, nrm, t), nrm);
+  const bool pos = N::re(alpha) >= 0.0;
+  beta = pos ? -nrm : nrm;
+  const double rb = pos ? -r : r;
+  taur = (beta - N::re(alpha)) * rb;
+  taui = -N::im(alpha) * rb;
+  const double dr = N::re(alpha) - beta, di = N::im(alpha);
+  const double den = dr * dr + di * di;
+  double w = __builtin_amdgcn_rcp(den);
+  w = fma(w, fma(-den, w, 1.0), w);
+  w = fma(w, fma(-den, w, 1.0), w);
+  scr = dr * w;
+  sci = -di * w;
+}
+
+// The panel factorisation in registers, 8 waves: G = 16, 32 or 64 lanes hold a column, so a pass takes 512 / G columns,
+// column c0 + t in lanes G t ..., lane g of it holding rows g + G u, u < RPL.  What bounds it is the number of
+// instructions from one reflector to the next (each of a wave's goes to all 64 / G columns of it): every lane reads its rows
+// of the unscaled reflector x from LDS once, forms |x|^2 and x^H y for its column together (v^H y = y_j + conj(s) x^H y
+// needs no scaling of x first), sums both over the G lanes, then the coefficients, and updates; the next column goes to
+// the other LDS buffer, and there is one barrier.  A column goes to memory from its registers when its pass is done.
+// Panels too tall for 32 columns in the registers take passes of 16 or 8, each after the reflectors of the passes before
+// it (read back from Vall), which need no barrier.
+// Means over the panels of a decomposition: 62 us with 16 waves, whole waves per column, the panel in LDS, two chained
+// reductions per column and IEEE divisions, 45 now (seven real blocks of up to 440 rows; 60 with this step but whole waves
+// per column, each wave issuing it for four columns in turn); 50 -> 36 (27 real blocks of up to 198 rows);
+// 280 -> 125 (19 complex blocks of up to 1134 rows, which were factored in place in memory).
+constexpr int kQrWaves = 8, kQrThreads = 64 * kQrWaves;
+
+// Sum over groups of G lanes, in all of them.
+template <int G>
+__device__ __attribute__((always_inline)) inline double group_sum(double v) {
+  if constexpr (G == 64) return wave_sum(v);
+  v += dpp_move<0xB1>(v);
+  v += dpp_move<0x4E>(v);
+  v += dpp_move<0x141>(v);
+  v += dpp_move<0x140>(v);
+  if constexpr (G == 32) v += __shfl_xor(v, 16);
+  return v;
+}
+
+// r += conj(x) y; y - x f; x f.  For real data no products with imaginary parts, which are zeros that the compiler may
+// not drop: they doubled the instructions and the registers of the loops below.
+template <bool CPLX>
+__device__ __attribute__((always_inline)) inline void add_dot(double& r, double& i, typename Num<CPLX>::T x,
+                                                              typename Num<CPLX>::T y) {
+  if constexpr (CPLX) {
+    r = fma(x.y, y.y, fma(x.x, y.x, r));
+    i = fma(-x.y, y.x, fma(x.x, y.y, i));
+  } else {
+    r = fma(x, y, r);
+  }
+}
+
+template <bool CPLX>
+__device__ __attribute__((always_inline)) inline typename Num<CPLX>::T sub_mul(typename Num<CPLX>::T y,
+                                                                               typename Num<CPLX>::T x, double fr,
+                                                                               double fi) {
+  if constexpr (CPLX)
+    return make_double2(fma(x.y, fi, fma(-x.x, fr, y.x)), fma(-x.y, fr, fma(-x.x, fi, y.y)));
+  else
+    return fma(-x, fr, y);
+}
+
+template <bool CPLX>
+__device__ __attribute__((always_inline)) inline typename Num<CPLX>::T mul_by(typename Num<CPLX>::T x, double fr,
+                                                                              double fi) {
+  if constexpr (CPLX)
+    return make_double2(fma(-x.y, fi, x.x * fr), fma(x.y, fr, x.x * fi));
+  else
+    return x * fr;
+}
+
+template <bool CPLX, int G, int RPL>
+__device__ __attribute__((always_inline)) inline void qr_pass(typename Num<CPLX>::T* __restrict__ W,
+                                                              typename Num<CPLX>::T* __restrict__ V, int64_t p,
+                                                              int L, int nb, int c0, typename Num<CPLX>::T* s_x,
+                                                              int xs, double* s_tr, double* s_ti, double* s_co,
+                                                              int tid) {
   typedef Num<CPLX> N;
   typedef typename N::T T;
-  constexpr int NS = YH_QR_NB / kWaves;  // column slots per wave
-  const T one = N::make(1.0, 0.0), zero = N::make(0.0, 0.0);
-  T Y[NS][RPL];
-#pragma unroll
-  for (int sl = 0; sl < NS; ++sl) {
-    const int c = wave + kWaves * sl;
-    const int64_t cc = c < nb ? c : nb - 1;
+  constexpr int NU = G < 32 ? 32 / G : 1;  // the slots that rows 0 .. 31 lie in
+  const T zero = N::make(0.0, 0.0);
+  const int c = c0 + tid / G, cend = min(nb, c0 + kQrThreads / G), g = tid & (G - 1), lane = tid & 63;
+  const bool mine = c < nb;
+  // rows g + G u of a column, at a copy of g that the compiler takes for a new value wherever a group of accesses
+  // starts: it would keep the addresses of all rows in registers otherwise
+  auto fresh = [&] {
+    int x = g;
+    asm volatile("" : "+v"(x));
+    return x;
+  };
+  auto row = [&](int x, int u) { return (int64_t)min(x + G * u, L - 1); };
+  T Y[RPL];
+  {
+    const T* col = W + (int64_t)min(c, nb - 1) * p;
+    const int x = fresh();
 #pragma unroll
     for (int u = 0; u < RPL; ++u) {
-      const int64_t r = lane + 64 * u;
-      const T v = P[(r < L ? r : L - 1) + cc * ld];
-      Y[sl][u] = ((c < nb) & (r < L)) ? v : zero;
+      const T v = col[row(x, u)];
+      Y[u] = pick(mine & (x + G * u < L), v, zero);
     }
   }
-  double pscr = 0.0, psci = 0.0, pbeta = 0.0;
-  for (int j = 0; j < nb; ++j) {
-    const T* x = P + (int64_t)j * ld;
-    if (j > 0) xn2 = s_nrm[j & 1];
-    const T alpha = x[j];
+#pragma unroll 1
+  for (int j = 0; j < c0; ++j) {  // the reflectors of the earlier passes: v = column j of V, zeros and one included
+    const T* vj = V + (int64_t)j * p;
+    const int x = fresh();
+    T v[RPL];
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) {
+      const T e = vj[row(x, u)];
+      v[u] = pick(x + G * u < L, e, zero);
+    }
+    double wr = 0.0, wi = 0.0;
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) add_dot<CPLX>(wr, wi, v[u], Y[u]);
+    wr = group_sum<G>(wr);
+    if constexpr (CPLX) wi = group_sum<G>(wi);
+    const T cw = mul_by<CPLX>(N::make(wr, wi), s_tr[j], CPLX ? -s_ti[j] : 0.0);  // conj(tau) v^H y
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) Y[u] = sub_mul<CPLX>(Y[u], v[u], N::re(cw), N::im(cw));
+  }
+  auto publish = [&](int j) {  // column j, if it is this lane's, into its LDS buffer
+    if (c == j) {
+      T* xn = s_x + (j & 1) * xs + g;
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) xn[G * u] = Y[u];
+    }
+  };
+  publish(c0);
+  __syncthreads();
+#pragma unroll 1
+  for (int j = c0; j < cend; ++j) {
+    const T* xj = s_x + (j & 1) * xs;
+    T x[RPL];
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) x[u] = xj[g + G * u];
+    const T alpha = xj[j];
+    // y_j of this column, from the lane that holds row j
+    T yj = Y[0];
+    if constexpr (NU == 2) yj = pick(j >= G, Y[1], yj);
+    const int from = (lane & ~(G - 1)) + (j & (G - 1));
+    const double yr = __shfl(N::re(yj), from), yi = CPLX ? __shfl(N::im(yj), from) : 0.0;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) x[u] = pick(g + G * u > j, x[u], zero);  // rows below j
+    double n2 = 0.0, dr = 0.0, di = 0.0;
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) {
+      if constexpr (CPLX)
+        n2 = fma(x[u].x, x[u].x, fma(x[u].y, x[u].y, n2));
+      else
+        n2 = fma(x[u], x[u], n2);
+      add_dot<CPLX>(dr, di, x[u], Y[u]);
+    }
+    n2 = group_sum<G>(n2);
+    dr = group_sum<G>(dr);
+    if constexpr (CPLX) di = group_sum<G>(di);
     double beta, taur, taui, scr, sci;
-    house_coeffs<CPLX>(alpha, xn2, beta, taur, taui, scr, sci);
-    if (j > 0) scale_column<CPLX>(P + (int64_t)(j - 1) * ld, j, L, pscr, psci, pbeta, tid);
-    if (tid == 0) {
+    house_coeffs_short<CPLX>(alpha, n2, beta, taur, taui, scr, sci);
+    if (!(n2 < HUGE_VAL)) {  // an infinity or NaN spoils the later columns (through taur), not the earlier ones
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) x[u] = zero;
+    }
+    const T sd = mul_by<CPLX>(N::make(dr, di), scr, -sci);  // conj(s) x^H y
+    const T w = N::make(yr + N::re(sd), yi + N::im(sd));    // v^H y
+    const T cw = mul_by<CPLX>(w, taur, -taui), fw = mul_by<CPLX>(cw, scr, sci);
+    // columns up to j are updated by zero: a branch around the update would keep two copies of Y in registers
+    const T cc = pick(c > j, cw, zero), f = pick(c > j, fw, zero);
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) Y[u] = sub_mul<CPLX>(Y[u], x[u], N::re(f), N::im(f));
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const T d = pick(g + G * u == j, cc, zero);
+      Y[u] = N::make(N::re(Y[u]) - N::re(d), N::im(Y[u]) - N::im(d));
+    }
+    publish(j + 1);
+    if (c == j && g == 0) {
+      s_co[j] = beta;
+      s_co[32 + j] = scr;
+      s_co[64 + j] = sci;
       s_tr[j] = taur;
       s_ti[j] = taui;
     }
-    if (wave + kWaves * (NS - 1) > j) {  // wave-uniform: this wave owns a later column
-      T v[RPL];  // v = [0 above j; 1; s x[j+1:]]
+    __syncthreads();  // the next reflector is visible; the buffer of this one may be overwritten
+  }
+  if (mine) {  // [R above; beta; 0] and [0; 1; s x]: the column below the diagonal was left unscaled
+    T *wc = W + (int64_t)c * p, *vc = V + (int64_t)c * p;
+    const double beta = s_co[c], scr = s_co[32 + c], sci = s_co[64 + c];
+    const int x = fresh();
 #pragma unroll
-      for (int u = 0; u < RPL; ++u) {
-        const int64_t r = lane + 64 * u;
-        const T xr = x[r < L ? r : L - 1];
-        const T sx = N::make(N::re(xr) * scr - N::im(xr) * sci, N::re(xr) * sci + N::im(xr) * scr);
-        v[u] = ((r > j) & (r < L)) ? sx : (r == j ? one : zero);
-      }
-#pragma unroll
-      for (int sl = 0; sl < NS; ++sl) {
-        const int c = wave + kWaves * sl;
-        if (c > j && c < nb) {  // wave-uniform
-          double wr = 0.0, wi = 0.0;  // w = v^H y
-#pragma unroll
-          for (int u = 0; u < RPL; ++u) {
-            wr += N::re(v[u]) * N::re(Y[sl][u]) + N::im(v[u]) * N::im(Y[sl][u]);
-            if constexpr (CPLX) wi += N::re(v[u]) * N::im(Y[sl][u]) - N::im(v[u]) * N::re(Y[sl][u]);
-          }
-          wr = wave_sum(wr);
-          if constexpr (CPLX) wi = wave_sum(wi);
-          const double cr = taur * wr + taui * wi, ci = taur * wi - taui * wr;  // conj(tau) w
-          double loc = 0.0;
-#pragma unroll
-          for (int u = 0; u < RPL; ++u) {
-            const int64_t r = lane + 64 * u;
-            Y[sl][u] = N::make(N::re(Y[sl][u]) - (N::re(v[u]) * cr - N::im(v[u]) * ci),
-                               N::im(Y[sl][u]) - (N::re(v[u]) * ci + N::im(v[u]) * cr));
-            loc += r > j + 1 ? N::abs2(Y[sl][u]) : 0.0;  // rows past L hold zeros
-          }
-          if (c == j + 1) {  // the next reflector: its tail norm, and the column itself into the LDS
-            loc = wave_sum(loc);
-            if (lane == 0) s_nrm[(j + 1) & 1] = loc;
-            T* y = P + (int64_t)c * ld;
-#pragma unroll
-            for (int u = 0; u < RPL; ++u) {
-              const int64_t r = lane + 64 * u;
-              if (r < L) y[r] = Y[sl][u];
-            }
-          }
-        }
+    for (int u = 0; u < RPL; ++u) {
+      const int r = x + G * u;
+      const T y = Y[u], v = mul_by<CPLX>(y, scr, sci);
+      if (r < L) {
+        wc[r] = u >= NU ? zero : pick(r < c, y, pick(r == c, N::make(beta, 0.0), zero));
+        vc[r] = u >= NU ? v : pick(r < c, zero, pick(r == c, N::make(1.0, 0.0), v));
       }
     }
-    pscr = scr;
-    psci = sci;
-    pbeta = beta;
-    __syncthreads();  // the next reflector and s_nrm visible; every thread has read alpha and s_nrm
   }
-  scale_column<CPLX>(P + (int64_t)(nb - 1) * ld, nb, L, pscr, psci, pbeta, tid);
 }
 
-constexpr int64_t kQrMaxRows = (int64_t)1 << 27;  // rows x YH_QR_NB panel elements < 2^32 (32-bit indices)
+// All passes of a panel in the registers' reach: 512 / G columns each.
+template <bool CPLX, int G, int RPL>
+__device__ __attribute__((always_inline)) inline void qr_passes(typename Num<CPLX>::T* W, typename Num<CPLX>::T* V,
+                                                                int64_t p, int L, int nb, typename Num<CPLX>::T* s_x,
+                                                                int xs, double* s_tr, double* s_ti, double* s_co,
+                                                                int tid) {
+  for (int c0 = 0; c0 < nb; c0 += kQrThreads / G) {
+    if (c0) __syncthreads();  // the reflectors and coefficients of the pass before are visible
+    qr_pass<CPLX, G, RPL>(W, V, p, L, nb, c0, s_x, xs, s_tr, s_ti, s_co, tid);
+  }
+}
+
+// Rows of the tallest panel the registers take (a lane has 256 VGPRs); taller ones are factored in place.
+template <bool CPLX>
+constexpr int kQrRegRows = 64 * (CPLX ? 23 : 46);
 
 // One panel of the blocked Householder QR (LAPACK geqrf / larfg / larft conventions): the
 // (p - k0) x nb panel at column k0 = step * YH_QR_NB is factored column by column,
 // H_j = I - tau_j v_j v_j^H with H_j^H x = beta e_1 (beta real), applying H_j^H to the panel's
 // later columns.  The vectors go to Vall, the R part back to W0, and -T, with H_1 ... H_nb =
-// I - V T V^H, to Tm.  The columns right of the panel are updated by grouped GEMMs on the host's plan.
-// The panel is staged in LDS (INPLACE false) or, when it does not fit, factored in place in W0
-// (leading dimension p; the workgroup's barriers order its global reads and writes, and the
-// panel of one block, a few hundred KB, stays in L2).
+// I - V T V^H, to Tm.  The columns right of the panel are updated by reflect_kernel.
+// INPLACE: the panel is factored in place in W0 (leading dimension p; the workgroup's barriers order its global reads
+// and writes), by 16 waves; else in registers (qr_pass), by 8.
 template <bool CPLX, bool INPLACE>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(INPLACE ? kThreads : kQrThreads)
     qr_panel_kernel(const int64_t* __restrict__ qdesc, const int32_t* __restrict__ ids,
                     typename Num<CPLX>::T* __restrict__ work, int step) {
   typedef Num<CPLX> N;
   typedef typename N::T T;
-  constexpr int NB = YH_QR_NB;
-  extern __shared__ double smem_raw[];
-  __shared__ double s_red[kWaves];
+  constexpr int NB = YH_QR_NB, NT = INPLACE ? kThreads : kQrThreads, NW = NT / 64;
   __shared__ double s_tr[NB], s_ti[NB];          // tau_j
   __shared__ double s_Zr[NB][NB], s_Zi[NB][NB];  // Z = V^H V (upper triangle), [row][col]
+  constexpr int kX = INPLACE ? 0 : 2 * kQrRegRows<CPLX>, kT = NB * (NB + 1);
+  __shared__ T s_x[kX > kT ? kX : kT];  // the reflectors, then T
+  T(*s_T)[NB + 1] = reinterpret_cast<T(*)[NB + 1]>(s_x);
   const QrDesc d = load_qr(qdesc + (int64_t)ids[blockIdx.x] * YH_QR_WORDS);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t k0 = (int64_t)step * NB;
   const int nb = (int)((d.k - k0) < NB ? (d.k - k0) : NB);
   const int64_t L = d.p - k0;
   const int64_t p = d.p;
-  T* W0 = work + d.w_off;
-  T* Vall = work + d.vall_off;
-  // the L x nb panel, column-major with leading dimension ld
-  const int64_t ld = INPLACE ? p : L;
-  T* P = INPLACE ? W0 + k0 + k0 * p : reinterpret_cast<T*>(smem_raw);
-  if (!INPLACE) {  // (the panel fits the LDS, so 32-bit element indices)
-    const uint32_t Lu = (uint32_t)L, n = (uint32_t)(L * nb);
-    for (uint32_t e = tid; e < n; e += kThreads) {
-      const uint32_t c = e / Lu, r = e - c * Lu;
-      P[e] = W0[(k0 + r) + (k0 + c) * p];
-    }
-    __syncthreads();
-  }
-  double xn2 = 0.0;
-  {
+  T* P = work + d.w_off + k0 + k0 * p;     // the L x nb panel, column-major with leading dimension p
+  T* V = work + d.vall_off + k0 + k0 * p;  // its reflectors
+  if constexpr (INPLACE) {
+    __shared__ double s_red[kWaves];
+    __shared__ double s_nrm[2];  // by column parity: column j's norm is read while j + 1's is written
     double loc = 0.0;
     for (int64_t r = 1 + tid; r < L; r += kThreads) loc += N::abs2(P[r]);
-    xn2 = block_sum(loc, s_red, lane, wave);
-  }
-  __shared__ double s_nrm[2];  // by column parity: column j's norm is read while j + 1's is written
-  bool done = false;
-  if constexpr (!INPLACE) {  // the later columns in registers (rows per lane: the smallest instance)
-    if (L <= 64 * 2) {
-      qr_columns_reg<CPLX, 2>(P, ld, L, nb, xn2, s_tr, s_ti, s_nrm, tid, lane, wave);
-      done = true;
-    } else if (!CPLX && L <= 64 * 4) {
-      qr_columns_reg<CPLX, 4>(P, ld, L, nb, xn2, s_tr, s_ti, s_nrm, tid, lane, wave);
-      done = true;
-    } else if (L <= 64 * kRegRows<CPLX>) {
-      qr_columns_reg<CPLX, kRegRows<CPLX>>(P, ld, L, nb, xn2, s_tr, s_ti, s_nrm, tid, lane, wave);
-      done = true;
+    const double xn2 = block_sum(loc, s_red, lane, wave);
+    qr_columns_mem<CPLX>(P, p, L, nb, xn2, s_tr, s_ti, s_nrm, tid, lane, wave);
+    __syncthreads();
+    for (int64_t e = tid; e < L * nb; e += kThreads) {
+      const int64_t c = (int64_t)((uint32_t)e / (uint32_t)L), r = e - c * L;  // L nb < 2^32 (q <= YH_SVD_MAX_Q)
+      const T v = P[r + c * p];
+      P[r + c * p] = pick(r <= c, v, N::make(0.0, 0.0));
+      V[r + c * p] = pick(r < c, N::make(0.0, 0.0), pick(r == c, N::make(1.0, 0.0), v));
     }
+  } else {
+    __shared__ double s_co[3 * NB];  // beta_j and s_j
+    constexpr int xs = kQrRegRows<CPLX>;
+    const int u = (int)((L + 63) / 64), l = (int)L;
+#define QR_PASSES(G, RPL) qr_passes<CPLX, G, RPL>(P, V, p, l, nb, s_x, xs, s_tr, s_ti, s_co, tid)
+    // the smallest instance in reach; a lane holds 2 RPL elements and at most 60 other registers
+    if constexpr (CPLX) {
+      if (u <= 1) QR_PASSES(16, 4);
+      else if (u <= 2) QR_PASSES(16, 8);
+      else if (l <= 208) QR_PASSES(16, 13);
+      else if (u <= 5) QR_PASSES(16, 20);
+      else if (u <= 6) QR_PASSES(16, 24);
+      else if (u <= 9) QR_PASSES(32, 18);
+      else if (u <= 12) QR_PASSES(32, 24);
+      else if (u <= 18) QR_PASSES(64, 18);
+      else QR_PASSES(64, 23);
+    } else {
+      if (u <= 1) QR_PASSES(16, 4);
+      else if (u <= 2) QR_PASSES(16, 8);
+      else if (l <= 208) QR_PASSES(16, 13);
+      else if (u <= 5) QR_PASSES(16, 20);
+      else if (u <= 7) QR_PASSES(16, 28);
+      else if (u <= 9) QR_PASSES(16, 36);
+      else if (u <= 12) QR_PASSES(16, 48);
+      else if (u <= 18) QR_PASSES(32, 36);
+      else if (u <= 24) QR_PASSES(32, 48);
+      else if (u <= 36) QR_PASSES(64, 36);
+      else QR_PASSES(64, 46);
+    }
+#undef QR_PASSES
   }
-  if (!done) qr_columns_mem<CPLX>(P, ld, L, nb, xn2, s_tr, s_ti, s_nrm, tid, lane, wave);
   __syncthreads();
   // T from T^-1 = diag(1 / tau) + striu(V^H V) (Joffrain, Low, Quintana-Orti, van de Geijn, Van Zee,
   // "Accumulating Householder transformations, revisited", ACM TOMS 32 (2006)): column j of T solves a
   // triangular system, T(j, j) = tau_j and T(i, j) = -tau_i sum_{i < l <= j} Z(i, l) T(l, j), Z = V^H V
   // (tau_i = 0 gives a zero row and column, as the larft recurrence does).
-  // Z's upper 16 x 16 tiles (00, 01, 11) are formed on the matrix cores by waves 0-11 (tile wave / 4,
-  // the rows cut into four parts whose products are summed in part order); then each wave solves two
-  // columns of T with no workgroup barrier, lanes 0-31 column wave and lanes 32-63 column wave + 16,
-  // lane l holding T(l, column).
+  // Z's upper 16 x 16 tiles (00, 01, 11) are formed on the matrix cores by the first 12 (of 8 waves: 6) waves (tile
+  // wave / parts, the rows cut into 4 (2) parts whose products are summed in part order).  The diagonal 16 x 16 blocks of T
+  // are solved for by 16 lanes per column, all columns at once, the block beside them by two products (whole
+  // columns of 32 by 32 lanes, two per wave at a time, took 8 us longer).
+  constexpr int PARTS = NW >= 12 ? 4 : 2;
   {
-    const int tile = wave >> 2, part = wave & 3;
+    const int tile = wave / PARTS, part = wave % PARTS;
     const int ti = tile == 2 ? 1 : 0, tj = tile == 0 ? 0 : 1;
     const bool active = tile < 3 && 16 * tj < nb;  // wave-uniform
     d4 accR = {0.0, 0.0, 0.0, 0.0}, accI = {0.0, 0.0, 0.0, 0.0};
     if (active) {
       const int64_t rbeg = 16 * ti;  // V(r, c) = 0 above the diagonal: rows below 16 ti give nothing
       const int64_t ns = L > rbeg ? (L - rbeg + 3) / 4 : 0;
-      const int64_t q4 = (ns + 3) / 4;
+      const int64_t q4 = (ns + PARTS - 1) / PARTS;
       const int64_t sb = part * q4, se = ns < sb + q4 ? ns : sb + q4;
       const int ca = 16 * ti + (lane & 15), cb = 16 * tj + (lane & 15);
       const int64_t cac = ca < nb ? ca : nb - 1, cbc = cb < nb ? cb : nb - 1;
-      const T one = N::make(1.0, 0.0), zero = N::make(0.0, 0.0);
-      for (int64_t st = sb; st < se; ++st) {
-        const int64_t r = rbeg + 4 * st + (lane >> 4);
-        const int64_t rc = r < L ? r : L - 1;
-        const T va = P[rc + cac * ld], vb = P[rc + cbc * ld];
-        // V(r, c): 0 above the diagonal, 1 on it, the stored vector below
-        const T a = ((ca < nb) & (r < L) & (r >= ca)) ? (r == ca ? one : va) : zero;
-        const T bb = ((cb < nb) & (r < L) & (r >= cb)) ? (r == cb ? one : vb) : zero;
+      const T zero = N::make(0.0, 0.0);
+      constexpr int UN = 4;
+      for (int64_t st = sb; st < se; st += UN) {
+        T va[UN], vb[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {  // all loads first; steps past the part's last one read and add zeros
+          const int64_t r = rbeg + 4 * (st + u) + (lane >> 4), rc = r < L ? r : L - 1;
+          va[u] = V[rc + cac * p];
+          vb[u] = V[rc + cbc * p];
+        }
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+          const bool in = (st + u < se) & (rbeg + 4 * (st + u) + (lane >> 4) < L);
+          const T a = pick(in & (ca < nb), va[u], zero), bb = pick(in & (cb < nb), vb[u], zero);
         accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(a), N::re(bb), accR, 0, 0, 0);
         if constexpr (CPLX) {  // conj(a) b
           accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::im(a), N::im(bb), accR, 0, 0, 0);
           accI = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(a), N::im(bb), accI, 0, 0, 0);
           accI = __builtin_amdgcn_mfma_f64_16x16x4f64(-N::im(a), N::re(bb), accI, 0, 0, 0);
         }
+        }
       }
     }
     // item v of lane l is Z(16 ti + l / 16 + 4 v, 16 tj + l % 16)
     const int zr0 = 16 * ti + (lane >> 4), zc = 16 * tj + (lane & 15);
-    for (int pp = 0; pp < 4; ++pp) {
+    for (int pp = 0; pp < PARTS; ++pp) {
       if (active && part == pp) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -2146,47 +2309,62 @@ __global__ void __launch_bounds__(kThreads)
       __syncthreads();
     }
   }
-  T* Tm = work + d.tm_off + (int64_t)step * NB * NB;
-  {
-    const int h = lane >> 5, l = lane & 31, jc = wave + 16 * h;
-    const bool col_ok = jc < nb;
+  // diagonal 16 x 16 blocks: column 4 wave + lane / 16 per 16 lanes, lane l of it holding row l of the block
+  T* const Tm = work + d.tm_off + (int64_t)step * NB * NB;
+  if (wave < 8) {
+    const int jc = 4 * wave + (lane >> 4), cc = jc & 15, b0 = jc - cc, l = lane & 15;
     double xr = 0.0, xi = 0.0;
-    if (col_ok && l == jc) {
+    if (jc < nb && l == cc) {
       xr = s_tr[jc];
       xi = s_ti[jc];
     }
-    for (int i = wave + 15; i >= 0; --i) {  // wave-uniform trip count; half 0 needs only i < wave
-      const double zr = s_Zr[i][l], zi = CPLX ? s_Zi[i][l] : 0.0;
-      // Z(i, l) T(l, jc) over i < l <= jc (T(l, jc) is zero for l > jc; Z below the diagonal is unset)
-      const bool use = (l > i) & (l <= jc) & col_ok;
-      double cr = use ? zr * xr - zi * xi : 0.0;
-      double cim = use ? zr * xi + zi * xr : 0.0;
-      cr += dpp_move<0xB1>(cr);
-      cr += dpp_move<0x4E>(cr);
-      cr += dpp_move<0x141>(cr);
-      cr += dpp_move<0x140>(cr);
-      const double sr = h ? read_lane(cr, 32) + read_lane(cr, 48) : read_lane(cr, 0) + read_lane(cr, 16);
-      double si = 0.0;
+    for (int i = 14; i >= 0; --i) {
+      // Z(i, l) T(l, jc) over i < l <= cc (T(l, jc) is zero for l > cc; Z below the diagonal is unset)
+      const double zr = s_Zr[b0 + i][b0 + l], zi = CPLX ? s_Zi[b0 + i][b0 + l] : 0.0;
+      const bool use = (l > i) & (l <= cc);
+      double sr, si = 0.0;
       if constexpr (CPLX) {
-        cim += dpp_move<0xB1>(cim);
-        cim += dpp_move<0x4E>(cim);
-        cim += dpp_move<0x141>(cim);
-        cim += dpp_move<0x140>(cim);
-        si = h ? read_lane(cim, 32) + read_lane(cim, 48) : read_lane(cim, 0) + read_lane(cim, 16);
+        sr = group_sum<16>(use ? zr * xr - zi * xi : 0.0);
+        si = group_sum<16>(use ? zr * xi + zi * xr : 0.0);
+      } else {
+        sr = group_sum<16>(use ? zr * xr : 0.0);
       }
-      if ((l == i) & (i < jc) & col_ok) {
-        const double tr_ = s_tr[i], ti_ = s_ti[i];
-        xr = -(tr_ * sr - ti_ * si);
-        xi = -(tr_ * si + ti_ * sr);
+      if ((l == i) & (i < cc) & (jc < nb)) {
+        const double tr_ = s_tr[b0 + i], ti_ = CPLX ? s_ti[b0 + i] : 0.0;
+        xr = -(CPLX ? tr_ * sr - ti_ * si : tr_ * sr);
+        xi = CPLX ? -(tr_ * si + ti_ * sr) : 0.0;
       }
     }
-    Tm[l + jc * NB] = (col_ok && l <= jc) ? N::make(-xr, -xi) : N::make(0.0, 0.0);
+    s_T[b0 + l][jc] = N::make(xr, xi);
+    s_T[16 - b0 + l][jc] = N::make(0.0, 0.0);
   }
-  for (int64_t e = tid; e < L * nb; e += kThreads) {
-    const int64_t c = (int64_t)((uint32_t)e / (uint32_t)L), r = e - c * L;  // L nb < 2^32 (q <= YH_SVD_MAX_Q)
-    const T v = P[r + c * ld];  // in place: the same element as the W0 store below
-    W0[(k0 + r) + (k0 + c) * p] = r <= c ? v : N::make(0.0, 0.0);
-    Vall[(k0 + r) + (k0 + c) * p] = r < c ? N::make(0.0, 0.0) : (r == c ? N::make(1.0, 0.0) : v);
+  __syncthreads();
+  if (nb > 16 && wave == 0) {  // T(0:16, 16:32) = -T11 (Z12 T22)
+    auto product = [&](auto a, auto b2) {
+      d4 rr = {0.0, 0.0, 0.0, 0.0}, ri = rr;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const T x = a(lane & 15, 4 * i + (lane >> 4)), y = b2(4 * i + (lane >> 4), lane & 15);
+        rr = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(x), N::re(y), rr, 0, 0, 0);
+        if constexpr (CPLX) {
+          rr = __builtin_amdgcn_mfma_f64_16x16x4f64(-N::im(x), N::im(y), rr, 0, 0, 0);
+          ri = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(x), N::im(y), ri, 0, 0, 0);
+          ri = __builtin_amdgcn_mfma_f64_16x16x4f64(N::im(x), N::re(y), ri, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s_T[(lane >> 4) + 4 * v][16 + (lane & 15)] = N::make(-rr[v], -ri[v]);
+    };
+    product([&](int i, int k) { return N::make(s_Zr[i][16 + k], CPLX ? s_Zi[i][16 + k] : 0.0); },
+            [&](int k, int j) { return s_T[16 + k][16 + j]; });
+    __builtin_amdgcn_wave_barrier();
+    product([&](int i, int k) { return N::make(-N::re(s_T[i][k]), -N::im(s_T[i][k])); },
+            [&](int k, int j) { return s_T[k][16 + j]; });
+  }
+  __syncthreads();
+  for (int e = tid; e < NB * NB; e += NT) {
+    const T t = s_T[e % NB][e / NB];
+    Tm[e] = N::make(-N::re(t), -N::im(t));
   }
 }
 
@@ -3215,9 +3393,8 @@ extern "C" int yastn_hip_svd_panel_finalize(void* U, void* S, void* Vh, const vo
 }
 
 extern "C" int yastn_hip_check_qr_plan(const int64_t* h_qdesc, const int64_t* h_blocks, const int32_t* h_ids,
-                                       int64_t n, int dtype, int64_t work_numel, int64_t lds_bytes) {
+                                       int64_t n, int dtype, int64_t work_numel) {
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
-  const int64_t isz = yh::itemsize_of(dtype);
   for (int64_t t = 0; t < n; ++t) {
     const int32_t b = h_ids[t];
     const int64_t* w = h_qdesc + (int64_t)b * YH_QR_WORDS;
@@ -3229,8 +3406,6 @@ extern "C" int yastn_hip_check_qr_plan(const int64_t* h_qdesc, const int64_t* h_
                  (long long)q);
     YH_CHECK_ARG((sm >= sn ? sm : sn) == p && (sm < sn ? sm : sn) == q, "qr block %d: shape mismatch", b);
     YH_CHECK_ARG(p <= kQrMaxRows, "qr block %d: %lld rows (at most %lld)", b, (long long)p, (long long)kQrMaxRows);
-    YH_CHECK_ARG(lds_bytes == 0 || p * YH_QR_NB * isz <= lds_bytes, "qr block %d: panel of %lld rows exceeds LDS",
-                 b, (long long)p);
     const bool ok = w[2] >= 0 && w[2] + p * q <= work_numel && w[3] >= 0 && w[3] + p * q <= work_numel &&
                     w[4] >= 0 && w[4] + np * YH_QR_NB * YH_QR_NB <= work_numel && w[5] >= 0 &&
                     w[5] + 2 * q * q <= work_numel && w[6] >= 0 && w[6] + 2 * YH_QR_NB * q <= work_numel;
@@ -3240,31 +3415,26 @@ extern "C" int yastn_hip_check_qr_plan(const int64_t* h_qdesc, const int64_t* h_
 }
 
 extern "C" int yastn_hip_svd_qr_panel(void* work, int dtype, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n,
-                                      int step, int64_t lds_bytes, hipStream_t stream) {
+                                      int step, int64_t max_rows, hipStream_t stream) {
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
-  YH_CHECK_ARG(step >= 0 && lds_bytes >= 0 && lds_bytes <= 160 * 1024, "qr panel step %d / lds %lld", step,
-               (long long)lds_bytes);
+  YH_CHECK_ARG(step >= 0 && max_rows >= 0, "qr panel step %d of %lld rows", step, (long long)max_rows);
   if (n == 0) return YH_OK;
-  const dim3 g((unsigned)n), t(kThreads);
-  if (lds_bytes == 0) {  // panels factored in place in the workspace
-    if (dtype == YH_F64)
-      hipLaunchKernelGGL((qr_panel_kernel<false, true>), g, t, 0, stream, d_qdesc, d_ids, (double*)work, step);
+  const dim3 g((unsigned)n);
+  const int64_t rows = max_rows - (int64_t)step * YH_QR_NB;
+  if (dtype == YH_F64) {
+    if (rows <= kQrRegRows<false>)
+      hipLaunchKernelGGL((qr_panel_kernel<false, false>), g, dim3(kQrThreads), 0, stream, d_qdesc, d_ids, (double*)work,
+                         step);
     else
-      hipLaunchKernelGGL((qr_panel_kernel<true, true>), g, t, 0, stream, d_qdesc, d_ids, (double2*)work, step);
-  } else if (dtype == YH_F64) {
-    const int st = yh::hip_status(hipFuncSetAttribute((const void*)qr_panel_kernel<false, false>,
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes),
-                                  "svd qr panel LDS size");
-    if (st) return st;
-    hipLaunchKernelGGL((qr_panel_kernel<false, false>), g, t, (size_t)lds_bytes, stream, d_qdesc, d_ids,
-                       (double*)work, step);
+      hipLaunchKernelGGL((qr_panel_kernel<false, true>), g, dim3(kThreads), 0, stream, d_qdesc, d_ids, (double*)work,
+                         step);
   } else {
-    const int st = yh::hip_status(hipFuncSetAttribute((const void*)qr_panel_kernel<true, false>,
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes),
-                                  "svd qr panel LDS size");
-    if (st) return st;
-    hipLaunchKernelGGL((qr_panel_kernel<true, false>), g, t, (size_t)lds_bytes, stream, d_qdesc, d_ids,
-                       (double2*)work, step);
+    if (rows <= kQrRegRows<true>)
+      hipLaunchKernelGGL((qr_panel_kernel<true, false>), g, dim3(kQrThreads), 0, stream, d_qdesc, d_ids, (double2*)work,
+                         step);
+    else
+      hipLaunchKernelGGL((qr_panel_kernel<true, true>), g, dim3(kThreads), 0, stream, d_qdesc, d_ids, (double2*)work,
+                         step);
   }
   return yh::hip_status(hipGetLastError(), "svd qr panel launch");
 }
@@ -3391,17 +3561,14 @@ extern "C" int yastn_hip_svd_precond_finalize(void* U, void* S, void* Vh, void* 
 
 extern "C" int yastn_hip_check_qr_op_plan(const int64_t* h_qdesc, const int64_t* h_qblocks, int64_t nblocks,
                                           int dtype, int64_t a_numel, int64_t q_numel, int64_t r_numel,
-                                          int64_t work_numel, int64_t lds_bytes) {
+                                          int64_t work_numel) {
   YH_CHECK_ARG(dtype == YH_F64 || dtype == YH_C128, "dtype %d", dtype);
-  const int64_t isz = yh::itemsize_of(dtype);
   for (int64_t b = 0; b < nblocks; ++b) {
     const int64_t* w = h_qdesc + b * YH_QR_WORDS;
     const int64_t* bw = h_qblocks + b * YH_QROP_WORDS;
     const int64_t m = w[0], n = w[1], k = w[7];
     YH_CHECK_ARG(m >= 1 && n >= 1 && k == (m < n ? m : n), "qr block %lld: %lld x %lld, k %lld", (long long)b,
                  (long long)m, (long long)n, (long long)k);
-    YH_CHECK_ARG(lds_bytes == 0 || m * YH_QR_NB * isz <= lds_bytes, "qr block %lld: panel of %lld rows exceeds LDS",
-                 (long long)b, (long long)m);
     YH_CHECK_ARG(m <= kQrMaxRows, "qr block %lld: %lld rows (at most %lld)", (long long)b, (long long)m,
                  (long long)kQrMaxRows);
     const int64_t np = (k + YH_QR_NB - 1) / YH_QR_NB;

@@ -761,9 +761,8 @@ class SvdPlan:
     an LDS-resident kernel, one workgroup per block, all in one launch.  Larger blocks use the panel
     path: W and V in a workspace, panels of width b, one launch per round of panel pairs.  For SVD
     blocks the panel path first factors W0 = Q R (blocked Householder QR: a panel kernel and a launch of block
-    reflectors per step; the p x YH_QR_NB panel is staged in LDS when every block's fits, else
-    factored in place in the workspace) and iterates on X = R^H; the p-side vectors are multiplied
-    by Q at the end (one launch).
+    reflectors per step; the panels are factored in registers, or in place in the workspace if one of them is too
+    tall) and iterates on X = R^H; the p-side vectors are multiplied by Q at the end (one launch).
     """
 
     def __init__(self, blocks, itemsize, mode, a_numel, u_numel, s_numel, v_numel, device):
@@ -895,15 +894,10 @@ class SvdPlan:
         """Panel lists of the Householder QR."""
         NB = L.YH_QR_NB
         self.h_qdesc = np.ascontiguousarray(qd)
-        pmax = max(int(qd[b, 0]) for b in pre)
-        # panel staged in LDS, or 0: factored in place in the workspace (the panel kernel's static LDS,
-        # the T matrices, takes ~17.5 KiB at 32 columns)
-        self.qr_lds = pmax * NB * itemsize
-        if self.qr_lds > L.device_lds_per_block() - 20 * 1024:
-            self.qr_lds = 0
+        self.qr_rows = max(int(qd[b, 0]) for b in pre)
         ids = np.array(pre, dtype=np.int32)
         L.call('yastn_hip_check_qr_plan', self.h_qdesc.ctypes.data, self.h_blocks.ctypes.data, ids.ctypes.data,
-               len(ids), self.dt, max(work, 0), self.qr_lds)
+               len(ids), self.dt, max(work, 0))
         self.d_qdesc = torch.from_numpy(self.h_qdesc).to(device)
         self.d_pre = torch.from_numpy(ids).to(device)
         self.qr_cols = max(int(qd[b, 1]) for b in pre)
@@ -970,9 +964,7 @@ class QrPlan:
     """Batched Householder QR of the blocks of backend.qr (meta rows (sl, (m, n), slQ, (m, k), slR,
     (k, n))): per block the workspace holds W0 (m x n), the reflectors (m x k), -T per panel, E (m x k)
     and scratch; the panel steps follow the preconditioning of the SVD (the columns of W0 right of each
-    panel after it, then E <- H_s E for the panels in reverse).  The
-    32-column Householder panels are staged in LDS when every block's fits (``lds`` > 0), else
-    factored in place in the workspace (``lds`` = 0)."""
+    panel after it, then E <- H_s E for the panels in reverse)."""
 
     def __init__(self, meta, itemsize, a_numel, sizes, device):
         NB = L.YH_QR_NB
@@ -994,14 +986,11 @@ class QrPlan:
         self.work_numel = max(work, 1)
         self.h_qdesc = np.ascontiguousarray(np.array(qd, dtype=np.int64).reshape(-1, L.YH_QR_WORDS))
         self.h_qblocks = np.ascontiguousarray(np.array(qb, dtype=np.int64).reshape(-1, L.YH_QROP_WORDS))
-        pmax = max((r[0] for r in qd), default=1)
+        self.qr_rows = max((r[0] for r in qd), default=1)
         self.max_k = max((r[7] for r in qd), default=0)
-        self.qr_lds = pmax * NB * itemsize
-        if self.qr_lds > L.device_lds_per_block() - 20 * 1024:  # static LDS of the panel kernel: ~17.5 KiB
-            self.qr_lds = 0
         self.native = True
         L.call('yastn_hip_check_qr_op_plan', self.h_qdesc.ctypes.data, self.h_qblocks.ctypes.data, self.nblocks,
-               self.dt, a_numel, sizes[0], sizes[1], self.work_numel, self.qr_lds)
+               self.dt, a_numel, sizes[0], sizes[1], self.work_numel)
         self.d_qdesc = torch.from_numpy(self.h_qdesc).to(device)
         self.d_qblocks = torch.from_numpy(self.h_qblocks).to(device)
         self.panel_steps = _panel_steps([(b, r[1], r[7]) for b, r in enumerate(qd)], device)
