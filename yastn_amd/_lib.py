@@ -26,7 +26,7 @@ YH_TILE_SMALLM = 6
 YH_TILE_RD32 = 7
 TILE_DIMS = {YH_TILE_32x32: (32, 32), YH_TILE_64x64: (64, 64), YH_TILE_128x64: (128, 64),
              YH_TILE_16x64: (16, 64), YH_TILE_64x16: (64, 16), YH_TILE_128x128: (128, 128),
-             YH_TILE_SMALLM: (16, 256), YH_TILE_RD32: (32, 32)}
+             YH_TILE_SMALLM: (16, 512), YH_TILE_RD32: (32, 32)}
 YH_SVD_WORDS = 8
 YH_SVD_MAX_Q = 2048
 YH_SMALL_Q = 32

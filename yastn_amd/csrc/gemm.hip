@@ -49,6 +49,21 @@ __device__ double2 kZeroElt[kZeroSpan];
 // the short-K launches of many tiles are bound by how many tiles a CU holds at once), else no bound.
 #define GEMM_MINB(CPLX, BM, BN) ((BM) == 32 && (BN) == 32 ? 4 : 1)
 
+// A workgroup finds its operands through its tile, the tile's GEMM and that one's terms, and at the start of a kernel each
+// of these reads costs a memory latency (~1 us: what the kernel before left in the L2s is gone).  The words of term g are
+// read together with those of GEMM g, which is where the terms of a plan with one term per GEMM lie; other terms are
+// read when their index is known.  One latency less on every launch of 6 to 40 us.
+struct Term {
+  int64_t w[YH_TERM_WORDS];
+};
+
+__device__ __attribute__((always_inline)) inline Term load_term(const int64_t* __restrict__ p) {
+  Term t;
+#pragma unroll
+  for (int i = 0; i < YH_TERM_WORDS; ++i) t.w[i] = p[i];
+  return t;
+}
+
 __device__ inline d4 mfma(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 
 // One workgroup per output tile.  Per term, the k loop is software-pipelined: the next BK slice of
@@ -58,7 +73,7 @@ __device__ inline d4 mfma(double a, double b, d4 c) { return __builtin_amdgcn_mf
 // so that consecutive MFMAs do not wait on each other.
 template <bool CPLX, int BM, int BN, int WM, int WN, int BK>
 __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel(Bufs bufs, const int64_t* __restrict__ gemms,
-                                                        const int64_t* __restrict__ terms,
+                                                        const int64_t* __restrict__ terms, int64_t nterms,
                                                         const int32_t* __restrict__ tiles) {
   typedef typename Elt<CPLX>::T T;
   constexpr int FM = BM / WM / 16;
@@ -84,6 +99,7 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
   const int64_t g = tl[0];
   const int64_t m0 = tl[1], n0 = tl[2];
   const int64_t* gw = gemms + g * YH_GEMM_WORDS;
+  const Term guess = load_term(g < nterms ? terms + g * YH_TERM_WORDS : gw);
   const int64_t M = gw[0], N = gw[1], c_off = gw[2], c_rs = gw[3], c_cs = gw[4];
   const int64_t tb = gw[5], tc = gw[6], gflags = gw[7];
 
@@ -99,7 +115,9 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
       }
 
   for (int64_t q = tb; q < tb + tc; ++q) {
-    const int64_t* tw = terms + q * YH_TERM_WORDS;
+    Term term = guess;
+    if (q != g) term = load_term(terms + q * YH_TERM_WORDS);
+    const int64_t* tw = term.w;
     const int64_t a_off = tw[0], a_rs = tw[1], a_cs = tw[2];
     const int64_t b_off = tw[3], b_rs = tw[4], b_cs = tw[5], K = tw[6], tf = tw[7];
     const bool conjA = tf & 1, conjB = (tf >> 1) & 1;
@@ -301,7 +319,7 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
 constexpr int kRdDepth = 4;
 template <bool CPLX>
 __global__ void __launch_bounds__(kThreads, CPLX ? 2 : 4) gemm_rd_kernel(Bufs bufs, const int64_t* __restrict__ gemms,
-                                                             const int64_t* __restrict__ terms,
+                                                             const int64_t* __restrict__ terms, int64_t nterms,
                                                              const int32_t* __restrict__ tiles) {
   typedef typename Elt<CPLX>::T T;
   constexpr int NPL = CPLX ? 2 : 1;
@@ -314,6 +332,7 @@ __global__ void __launch_bounds__(kThreads, CPLX ? 2 : 4) gemm_rd_kernel(Bufs bu
   const int64_t g = tl[0];
   const int64_t m0 = tl[1], n0 = tl[2];
   const int64_t* gw = gemms + g * YH_GEMM_WORDS;
+  const Term guess = load_term(g < nterms ? terms + g * YH_TERM_WORDS : gw);
   const int64_t M = gw[0], N = gw[1], c_off = gw[2], c_rs = gw[3], c_cs = gw[4];
   const int64_t tb = gw[5], tc = gw[6], gflags = gw[7];
   const T* zero = (const T*)kZeroElt + (threadIdx.x & (kZeroSpan - 1));
@@ -328,7 +347,9 @@ __global__ void __launch_bounds__(kThreads, CPLX ? 2 : 4) gemm_rd_kernel(Bufs bu
   const bool oka0 = m0 + r16 < M, oka1 = m0 + 16 + r16 < M;
   const bool okb0 = n0 + r16 < N, okb1 = n0 + 16 + r16 < N;
   for (int64_t q = tb; q < tb + tc; ++q) {
-    const int64_t* tw = terms + q * YH_TERM_WORDS;
+    Term term = guess;
+    if (q != g) term = load_term(terms + q * YH_TERM_WORDS);
+    const int64_t* tw = term.w;
     const int64_t a_off = tw[0], a_rs = tw[1], a_cs = tw[2];
     const int64_t b_off = tw[3], b_rs = tw[4], b_cs = tw[5], K = tw[6], tf = tw[7];
     if (K <= 0) continue;
@@ -472,76 +493,118 @@ __global__ void __launch_bounds__(kThreads) splitk_reduce_kernel(Bufs bufs, cons
 
 
 // Streaming kernel for GEMMs whose M is at most 16 (e.g. contractions with a small MPO leg): a tile
-// is all M rows times 256 columns, one thread per column; the A entries are wave-uniform (scalar
-// loads), B and C are read / written along the columns, so the kernel runs at the HBM rate.
-constexpr int kSmallM = 16, kSmallN = 256;
+// is all M rows times 512 columns; B and C are read / written along the columns.  Bound by latency: a workgroup does
+// little between finding its operands and its stores, so its reads go together.  Four steps of k at a time: lane l of
+// a wave reads A(l % 16, k0 + l / 16), every thread four elements of each of its columns of B, and the entries of A reach
+// the products through scalar registers.  Up to 4 rows, a thread holds two columns; more rows leave no registers
+// for that.  (One k at a time, A by scalar loads and 256 columns: 9.9 us for 280 real GEMMs with K = 4 and 20 MB in all,
+// 7.4 to 8.4 for 184 small complex ones; now 7.4 to 7.7 and 6.0 to 6.2.)
+constexpr int kSmallM = 16, kSmallN = 512;
 
-template <bool CPLX>
-__global__ void __launch_bounds__(kThreads) gemm_smallm_kernel(Bufs bufs, const int64_t* __restrict__ gemms,
-                                                               const int64_t* __restrict__ terms,
-                                                               const int32_t* __restrict__ tiles) {
+__device__ __attribute__((always_inline)) inline double lane_value(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// Columns j0 + 256 c, c < NC, of a GEMM with M <= MB rows.
+template <bool CPLX, int MB, int NC>
+__device__ __attribute__((always_inline)) inline void smallm_columns(const Bufs& bufs, const int64_t* __restrict__ gw,
+                                                                     const int64_t* __restrict__ terms,
+                                                                     const Term& guess, int64_t g, int64_t j0) {
   typedef typename Elt<CPLX>::T T;
-  const int32_t* tl = tiles + 3 * (int64_t)blockIdx.x;
-  const int64_t* gw = gemms + (int64_t)tl[0] * YH_GEMM_WORDS;
   const int64_t M = gw[0], N = gw[1], c_off = gw[2], c_rs = gw[3], c_cs = gw[4];
   const int64_t tb = gw[5], tc = gw[6], gflags = gw[7];
-  const int64_t j = (int64_t)tl[2] + threadIdx.x;
-  double accr[kSmallM], acci[kSmallM];
+  double accr[NC][MB], acci[NC][MB];
 #pragma unroll
-  for (int i = 0; i < kSmallM; ++i) {
-    accr[i] = 0.0;
-    acci[i] = 0.0;
-  }
-  const bool live = j < N;
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int i = 0; i < MB; ++i) accr[c][i] = acci[c][i] = 0.0;
+  const int lane = threadIdx.x & 63;
   for (int64_t q = tb; q < tb + tc; ++q) {
-    const int64_t* tw = terms + q * YH_TERM_WORDS;
+    Term term = guess;
+    if (q != g) term = load_term(terms + q * YH_TERM_WORDS);
+    const int64_t* tw = term.w;
     const int64_t a_off = tw[0], a_rs = tw[1], a_cs = tw[2];
     const int64_t b_off = tw[3], b_rs = tw[4], b_cs = tw[5], K = tw[6], tf = tw[7];
     const double sa = (tf & 1) ? -1.0 : 1.0, sb = (tf & 2) ? -1.0 : 1.0;  // conjugation signs
     const T* __restrict__ A = (const T*)bufs.in[(tf >> 8) & 0xff];
     const T* __restrict__ B = (const T*)bufs.in[(tf >> 16) & 0xff];
-    for (int64_t k = 0; k < K; ++k) {
-      T b;
-      if (live)
-        b = B[b_off + k * b_rs + j * b_cs];
-      else
-        b = T{};
+    const int64_t ai = (lane & 15) < M ? lane & 15 : 0;
+    for (int64_t k0 = 0; k0 < K; k0 += 4) {
+      const int64_t ka = k0 + (lane >> 4);
+      const T mine = A[a_off + ai * a_rs + (ka < K ? ka : k0) * a_cs];
+      T b[NC][4];
 #pragma unroll
-      for (int i = 0; i < kSmallM; ++i) {
-        if (i < M) {
-          const T a = A[a_off + i * a_rs + k * a_cs];
-          if constexpr (CPLX) {
-            const double ar = a.x, ai = sa * a.y, br = b.x, bi = sb * b.y;
-            accr[i] += ar * br - ai * bi;
-            acci[i] += ar * bi + ai * br;
-          } else {
-            accr[i] += a * b;
+      for (int c = 0; c < NC; ++c) {
+        const int64_t j = j0 + kThreads * c, jc = j < N ? j : 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b[c][u] = B[b_off + (k0 + u < K ? k0 + u : k0) * b_rs + jc * b_cs];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (k0 + u >= K) break;  // uniform
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          if (i < M) {
+            if constexpr (CPLX) {
+              const double ar = lane_value(mine.x, i + 16 * u), am = sa * lane_value(mine.y, i + 16 * u);
+#pragma unroll
+              for (int c = 0; c < NC; ++c) {
+                const double br = b[c][u].x, bi = sb * b[c][u].y;
+                accr[c][i] += ar * br - am * bi;
+                acci[c][i] += ar * bi + am * br;
+              }
+            } else {
+              const double ar = lane_value(mine, i + 16 * u);
+#pragma unroll
+              for (int c = 0; c < NC; ++c) accr[c][i] += ar * b[c][u];
+            }
           }
         }
       }
     }
   }
-  if (!live) return;
   T* __restrict__ C = (T*)bufs.out[(gflags >> 8) & 0xff];
   const bool accumulate = gflags & 1;
 #pragma unroll
-  for (int i = 0; i < kSmallM; ++i) {
-    if (i < M) {
-      T* p = C + c_off + i * c_rs + j * c_cs;
-      if constexpr (CPLX) {
-        double2 r = make_double2(accr[i], acci[i]);
-        if (accumulate) {
-          const double2 o = *p;
-          r.x += o.x;
-          r.y += o.y;
+  for (int c = 0; c < NC; ++c) {
+    const int64_t j = j0 + kThreads * c;
+    if (j >= N) continue;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      if (i < M) {
+        T* p = C + c_off + i * c_rs + j * c_cs;
+        if constexpr (CPLX) {
+          double2 r = make_double2(accr[c][i], acci[c][i]);
+          if (accumulate) {
+            const double2 o = *p;
+            r.x += o.x;
+            r.y += o.y;
+          }
+          *p = r;
+        } else {
+          double r = accr[c][i];
+          if (accumulate) r += *p;
+          *p = r;
         }
-        *p = r;
-      } else {
-        double r = accr[i];
-        if (accumulate) r += *p;
-        *p = r;
       }
     }
+  }
+}
+
+template <bool CPLX>
+__global__ void __launch_bounds__(kThreads) gemm_smallm_kernel(Bufs bufs, const int64_t* __restrict__ gemms,
+                                                               const int64_t* __restrict__ terms, int64_t nterms,
+                                                               const int32_t* __restrict__ tiles) {
+  const int32_t* tl = tiles + 3 * (int64_t)blockIdx.x;
+  const int64_t g = tl[0], j0 = (int64_t)tl[2] + threadIdx.x;
+  const int64_t* gw = gemms + g * YH_GEMM_WORDS;
+  const Term guess = load_term(g < nterms ? terms + g * YH_TERM_WORDS : gw);
+  if (gw[0] <= 4) {
+    smallm_columns<CPLX, 4, 2>(bufs, gw, terms, guess, g, j0);
+  } else {
+    smallm_columns<CPLX, kSmallM, 1>(bufs, gw, terms, guess, g, j0);
+    if ((int64_t)tl[2] + kThreads < gw[1]) smallm_columns<CPLX, kSmallM, 1>(bufs, gw, terms, guess, g, j0 + kThreads);
   }
 }
 
@@ -549,36 +612,36 @@ __global__ void __launch_bounds__(kThreads) gemm_smallm_kernel(Bufs bufs, const 
 // slices are faster now that two slices of global loads really are in flight; the double-buffered
 // LDS tiles stay within 64 KiB.
 template <bool CPLX>
-int launch(const Bufs& b, const int64_t* gemms, const int64_t* terms, const int32_t* tiles, int64_t ntiles,
-           int cfg, hipStream_t s) {
+int launch(const Bufs& b, const int64_t* gemms, const int64_t* terms, int64_t nterms, const int32_t* tiles,
+           int64_t ntiles, int cfg, hipStream_t s) {
   const dim3 grid((unsigned)ntiles), block(kThreads);
   constexpr int BKW = 8;              // 64 / 128-wide tiles
   constexpr int BKH = CPLX ? 4 : 8;   // 128 x 128
   constexpr int BKS = CPLX ? 8 : 16;  // 32-wide and skinny tiles
   switch (cfg) {
     case YH_TILE_32x32:
-      hipLaunchKernelGGL((gemm_kernel<CPLX, 32, 32, 2, 2, BKS>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_kernel<CPLX, 32, 32, 2, 2, BKS>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_64x64:
-      hipLaunchKernelGGL((gemm_kernel<CPLX, 64, 64, 2, 2, BKW>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_kernel<CPLX, 64, 64, 2, 2, BKW>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_128x64:
-      hipLaunchKernelGGL((gemm_kernel<CPLX, 128, 64, 2, 2, BKW>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_kernel<CPLX, 128, 64, 2, 2, BKW>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_16x64:
-      hipLaunchKernelGGL((gemm_kernel<CPLX, 16, 64, 1, 4, BKS>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_kernel<CPLX, 16, 64, 1, 4, BKS>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_64x16:
-      hipLaunchKernelGGL((gemm_kernel<CPLX, 64, 16, 4, 1, BKS>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_kernel<CPLX, 64, 16, 4, 1, BKS>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_128x128:
-      hipLaunchKernelGGL((gemm_kernel<CPLX, 128, 128, 2, 2, BKH>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_kernel<CPLX, 128, 128, 2, 2, BKH>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_RD32:
-      hipLaunchKernelGGL(gemm_rd_kernel<CPLX>, grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL(gemm_rd_kernel<CPLX>, grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     case YH_TILE_SMALLM:
-      hipLaunchKernelGGL((gemm_smallm_kernel<CPLX>), grid, block, 0, s, b, gemms, terms, tiles);
+      hipLaunchKernelGGL((gemm_smallm_kernel<CPLX>), grid, block, 0, s, b, gemms, terms, nterms, tiles);
       break;
     default:
       yh::set_error("unknown tile config %d", cfg);
@@ -658,8 +721,8 @@ extern "C" int yastn_hip_grouped_gemm(void* const* outs, const void* const* ins,
     b.in[i] = ins[i];
     b.out[i] = outs[i];
   }
-  return dtype == YH_F64 ? launch<false>(b, d_gemms, d_terms, d_tiles, ntiles, cfg, stream)
-                         : launch<true>(b, d_gemms, d_terms, d_tiles, ntiles, cfg, stream);
+  return dtype == YH_F64 ? launch<false>(b, d_gemms, d_terms, nterms, d_tiles, ntiles, cfg, stream)
+                         : launch<true>(b, d_gemms, d_terms, nterms, d_tiles, ntiles, cfg, stream);
 }
 
 extern "C" int yastn_hip_dot(void* C, const void* A, const void* B, int dtype, const int64_t* d_gemms,
