@@ -11,6 +11,9 @@ from yastn_amd import plans as P
 pytestmark = pytest.mark.gpu
 
 COLUMNS = (1, 63, 255, 256, 257, 511, 512, 513, 769)
+DEPTHS = (1, 3, 4, 5, 8, 9, 16, 17, 39, 40, 41, 47, 48, 80, 81, 95, 96, 97)  # short and steady k loops, with remainders
+ROWS = ((1, 2, 3, 4), (1, 4, 5, 16), (17, 64, 65, 130))
+CASES = [(r, c) for r in ROWS for c in sorted(L.TILE_DIMS) if c != L.YH_TILE_SMALLM or max(r) <= L.TILE_DIMS[c][0]]
 
 
 def _strides(rng, rows, cols):
@@ -24,8 +27,7 @@ def _entries(rng, n, cplx):
 
 
 @pytest.mark.parametrize('cplx', [False, True])
-@pytest.mark.parametrize('cfg', sorted(L.TILE_DIMS))
-@pytest.mark.parametrize('rows', [(1, 2, 3, 4), (1, 4, 5, 16)])
+@pytest.mark.parametrize('rows, cfg', CASES)
 def test_terms_and_tile_edges(rows, cfg, cplx):
     rng = np.random.default_rng(100 * cfg + len(rows) + rows[-1] + cplx)
     gemms, terms, mats, na, nb, nc = [], [], [], 0, 0, 0
@@ -34,7 +36,7 @@ def test_terms_and_tile_edges(rows, cfg, cplx):
         rs, cs = _strides(rng, M, N)
         gemms.append((M, N, nc, rs, cs, len(terms), tc, i % 2))
         for _ in range(tc):
-            K = int(rng.integers(1, 21))
+            K = int(rng.choice(DEPTHS))
             (ars, acs), (brs, bcs) = _strides(rng, M, K), _strides(rng, K, N)
             flags = int(rng.integers(4)) if cplx else 0
             terms.append((na, ars, acs, nb, brs, bcs, K, flags | (1 << 16)))

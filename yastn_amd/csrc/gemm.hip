@@ -71,6 +71,11 @@ __device__ inline d4 mfma(double a, double b, d4 c) { return __builtin_amdgcn_mf
 // LDS buffers, then stored into the other buffer; one barrier per slice.  Tiles with a single 16x16
 // fragment per wave keep NS partial accumulators (k sub-steps rotate over them, summed at the end)
 // so that consecutive MFMAs do not wait on each other.
+// What bounds large GEMMs is the issue of other vector instructions between the FP64 MFMAs, so a load in the loop over
+// full slices costs one 64-bit add: rows and columns are clamped once per term, and only the last slices test k.  (With
+// the tests and a 64-bit multiply in every slice, 4096 x 4096 x 1024 in 64 x 64 tiles: real 713 us, complex 2130;
+// now 625 and 2010, 55 and 68 TFLOP/s.  21 complex blocks up to 1134 cubed: 870 us, now 821.)  Padding rows of the LDS
+// tiles by 1, 4, 8 or 16 elements instead of 2 measured 0 to 12 % slower; a raised wave priority made no difference.
 template <bool CPLX, int BM, int BN, int WM, int WN, int BK>
 __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel(Bufs bufs, const int64_t* __restrict__ gemms,
                                                         const int64_t* __restrict__ terms, int64_t nterms,
@@ -129,10 +134,9 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
 
     // per-thread slice coordinates (fixed for the term); the k coordinate advances by BK per slice
     int a_i[A_PER], a_k[A_PER], b_j[B_PER], b_k[B_PER];
-    bool a_in[A_PER], b_in[B_PER];
 #pragma unroll
     for (int p = 0; p < A_PER; ++p) {
-      const int e = tid + p * kThreads;
+      const int e = (tid + p * kThreads) % (BM * BK);
       if (a_kfast) {
         a_k[p] = e % BK;
         a_i[p] = e / BK;
@@ -140,11 +144,10 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
         a_i[p] = e % BM;
         a_k[p] = e / BM;
       }
-      a_in[p] = (A_FULL || e < BM * BK) && (m0 + a_i[p] < M);
     }
 #pragma unroll
     for (int p = 0; p < B_PER; ++p) {
-      const int e = tid + p * kThreads;
+      const int e = (tid + p * kThreads) % (BN * BK);
       if (b_nfast) {
         b_j[p] = e % BN;
         b_k[p] = e / BN;
@@ -152,28 +155,46 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
         b_k[p] = e % BK;
         b_j[p] = e / BK;
       }
-      b_in[p] = (B_FULL || e < BN * BK) && (n0 + b_j[p] < N);
     }
 
     // Two register sets: while slice s is consumed from LDS, slice s+1 waits in one set (loaded an
     // iteration earlier) and slice s+2 is being loaded into the other, so two slices of global loads
     // are in flight; slice s+1 goes to the other LDS buffer at the end of the iteration.
     T ra0[A_PER], rb0[B_PER], ra1[A_PER], rb1[B_PER];
-    // Every lane issues every load; an element outside the operand is read from kZeroElt.  (A select
-    // after the load would be hoisted by the scheduler and wait for loads still meant to be in flight.)
+    // Every lane issues every load.  Rows past M and columns past N read the last one, since they only reach
+    // entries of C that are not stored; k past K reads kZeroElt.  (A select after the load would be hoisted by the
+    // scheduler and wait for loads still meant to be in flight.)  a_next / b_next point into the next slice to load.
     const T* zero = (const T*)kZeroElt + (tid & (kZeroSpan - 1));
-    const T* a_row[A_PER];
-    const T* b_col[B_PER];
+    const T* a_next[A_PER];
+    const T* b_next[B_PER];
 #pragma unroll
-    for (int p = 0; p < A_PER; ++p) a_row[p] = A + a_off + (m0 + a_i[p]) * a_rs + a_k[p] * a_cs;
+    for (int p = 0; p < A_PER; ++p) a_next[p] = A + a_off + min(m0 + a_i[p], M - 1) * a_rs + a_k[p] * a_cs;
 #pragma unroll
-    for (int p = 0; p < B_PER; ++p) b_col[p] = B + b_off + b_k[p] * b_rs + (n0 + b_j[p]) * b_cs;
+    for (int p = 0; p < B_PER; ++p) b_next[p] = B + b_off + b_k[p] * b_rs + min(n0 + b_j[p], N - 1) * b_cs;
+    const int64_t a_step = BK * a_cs, b_step = BK * b_rs;
+    auto load_full = [&](T* ra, T* rb) {  // a slice with all of its k inside
+#pragma unroll
+      for (int p = 0; p < A_PER; ++p) {
+        ra[p] = *a_next[p];
+        a_next[p] += a_step;
+      }
+#pragma unroll
+      for (int p = 0; p < B_PER; ++p) {
+        rb[p] = *b_next[p];
+        b_next[p] += b_step;
+      }
+    };
     auto load = [&](int64_t k0, T* ra, T* rb) {
-      const int64_t da = k0 * a_cs, db = k0 * b_rs;
 #pragma unroll
-      for (int p = 0; p < A_PER; ++p) ra[p] = *((a_in[p] & (k0 + a_k[p] < K)) ? a_row[p] + da : zero);
+      for (int p = 0; p < A_PER; ++p) {
+        ra[p] = *(k0 + a_k[p] < K ? a_next[p] : zero);
+        a_next[p] += a_step;
+      }
 #pragma unroll
-      for (int p = 0; p < B_PER; ++p) rb[p] = *((b_in[p] & (k0 + b_k[p] < K)) ? b_col[p] + db : zero);
+      for (int p = 0; p < B_PER; ++p) {
+        rb[p] = *(k0 + b_k[p] < K ? b_next[p] : zero);
+        b_next[p] += b_step;
+      }
     };
     auto store = [&](int buf, const T* ra, const T* rb) {
 #pragma unroll
@@ -231,15 +252,28 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            accR[s][i][j] = mfma(ar[ks][i], br[ks][j], accR[s][i][j]);
-            if constexpr (CPLX) {
-              accR[s][i][j] = mfma(-ai[ks][i], bi[ks][j], accR[s][i][j]);
-              accI[s][i][j] = mfma(ar[ks][i], bi[ks][j], accI[s][i][j]);
-              accI[s][i][j] = mfma(ai[ks][i], br[ks][j], accI[s][i][j]);
-            }
-          }
+          for (int j = 0; j < FN; ++j) accR[s][i][j] = mfma(ar[ks][i], br[ks][j], accR[s][i][j]);
+        if constexpr (CPLX) {  // no product waits for the one right before it
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) accI[s][i][j] = mfma(ar[ks][i], bi[ks][j], accI[s][i][j]);
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) accR[s][i][j] = mfma(-ai[ks][i], bi[ks][j], accR[s][i][j]);
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) accI[s][i][j] = mfma(ai[ks][i], br[ks][j], accI[s][i][j]);
+        }
       }
+    };
+
+    // Complex tiles of several fragments: the reads above stay ahead of the products (the scheduler would sink them to
+    // their uses, to save registers).  Real and 32 x 32 tiles measured no faster with it.
+    auto issued = [&]() {
+      if constexpr (CPLX && FM * FN >= 4) __builtin_amdgcn_sched_barrier(0);
     };
 
     const int64_t ns = (K + BK - 1) / BK;  // slices
@@ -254,18 +288,34 @@ __global__ void __launch_bounds__(kThreads, GEMM_MINB(CPLX, BM, BN)) gemm_kernel
     __syncthreads();
     read_frag(0, far0, fai0, fbr0, fbi0);
     int64_t s = 0;
+    for (const int64_t full = K / BK; s + 4 < full; s += 2) {  // as below, with slices s+3 and s+4 full
+      store(1, ra0, rb0);
+      load_full(ra0, rb0);
+      __syncthreads();
+      read_frag(1, far1, fai1, fbr1, fbi1);
+      issued();
+      mma(far0, fai0, fbr0, fbi0);
+      store(0, ra1, rb1);
+      load_full(ra1, rb1);
+      __syncthreads();
+      read_frag(0, far0, fai0, fbr0, fbi0);
+      issued();
+      mma(far1, fai1, fbr1, fbi1);
+    }
     for (; s + 1 < ns; s += 2) {
       // fragments 0 hold slice s; register set 0 slice s+1, set 1 slice s+2
       store(1, ra0, rb0);
       load((s + 3) * BK, ra0, rb0);
       __syncthreads();
       read_frag(1, far1, fai1, fbr1, fbi1);
+      issued();
       mma(far0, fai0, fbr0, fbi0);
       // fragments 1 hold slice s+1; set 1 slice s+2 (all zeros past the end), set 0 slice s+3
       store(0, ra1, rb1);
       load((s + 4) * BK, ra1, rb1);
       __syncthreads();
       read_frag(0, far0, fai0, fbr0, fbi0);
+      issued();
       mma(far1, fai1, fbr1, fbi1);
     }
     if (s < ns) mma(far0, fai0, fbr0, fbi0);  // odd slice count: fragments 0 hold the last slice
