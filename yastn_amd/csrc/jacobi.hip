@@ -660,10 +660,15 @@ __device__ inline void tile_of(int tl, int T16, int& ti, int& tj) {
 }
 
 // Partial Gram tiles of one (row chunk, job): the chunk's nc columns are staged in LDS (odd column
-// stride, so the 16 columns of a tile fall in different banks); each wave forms upper-triangle tiles
-// on the matrix cores (lane l supplies A(l % 16, k) = conj(Wp[k, ti 16 + l % 16]) and B(k, l % 16) =
-// Wp[k, tj 16 + l % 16], k = k0 + l / 16) and stores them in the MFMA result order (item v at v 64 + l).
+// stride, so the 16 columns of a tile fall in different banks; zeros past nc and past the rows); each wave forms
+// upper-triangle tiles on the matrix cores (lane l supplies A(l % 16, k) = conj(Wp[k, ti 16 + l % 16]) and
+// B(k, l % 16) = Wp[k, tj 16 + l % 16], k = k0 + l / 16) and stores them in the MFMA result order (item v at v 64 + l).
 // NST = 2 b kGramRows / kChunkThreads staged elements per thread (8 for b <= 16, 16 for b <= 32).
+// A pair of 16-column panels has 3 tiles for 4 waves: which wave is left out changes with the workgroup, as the
+// workgroups of a CU would otherwise all leave the same SIMD idle.  Column addresses are wave-uniform and the zeros
+// spare a test per operand: 5.7 us a round instead of 6.1 (27 real blocks up to 198 x 198).  Large complex blocks are
+// bound by memory (34 us for 105 MB); reading a chunk ahead of the products of the last one made no difference there
+// and cost the small ones 5 %.
 template <bool CPLX, int NST>
 __global__ void __launch_bounds__(kChunkThreads)
     panel_gram_kernel(const int64_t* __restrict__ blocks, const int32_t* __restrict__ jobs,
@@ -672,7 +677,8 @@ __global__ void __launch_bounds__(kChunkThreads)
   typedef Num<CPLX> N;
   typedef typename N::T T;
   extern __shared__ double smem_raw[];
-  constexpr int ld = kGramRows + 1;
+  constexpr int ld = kGramRows + 1, waves = kChunkThreads / 64;
+  static_assert(kGramRows == 64, "a wave stages one column at a time");
   if (sweep_done(state, sweep)) return;
   const int32_t* jb = jobs + 3 * (int64_t)blockIdx.y;
   const BlockDesc d = load_desc(blocks + (int64_t)jb[0] * YH_SVD_WORDS);
@@ -680,45 +686,43 @@ __global__ void __launch_bounds__(kChunkThreads)
   const int64_t r0 = (int64_t)blockIdx.x * kGramRows;
   if (r0 >= pp.p) return;  // uniform: beyond this block's rows
   const int rows = (int)min((int64_t)kGramRows, pp.p - r0);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const T* W = work + d.work_off;
   T* S = reinterpret_cast<T*>(smem_raw);
   {
     // all NST loads of a thread are issued before its first LDS store
-    // (an element outside the chunk reads W[0] and is stored as zero)
+    // (an element outside the chunk reads one inside and is stored as zero)
     T v[NST];
+    const T* src = W + r0 + min(lane, rows - 1);
 #pragma unroll
     for (int i = 0; i < NST; ++i) {
-      const int e = tid + i * kChunkThreads;
-      const int l = e / kGramRows, r = e - l * kGramRows;
-      const bool ok = (l < pp.nc) & (r < rows);
-      v[i] = W[ok ? pp.col(l) * pp.p + r0 + r : 0];
+      const int l = wave + waves * i;
+      v[i] = src[(l < pp.nc ? pp.col(l) : pp.c0i) * pp.p];
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the stores (no interleaving)
+    const T zero = N::make(0.0, 0.0);
 #pragma unroll
     for (int i = 0; i < NST; ++i) {
-      const int e = tid + i * kChunkThreads;
-      const int l = e / kGramRows, r = e - l * kGramRows;
-      if (l < pp.nc) S[l * ld + r] = r < rows ? v[i] : N::make(0.0, 0.0);
+      const int l = wave + waves * i;
+      S[l * ld + lane] = pick((l < pp.nc) & (lane < rows), v[i], zero);
     }
   }
   __syncthreads();
   const int T16 = (pp.nc + 15) / 16, ntile = T16 * (T16 + 1) / 2;
   const int T16m = (2 * b + 15) / 16, ntmax = T16m * (T16m + 1) / 2;
-  for (int tl = wave; tl < ntile; tl += kChunkThreads / 64) {
+  for (int tl = (wave + (int)(blockIdx.x + blockIdx.y)) & (waves - 1); tl < ntile; tl += waves) {
     int ti, tj;
     tile_of(tl, T16, ti, tj);
-    const int ca = ti * 16 + (lane & 15), cb = tj * 16 + (lane & 15);
+    const T* sa = S + (ti * 16 + (lane & 15)) * ld + (lane >> 4);
+    const T* sb = S + (tj * 16 + (lane & 15)) * ld + (lane >> 4);
     d4 accR = {0.0, 0.0, 0.0, 0.0}, accI = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int k0 = 0; k0 < kGramRows; k0 += 4) {
-      const int k = k0 + (lane >> 4);
-      const T a = ca < pp.nc ? S[ca * ld + k] : N::make(0.0, 0.0);
-      const T bb = cb < pp.nc ? S[cb * ld + k] : N::make(0.0, 0.0);
+      const T a = sa[k0], bb = sb[k0];
       accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(a), N::re(bb), accR, 0, 0, 0);
       if constexpr (CPLX) {  // conj(a) b
-        accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::im(a), N::im(bb), accR, 0, 0, 0);
         accI = __builtin_amdgcn_mfma_f64_16x16x4f64(N::re(a), N::im(bb), accI, 0, 0, 0);
+        accR = __builtin_amdgcn_mfma_f64_16x16x4f64(N::im(a), N::im(bb), accR, 0, 0, 0);
         accI = __builtin_amdgcn_mfma_f64_16x16x4f64(-N::im(a), N::re(bb), accI, 0, 0, 0);
       }
     }
@@ -1025,6 +1029,7 @@ __device__ __attribute__((always_inline)) inline bool rotation_short(double a, d
 // In-kernel clocks, 440-row pairs: partial sums 2.5 us, sweep 6.0 us (complex 3.5 and 8.9), against 3 and 13.5 us
 // with 1024 threads, G and Q in LDS and two barriers per sub-round, where one lane computed a slot's parameters while
 // the others waited.  The update holds Q's fragments in registers and reads each stripe one ahead of the products.
+// The update's addresses are one 64-bit add per element (with a 64-bit multiply each: 1.5 to 2.5 % more a round).
 // Kernel time per round: 13.7 us against 21.9 (27 blocks up to 198 x 198), 12.5 against 20 (one 440 x 440 block).
 // Panels of 32 columns with 1024 threads of the same layout move W and V half as often but measured slower
 // (440 x 440: 10.4 against 7.9 ms; four complex 1100 x 1100: 124 against 116 ms).
@@ -1057,17 +1062,34 @@ __global__ void __launch_bounds__(kPairThreads)
   const int sw = (int)((p + 15) / 16), sv = (int)((pp.q + 15) / 16);
   const int per = (sw + sv + (int)gridDim.y - 1) / (int)gridDim.y;
   const int s0 = (int)blockIdx.y * per, s1 = min(sw + sv, s0 + per);
-  auto stripe_col = [&](int st) {  // column c of stripe st's matrix (W, or V after sw stripes)
-    const bool isv = st >= sw;
+  // a lane's eight columns: pointers to them in the matrix of the stripe being read (W, or V after sw stripes), so that
+  // a stripe costs one 64-bit add per element; rows past the matrix read its last one and are not stored
+  uint32_t cidx[KS];
+  T* cp[KS];
+#pragma unroll
+  for (int i = 0; i < KS; ++i) {
+    const int c = 4 * i + (lane >> 4);
+    cidx[i] = (uint32_t)pp.col(c < nc ? c : 0);
+  }
+  auto columns = [&](bool isv) {
     T* X = isv ? Wd + p * pp.q : Wd;
-    const int64_t ldx = isv ? pp.q : p;
-    return [=](int c) { return X + pp.col(c) * ldx; };
+    const uint32_t ldx = (uint32_t)(isv ? pp.q : p);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) cp[i] = X + (uint64_t)cidx[i] * ldx;
   };
   auto stripe_rows = [&](int st) { return st >= sw ? (int)pp.q : (int)p; };
-  auto stripe_idx = [&](int st) { return st >= sw ? st - sw : st; };
+  auto stripe_row = [&](int st) { return (st >= sw ? st - sw : st) * 16 + (lane & 15); };
   T x[KS];
+  auto read_stripe = [&](int st) {
+    const uint32_t r = (uint32_t)min(stripe_row(st), stripe_rows(st) - 1);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) x[i] = cp[i][r];
+  };
   int st = s0 + wave;
-  if (st < s1) stripe_load<CPLX, KS>(x, stripe_col(st), stripe_rows(st), stripe_idx(st), nc, lane);
+  if (st < s1) {
+    columns(st >= sw);
+    read_stripe(st);
+  }
   // ---- G: sums of the chunks' partial tiles (16 x 16 row-major, so thread (k, l) reads its own entries), all
   // loads of a group in flight, summed in chunk order
   T A = N::make(0.0, 0.0), C = A, B = A, D = A;
@@ -1225,13 +1247,19 @@ __global__ void __launch_bounds__(kPairThreads)
     }
   const int tiles = intra ? 1 : 2;
   for (; st < s1; st += kPairThreads / 64) {
-    auto col = stripe_col(st);
-    const int rows = stripe_rows(st), row = stripe_idx(st) * 16 + (lane & 15);
+    const int rows = stripe_rows(st), row = stripe_row(st);
     T y[KS];
 #pragma unroll
     for (int i = 0; i < KS; ++i) y[i] = x[i];
+    if (nc < 2 * b) {  // uniform
+#pragma unroll
+      for (int i = 0; i < KS; ++i) y[i] = pick(4 * i + (lane >> 4) < nc, y[i], N::make(0.0, 0.0));
+    }
     const int nx = st + kPairThreads / 64;
-    if (nx < s1) stripe_load<CPLX, KS>(x, stripe_col(nx), stripe_rows(nx), stripe_idx(nx), nc, lane);
+    const bool cross = nx < s1 && st < sw && nx >= sw;  // uniform, once at most: from W to V
+    if (cross) columns(true);
+    if (nx < s1) read_stripe(nx);
+    if (cross) columns(false);
 #pragma unroll
     for (int tj = 0; tj < 2; ++tj) {
       if (tj < tiles) {
@@ -1248,10 +1276,11 @@ __global__ void __launch_bounds__(kPairThreads)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int c = tj * 16 + (lane >> 4) + 4 * v;
-          if (row < rows && c < nc) col(c)[row] = N::make(accR[v], accI[v]);
+          if (row < rows && c < nc) cp[4 * tj + v][(uint32_t)row] = N::make(accR[v], accI[v]);
         }
       }
     }
+    if (cross) columns(true);
   }
 }
 
@@ -3276,9 +3305,9 @@ extern "C" int yastn_hip_svd_panel_sweep(void* work, const double* floors, int d
   const int gch = (int)((maxch_p * (int64_t)kChunkRows + kGramRows - 1) / kGramRows);  // Gram chunks
   YH_CHECK_ARG(part_numel >= maxn * gch * ntmax * 256 * (cplx ? 2 : 1), "partial Gram buffer too small");
   const int64_t lds_inner = 2 * (2 * b) * (2 * b + 1) * isz;
-  const int64_t lds_gram = (2 * b) * (kGramRows + 1) * isz;
   // the inner kernel's stripe registers cover 4 KS columns: 32 (KS = 8) for b <= 16, else 64
   const bool wide = 2 * b > 32;
+  const int64_t lds_gram = (wide ? 64 : 32) * (kGramRows + 1) * isz;  // all columns the Gram kernel stages
   const void* inner = cplx ? (wide ? (const void*)panel_inner_kernel<true, 16> : (const void*)panel_inner_kernel<true, 8>)
                            : (wide ? (const void*)panel_inner_kernel<false, 16> : (const void*)panel_inner_kernel<false, 8>);
   int st = yh::hip_status(hipFuncSetAttribute(inner, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_inner),
