@@ -1,19 +1,21 @@
 // Batched one-sided Jacobi SVD (Hestenes) and Hermitian eigendecomposition, FP64 / complex128.
 //
-// One workgroup per block.  The block is copied into a column-major working
+// The block is copied into a column-major working
 // matrix W (p x q, p = max(m,n), q = min(m,n); W = A, or A^H when m < n) and a
 // q x q rotation accumulator V = I.  Each sweep visits all column pairs in the
-// round-robin (circle) order, so the q/2 pairs of a round are disjoint and the
-// 16 waves work on different pairs concurrently; a pair is rotated when
-// |w_i^H w_j| > tol * ||w_i|| ||w_j||.  Converged when a sweep rotates nothing.
+// round-robin (circle) order, so the q/2 pairs of a round are disjoint and are
+// rotated concurrently; a pair is rotated when |w_i^H w_j| > tol * ||w_i|| ||w_j||.
+// Converged when a sweep rotates nothing, or only by angles whose squares are
+// below tol / sqrt(2 q) (rotation_short).
 // Then sigma_j = ||w_j||, U = W Sigma^-1 (or V for m < n), sorted descending.
 //
 // Hermitian eigh reuses the same iteration on B = A + mu I, mu = max row
 // abs-sum (Gershgorin, so B is positive semidefinite): the right rotations V are
 // the eigenvectors and lambda_j = sigma_j - mu, written ascending.
 //
-// Blocks whose W and V fit in YH_SVD_LDS_BYTES go through an LDS-resident instance of the
-// kernel (all sweeps in one launch); larger blocks use the panel path below.
+// Blocks of up to YH_SMALL_Q columns are decomposed by one workgroup each in one launch (small_kernel), larger ones
+// by rounds of panel pairs (panel_gram_kernel, panel_pair_kernel), for SVD after a QR of the columns sorted by norm.
+// jacobi_kernel, one workgroup of 16 waves per block with W and V in LDS, serves plans that ask for it past that size.
 #include <float.h>
 
 #include <algorithm>
@@ -604,7 +606,7 @@ __device__ __attribute__((always_inline)) inline void stripe_mul_store(const typ
 // A round of the panel Jacobi runs two kernels over the (block, panel i, panel j) jobs of the round:
 //  1. panel_gram_kernel: the Gram matrix G = Wp^H Wp (nc x nc) of the pair's nc = |I| + |J| columns
 //     Wp, as partial sums over chunks of kGramRows rows, one workgroup per (chunk, job);
-//  2. panel_inner_kernel: per job, `slices` workgroups each sum the partials and run the same inner
+//  2. panel_pair_kernel (panels of 16 columns) or panel_inner_kernel (other widths): per job, `slices` workgroups each sum the partials and run the same inner
 //     sweep of rotations on G (the same quantities and criterion as Hestenes rotations of the
 //     columns; identical arithmetic, so identical results), accumulating the rotation Q (nc x nc), and
 //     then update their slice of the pair's rows of W and V by Q in place.
@@ -1292,7 +1294,7 @@ __global__ void __launch_bounds__(kPairThreads)
 // rotation on the matrix cores; it stops when a sweep rotates nothing.  Like the panel path and unlike jacobi_kernel,
 // a rotation costs no pass over the columns: a sweep of 32 columns takes 31 sub-rounds of about 0.4 us.
 // Kernel time, one block (jacobi_kernel in brackets): 16 x 16 64 us (91), 32 x 32 161 us (440).
-// sweeps each wait for the host; past 32 columns the panel path's several workgroups win.
+// Past 32 columns the panel path's several workgroups win.
 constexpr int kSmallQ = YH_SMALL_Q, kSmallThreads = 256;
 
 // LDS elements of a block: W, V and the two exchange buffers (the accumulated rotation overlays them).
