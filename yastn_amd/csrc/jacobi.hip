@@ -21,6 +21,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "ranking.h"
 
 namespace {
 
@@ -336,8 +337,7 @@ __device__ void finalize_block(const BlockDesc& d, const typename Num<CPLX>::T* 
       const double sj = S[d.s_off + j];
       int cnt = 0;
       for (int64_t i = 0; i < q; ++i) {
-        const double si = S[d.s_off + i];
-        cnt += (si > sj) || (si == sj && i < j);
+        cnt += ranks_before(S[d.s_off + i], i, sj, j);
       }
       rk[z] = cnt;
       sg[z] = sj;
@@ -1511,7 +1511,7 @@ __device__ __attribute__((always_inline)) inline void small_block(
   if (tid < q) {
     const double sj = s_sig[tid];
     int rk = 0;
-    for (int i = 0; i < q; ++i) rk += (s_sig[i] > sj) || (s_sig[i] == sj && i < tid);
+    for (int i = 0; i < q; ++i) rk += ranks_before(s_sig[i], i, sj, tid);
     const int pos = MODE == 1 ? q - 1 - rk : rk;
     s_col[pos] = tid;
     S[d.s_off + pos] = MODE == 1 ? sj - mu : sj;
@@ -2741,14 +2741,14 @@ __global__ void __launch_bounds__(kThreads)
   for (int64_t j = tid; j < qd.q; j += kThreads) {
     double t = 0.0;
     for (int i = 0; i < parts; ++i) t += y.part[i * qd.q + j];
-    y.norm[j] = t == t ? t : HUGE_VAL;  // a total order also for NaN
+    y.norm[j] = t;
     total += t;
   }
   total = block_sum(total, s_red, tid & 63, tid >> 6);
   if (tid == 0) floors[bidx] = DBL_EPSILON * DBL_EPSILON * total;
 }
 
-// rank(j) of norms[j] in descending order, ties by index, one wave per j: f(j, rank).
+// rank(j) of norms[j] (ranks_before), one wave per j: f(j, rank).
 template <typename F>
 __device__ __attribute__((always_inline)) inline void rank_columns(const double* norms, int64_t q, F f) {
   const int lane = threadIdx.x & 63;
@@ -2757,8 +2757,7 @@ __device__ __attribute__((always_inline)) inline void rank_columns(const double*
     const double nj = norms[j];
     double cnt = 0.0;
     for (int64_t i = lane; i < q; i += 64) {
-      const double ni = norms[i];
-      cnt += (ni > nj) || (ni == nj && i < j) ? 1.0 : 0.0;
+      cnt += ranks_before(norms[i], i, nj, j) ? 1.0 : 0.0;
     }
     const int64_t r = (int64_t)wave_sum(cnt);
     if (lane == 0) f(j, r);
