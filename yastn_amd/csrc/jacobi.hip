@@ -3011,6 +3011,19 @@ __global__ void __launch_bounds__(kTileThreads)
 constexpr int kTrsmRows = 16, kTrsmWaves = 8, kTrsmThreads = 64 * kTrsmWaves;
 __host__ __device__ inline int64_t trsm_ld(int64_t k) { return ((k + 15) / 16 * 16) | 1; }  // odd: rows in other banks
 
+// Beside the rows' X: the partial sums of waves 1-7, R1(J, J) of two steps and the reciprocals of its diagonal.
+template <typename T>
+struct TrsmShared {
+  T part[kTrsmWaves - 1][16][17];
+  T R[2][16][17];
+  double ri[2][16];
+};
+
+// Whether 16 rows of k columns fit the 160 KB of LDS beside TrsmShared (39 KB complex, 20 KB real): k <= 480 complex,
+// 1008 real (whose rows are also kept to 128 KB).
+template <typename T>
+constexpr int64_t kTrsmRowBytes = std::min<int64_t>(128 * 1024, 160 * 1024 - sizeof(TrsmShared<T>));
+
 template <bool CPLX, bool IN_LDS>
 __global__ void __launch_bounds__(kTrsmThreads)
     qr_adj_trsm_kernel(const int64_t* __restrict__ words, const typename Num<CPLX>::T* __restrict__ B,
@@ -3018,9 +3031,10 @@ __global__ void __launch_bounds__(kTrsmThreads)
   typedef Num<CPLX> N;
   typedef typename N::T T;
   extern __shared__ double smem_raw[];
-  __shared__ T s_part[kTrsmWaves - 1][16][17];  // partial sums of waves 1-7
-  __shared__ T s_R[2][16][17];                  // R1(J, J)
-  __shared__ double s_ri[2][16];                // the reciprocals of its diagonal
+  __shared__ TrsmShared<T> sh;
+  auto& s_part = sh.part;
+  auto& s_R = sh.R;
+  auto& s_ri = sh.ri;
   const int64_t* w = words + (int64_t)blockIdx.y * YH_QRADJ_WORDS;
   const int64_t m = w[0], n = w[1], k = w[2], b_off = w[4], ga_off = w[5], r_off = w[6];
   const int64_t r0 = (int64_t)blockIdx.x * kTrsmRows;
@@ -3675,7 +3689,7 @@ extern "C" int yastn_hip_qr_adjoint_trsm(void* gA, const void* B, const void* R,
   YH_CHECK_ARG(max_k >= 0 && max_k * yh::itemsize_of(dtype) <= 65536, "qr adjoint row of %lld", (long long)max_k);
   const dim3 g((unsigned)yh::cdiv(max_rows, kTrsmRows), (unsigned)nblocks);
   const int64_t lds = kTrsmRows * trsm_ld(max_k) * yh::itemsize_of(dtype);
-  const bool in_lds = lds <= 128 * 1024;
+  const bool in_lds = lds <= (dtype == YH_F64 ? kTrsmRowBytes<double> : kTrsmRowBytes<double2>);
   if (in_lds) {
     const int st = yh::hip_status(hipFuncSetAttribute(dtype == YH_F64 ? (const void*)qr_adj_trsm_kernel<false, true>
                                                                       : (const void*)qr_adj_trsm_kernel<true, true>,
