@@ -3007,7 +3007,9 @@ __global__ void __launch_bounds__(kTileThreads)
 // to add; their parts are summed in wave order.  The rows' X stays in LDS (IN_LDS) or, where it does not fit, is
 // read back from gA, where this workgroup has written it.
 // 13 blocks of up to 440 columns: 175 us, against 523 with one row per workgroup, a barrier per column and R read along
-// its columns.
+// its columns.  What a lane holds at once is kept to its 256 registers: with the reads of all parts and of R's triangle issued
+// together, 475 of them spilled (complex; 118 real), and QR with its adjoint of 200 complex 33 x 33 blocks took 383 us instead
+// of 250, of four 600 x 600 ones 3.79 ms instead of 3.26.
 constexpr int kTrsmRows = 16, kTrsmWaves = 8, kTrsmThreads = 64 * kTrsmWaves;
 __host__ __device__ inline int64_t trsm_ld(int64_t k) { return ((k + 15) / 16 * 16) | 1; }  // odd: rows in other banks
 
@@ -3091,27 +3093,28 @@ __global__ void __launch_bounds__(kTrsmThreads)
         const int buf = (int)(J & 1);
         T x[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          double tr = 0.0, ti = 0.0;
+        for (int j = 0; j < 16; ++j) x[j] = zero;
+#pragma unroll 1
+        for (int u = 0; u < kTrsmWaves - 1; ++u) {  // 16 reads at a time: all 112 together would not fit the registers
 #pragma unroll
-          for (int u = 0; u < kTrsmWaves - 1; ++u) {
-            tr += N::re(s_part[u][lane][j]);
-            ti += N::im(s_part[u][lane][j]);
+          for (int j = 0; j < 16; ++j) {
+            const T t = s_part[u][lane][j];
+            x[j] = N::make(N::re(x[j]) + N::re(t), N::im(x[j]) + N::im(t));
           }
-          x[j] = N::make(N::re(b[j]) - tr, N::im(b[j]) - ti);
         }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = N::make(N::re(b[j]) - N::re(x[j]), N::im(b[j]) - N::im(x[j]));
         if (J > 0) load_b(j0 - 16);
-        const double mine = s_ri[buf][lane];
-        const bool plain = __all(mine <= DBL_MAX && mine >= -DBL_MAX);  // no zero or denormal diagonal (16 lanes active)
+        // the product with the reciprocal is corrected by its residual unless it is infinite or NaN, as the quotient is then (a
+        // zero diagonal); without a branch, whose two sides would both hold their reads of R
+        auto quotient = [](double a, double r, double ri) {
+          const double t = a * ri;
+          return fabs(t) <= DBL_MAX ? fma(fma(-t, r, a), ri, t) : t;
+        };
 #pragma unroll
         for (int j = 15; j >= 0; --j) {
           const double rjj = N::re(s_R[buf][j][j]), ri = s_ri[buf][j];
-          if (plain) {
-            const double qr = N::re(x[j]) * ri, qi = N::im(x[j]) * ri;
-            x[j] = N::make(fma(fma(-qr, rjj, N::re(x[j])), ri, qr), CPLX ? fma(fma(-qi, rjj, N::im(x[j])), ri, qi) : 0.0);
-          } else {
-            x[j] = N::make(N::re(x[j]) / rjj, N::im(x[j]) / rjj);
-          }
+          x[j] = N::make(quotient(N::re(x[j]), rjj, ri), CPLX ? quotient(N::im(x[j]), rjj, ri) : 0.0);
 #pragma unroll
           for (int i = 0; i < j; ++i) {  // x_i -= x_j conj(R(i, j))
             const T rij = s_R[buf][i][j];
