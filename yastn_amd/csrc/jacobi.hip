@@ -6,7 +6,7 @@
 // round-robin (circle) order, so the q/2 pairs of a round are disjoint and are
 // rotated concurrently; a pair is rotated when |w_i^H w_j| > tol * ||w_i|| ||w_j||.
 // Converged when a sweep rotates nothing, or only by angles whose squares are
-// below tol / sqrt(2 q) (rotation_short).
+// below tol / (2 q) (rotation_short).
 // Then sigma_j = ||w_j||, U = W Sigma^-1 (or V for m < n), sorted descending.
 //
 // Hermitian eigh reuses the same iteration on B = A + mu I, mu = max row
@@ -984,9 +984,9 @@ __device__ __attribute__((always_inline)) inline double rsq_half(double x) {
 // rotation() itself.  Returns false with c = 1, s = 0 where rotation() does not rotate.
 // `more` is set by a rotation after which another sweep is needed.  A sweep leaves of the cosine of a pair what its
 // later rotations bring back, at most 2 (q - 2) products of a sine and a cosine of the sweep (Drmac, Veselic, "New fast
-// and accurate Jacobi SVD algorithm II", SIAM J. Matrix Anal. Appl. 29 (2008), stop by such a product).  With sines and
-// cosines of at most sqrt(last2), last2 = tol / sqrt(2 q) (about 1.2e-8 each), what is left is at the tolerance,
-// with their products taken as a random walk: the sweep that only verifies this (one of 8 to 11) is not run.
+// and accurate Jacobi SVD algorithm II", SIAM J. Matrix Anal. Appl. 29 (2008), stop by such a product).  With squares of
+// sines and cosines of at most last2 = tol / (2 q), what is left is below the tolerance even if all products add up, and the
+// sweep that only verifies this is not run.
 // Clusters, whose sines are large at any cosine, rotate on until no pair does.
 template <bool CPLX>
 __device__ __attribute__((always_inline)) inline bool rotation_short(double a, double b, double gr, double gi,
@@ -1125,7 +1125,7 @@ __global__ void __launch_bounds__(kPairThreads)
     B = N::make(sum[2][0], sum[2][1]);
   }
   const double tol = DBL_EPSILON * sqrt((double)(p > 1 ? p : 1));
-  const double tol2 = tol * tol, floor2 = floors[jb[0]], last2 = tol / sqrt(2.0 * (double)pp.q);
+  const double tol2 = tol * tol, floor2 = floors[jb[0]], last2 = tol / (2.0 * (double)pp.q);
   bool any = false, more = false;
   // one step of the block: rows by the rotation of slot k (J^H), columns by that of slot l (J)
   auto turn = [&](double ck, double srk, double sik, double cl, double srl, double sil) {
@@ -1360,7 +1360,7 @@ __device__ __attribute__((always_inline)) inline void small_block(
     }
     __syncthreads();
   }
-  const double tol = DBL_EPSILON * sqrt((double)(p > 1 ? p : 1)), tol2 = tol * tol, last2 = tol / sqrt(2.0 * q);
+  const double tol = DBL_EPSILON * sqrt((double)(p > 1 ? p : 1)), tol2 = tol * tol, last2 = tol / (2.0 * q);
   double f = 0.0;
   for (int c = wave; c < q; c += kWavesS)
     for (int r = lane; r < p; r += 64) f += N::abs2(W[c * ldw + r]);
