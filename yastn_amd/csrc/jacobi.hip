@@ -978,8 +978,10 @@ __device__ __attribute__((always_inline)) inline double rsq_half(double x) {
 
 // The rotation of rotation() in a shorter chain of dependent operations: with d = b - a, r = sqrt(d^2 + 4 |g|^2)
 // and m = |d| + r, tan(theta) = 2 |g| / m, so c = m / n and s e^{i phi} = sgn(d) 2 g / n with n^2 = m^2 + 4 |g|^2:
-// two reciprocal square roots and no division.  An error of r only tilts the angle (the next sweep sees it); an
-// error of 1 / n scales c and s alike and is removed to rounding by one Newton step on c^2 + s^2 = 1, so that the
+// two reciprocal square roots and no division.  An error of r only tilts the angle: it leaves 2^-45 of the
+// cosine rotated away, which the next sweep sees, and after the last one that is below 2^-45 sqrt(last2) (a second Newton
+// step in r left reconstruction, orthogonality and singular values of blocks of 60 to 1100 columns as they are, and
+// cost 0 to 4 %); an error of 1 / n scales c and s alike and is removed to rounding by one Newton step on c^2 + s^2 = 1, so that the
 // rotations stay orthogonal (c is exactly 1 for tiny angles).  Squares that leave the exponent range take
 // rotation() itself.  Returns false with c = 1, s = 0 where rotation() does not rotate.
 // `more` is set by a rotation after which another sweep is needed.  A sweep leaves of the cosine of a pair what its
