@@ -2413,6 +2413,7 @@ __global__ void __launch_bounds__(INPLACE ? kThreads : kQrThreads)
 // 16 columns.  As three grouped GEMMs per panel (84 launches of 7-19 us for seven blocks of up to 440 x 440, 700 us) the
 // launches and their ramps ruled: 290 us now (1.77 -> 1.47 ms for that QR with its adjoint); the QR of one 3000 x 3000
 // complex block 86 -> 75 ms, of 40 x 40 0.168 -> 0.124: faster at every size, so there is no other path.
+constexpr int64_t kMaxGridY = 65535;
 constexpr int kReflCols = 16, kReflWaves = 8, kReflThreads = 64 * kReflWaves;
 
 template <bool CPLX>
@@ -2424,7 +2425,7 @@ template <bool CPLX, int MODE>
 __global__ void __launch_bounds__(kReflThreads)
     reflect_kernel(const int64_t* __restrict__ blocks, const int64_t* __restrict__ qdesc,
                    const int32_t* __restrict__ ids, typename Num<CPLX>::T* work, typename Num<CPLX>::T* U,
-                   typename Num<CPLX>::T* Vh, int step) {
+                   typename Num<CPLX>::T* Vh, int step, int64_t slab0) {
   typedef Num<CPLX> N;
   typedef typename N::T T;
   constexpr int NB = YH_QR_NB, NPL = CPLX ? 2 : 1;
@@ -2462,7 +2463,7 @@ __global__ void __launch_bounds__(kReflThreads)
     cs = p;
     ncol = K;
   }
-  const int64_t j0 = (int64_t)blockIdx.y * kReflCols;
+  const int64_t j0 = (slab0 + blockIdx.y) * kReflCols;
   if (j0 >= ncol) return;  // uniform
   if (MODE == 2) shi = min(shi, (int)((j0 + kReflCols - 1) / NB));  // column j of E is e_j, zero below, until panel j / NB
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3495,17 +3496,19 @@ template <bool CPLX, int MODE>
 int launch_reflect(const int64_t* d_blocks, const int64_t* d_qdesc, const int32_t* d_ids, int64_t n, void* work, void* U,
                    void* Vh, int step, int64_t max_cols, hipStream_t stream) {
   typedef typename Num<CPLX>::T T;
+  YH_CHECK_ARG(n >= 0 && n <= INT32_MAX && max_cols >= 0, "reflector grid %lld x %lld", (long long)n,
+               (long long)max_cols);
   const int64_t slabs = yh::cdiv(max_cols, kReflCols);
-  YH_CHECK_ARG(n >= 0 && n <= INT32_MAX && max_cols >= 0 && slabs <= 65535, "reflector grid %lld x %lld", (long long)n,
-               (long long)slabs);
   if (n == 0 || slabs == 0) return YH_OK;
   const int st = yh::hip_status(hipFuncSetAttribute((const void*)reflect_kernel<CPLX, MODE>,
                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                                     (int)reflect_lds<CPLX>()),
                                 "reflector LDS size");
   if (st) return st;
-  hipLaunchKernelGGL((reflect_kernel<CPLX, MODE>), dim3((unsigned)n, (unsigned)slabs), dim3(kReflThreads),
-                     reflect_lds<CPLX>(), stream, d_blocks, d_qdesc, d_ids, (T*)work, (T*)U, (T*)Vh, step);
+  for (int64_t s0 = 0; s0 < slabs; s0 += kMaxGridY)  // one launch up to a million columns
+    hipLaunchKernelGGL((reflect_kernel<CPLX, MODE>), dim3((unsigned)n, (unsigned)std::min(slabs - s0, kMaxGridY)),
+                       dim3(kReflThreads), reflect_lds<CPLX>(), stream, d_blocks, d_qdesc, d_ids, (T*)work, (T*)U,
+                       (T*)Vh, step, s0);
   return yh::hip_status(hipGetLastError(), "reflector launch");
 }
 
