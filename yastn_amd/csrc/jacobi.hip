@@ -25,6 +25,8 @@
 
 namespace {
 
+constexpr int64_t kMaxGridY = 65535;  // workgroups of a launch along y
+
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 // Zero elements (never written), read in place of elements outside a matrix so that loads need no
@@ -2413,7 +2415,6 @@ __global__ void __launch_bounds__(INPLACE ? kThreads : kQrThreads)
 // 16 columns.  As three grouped GEMMs per panel (84 launches of 7-19 us for seven blocks of up to 440 x 440, 700 us) the
 // launches and their ramps ruled: 290 us now (1.77 -> 1.47 ms for that QR with its adjoint); the QR of one 3000 x 3000
 // complex block 86 -> 75 ms, of 40 x 40 0.168 -> 0.124: faster at every size, so there is no other path.
-constexpr int64_t kMaxGridY = 65535;
 constexpr int kReflCols = 16, kReflWaves = 8, kReflThreads = 64 * kReflWaves;
 
 template <bool CPLX>
@@ -3322,9 +3323,10 @@ extern "C" int yastn_hip_svd_panel_sweep(void* work, const double* floors, int d
     end = h_rounds[2 * r] + h_rounds[2 * r + 1];
     maxn = std::max(maxn, h_rounds[2 * r + 1]);
   }
-  YH_CHECK_ARG(maxn <= 65535, "jobs per round %lld", (long long)maxn);
+  YH_CHECK_ARG(maxn <= INT32_MAX, "jobs per round %lld", (long long)maxn);
   const int gch = (int)((maxch_p * (int64_t)kChunkRows + kGramRows - 1) / kGramRows);  // Gram chunks
-  YH_CHECK_ARG(part_numel >= maxn * gch * ntmax * 256 * (cplx ? 2 : 1), "partial Gram buffer too small");
+  YH_CHECK_ARG(part_numel >= std::min(maxn, kMaxGridY) * gch * ntmax * 256 * (cplx ? 2 : 1),
+               "partial Gram buffer too small");
   const int64_t lds_inner = 2 * (2 * b) * (2 * b + 1) * isz;
   // the inner kernel's stripe registers cover 4 KS columns: 32 (KS = 8) for b <= 16, else 64
   const bool wide = 2 * b > 32;
@@ -3341,49 +3343,51 @@ extern "C" int yastn_hip_svd_panel_sweep(void* work, const double* floors, int d
                         "svd panel gram LDS size");
   if (st) return st;
   for (int64_t r = 0; r < nrounds; ++r) {
-    const int64_t off = h_rounds[2 * r], n = h_rounds[2 * r + 1];
-    if (n == 0) continue;
-    const int32_t* jobs = d_jobs + 3 * off;
-    const dim3 gg((unsigned)gch, (unsigned)n), gi((unsigned)n, (unsigned)slices);
-    if (cplx) {
-      if (wide)
-        hipLaunchKernelGGL((panel_gram_kernel<true, 16>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
-                           jobs, (const double2*)work, (double*)part, b, gch, d_state, sweep);
-      else
-        hipLaunchKernelGGL((panel_gram_kernel<true, 8>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
-                           jobs, (const double2*)work, (double*)part, b, gch, d_state, sweep);
-      if (b == 16)
-        hipLaunchKernelGGL((panel_pair_kernel<true>), gi, dim3(kPairThreads), 0, stream, d_blocks, jobs, (double2*)work,
-                           floors, (const double*)part, d_state, sweep, gch);
-      else if (wide)
-        hipLaunchKernelGGL((panel_inner_kernel<true, 16>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
-                           d_blocks, jobs, (double2*)work, floors, (const double*)part, d_state, sweep, b, gch,
-                           lds_inner);
-      else
-        hipLaunchKernelGGL((panel_inner_kernel<true, 8>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
-                           d_blocks, jobs, (double2*)work, floors, (const double*)part, d_state, sweep, b, gch,
-                           lds_inner);
-    } else {
-      if (wide)
-        hipLaunchKernelGGL((panel_gram_kernel<false, 16>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
-                           jobs, (const double*)work, (double*)part, b, gch, d_state, sweep);
-      else
-        hipLaunchKernelGGL((panel_gram_kernel<false, 8>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
-                           jobs, (const double*)work, (double*)part, b, gch, d_state, sweep);
-      if (b == 16)
-        hipLaunchKernelGGL((panel_pair_kernel<false>), gi, dim3(kPairThreads), 0, stream, d_blocks, jobs, (double*)work,
-                           floors, (const double*)part, d_state, sweep, gch);
-      else if (wide)
-        hipLaunchKernelGGL((panel_inner_kernel<false, 16>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
-                           d_blocks, jobs, (double*)work, floors, (const double*)part, d_state, sweep, b, gch,
-                           lds_inner);
-      else
-        hipLaunchKernelGGL((panel_inner_kernel<false, 8>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
-                           d_blocks, jobs, (double*)work, floors, (const double*)part, d_state, sweep, b, gch,
-                           lds_inner);
+    // the jobs of a round do not touch each other: a round of more than the Gram kernel's grid takes is split
+    for (int64_t c0 = 0; c0 < h_rounds[2 * r + 1]; c0 += kMaxGridY) {
+      const int64_t off = h_rounds[2 * r] + c0, n = std::min(h_rounds[2 * r + 1] - c0, kMaxGridY);
+      const int32_t* jobs = d_jobs + 3 * off;
+      const dim3 gg((unsigned)gch, (unsigned)n), gi((unsigned)n, (unsigned)slices);
+      if (cplx) {
+        if (wide)
+          hipLaunchKernelGGL((panel_gram_kernel<true, 16>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
+                             jobs, (const double2*)work, (double*)part, b, gch, d_state, sweep);
+        else
+          hipLaunchKernelGGL((panel_gram_kernel<true, 8>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
+                             jobs, (const double2*)work, (double*)part, b, gch, d_state, sweep);
+        if (b == 16)
+          hipLaunchKernelGGL((panel_pair_kernel<true>), gi, dim3(kPairThreads), 0, stream, d_blocks, jobs, (double2*)work,
+                             floors, (const double*)part, d_state, sweep, gch);
+        else if (wide)
+          hipLaunchKernelGGL((panel_inner_kernel<true, 16>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
+                             d_blocks, jobs, (double2*)work, floors, (const double*)part, d_state, sweep, b, gch,
+                             lds_inner);
+        else
+          hipLaunchKernelGGL((panel_inner_kernel<true, 8>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
+                             d_blocks, jobs, (double2*)work, floors, (const double*)part, d_state, sweep, b, gch,
+                             lds_inner);
+      } else {
+        if (wide)
+          hipLaunchKernelGGL((panel_gram_kernel<false, 16>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
+                             jobs, (const double*)work, (double*)part, b, gch, d_state, sweep);
+        else
+          hipLaunchKernelGGL((panel_gram_kernel<false, 8>), gg, dim3(kChunkThreads), (size_t)lds_gram, stream, d_blocks,
+                             jobs, (const double*)work, (double*)part, b, gch, d_state, sweep);
+        if (b == 16)
+          hipLaunchKernelGGL((panel_pair_kernel<false>), gi, dim3(kPairThreads), 0, stream, d_blocks, jobs, (double*)work,
+                             floors, (const double*)part, d_state, sweep, gch);
+        else if (wide)
+          hipLaunchKernelGGL((panel_inner_kernel<false, 16>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
+                             d_blocks, jobs, (double*)work, floors, (const double*)part, d_state, sweep, b, gch,
+                             lds_inner);
+        else
+          hipLaunchKernelGGL((panel_inner_kernel<false, 8>), gi, dim3(kInnerThreads), (size_t)lds_inner, stream,
+                             d_blocks, jobs, (double*)work, floors, (const double*)part, d_state, sweep, b, gch,
+                             lds_inner);
+      }
+      st = yh::hip_status(hipGetLastError(), "svd panel round launch");
+      if (st) return st;
     }
-    st = yh::hip_status(hipGetLastError(), "svd panel round launch");
-    if (st) return st;
   }
   return YH_OK;
 }
