@@ -15,7 +15,8 @@
 //
 // Blocks of up to YH_SMALL_Q columns are decomposed by one workgroup each in one launch (small_kernel), larger ones
 // by rounds of panel pairs (panel_gram_kernel, panel_pair_kernel), for SVD after a QR of the columns sorted by norm.
-// jacobi_kernel, one workgroup of 16 waves per block with W and V in LDS, serves plans that ask for it past that size.
+// jacobi_kernel, one workgroup of 16 waves per block with W and V in LDS, is the better one for few or tall columns and for
+// Hermitian blocks a little too large for small_kernel (the host plan chooses, with the measurements).
 #include <float.h>
 
 #include <algorithm>

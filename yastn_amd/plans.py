@@ -707,11 +707,17 @@ def _circle_pair(ne, r, k):
 
 PRECOND = True  # QR-precondition the panel path of SVD blocks (off: plain one-sided Jacobi on W0)
 # Blocks with more columns than this take the panel path (SVD blocks QR-preconditioned) even where they fit one
-# workgroup, whose sweeps outlast the panel rounds past this size.  Up to 32 columns the one-workgroup kernel is
-# yastn_hip_jacobi_small; larger caps send blocks of more columns to yastn_hip_svd / yastn_hip_eigh.
+# workgroup, whose sweeps outlast the panel rounds past this size.  Up to 32 columns sixteen_waves below chooses between
+# yastn_hip_jacobi_small and yastn_hip_svd / yastn_hip_eigh; larger caps send blocks of more columns to the latter.
 # Measured, 25 Hermitian blocks of 1 ... 106 columns (eigh): cap 128 4.94 ms, 48 2.73, 32 2.12, 16 2.22.
 SVD_LDS_MAX_Q = int(os.environ.get('YASTN_HIP_SVD_LDS_MAX_Q', '32'))
 EIGH_LDS_MAX_Q = int(os.environ.get('YASTN_HIP_EIGH_LDS_MAX_Q', '32'))
+# Up to this many columns a call's Hermitian blocks, at most one per CU (complex: four), all run as one workgroup of 16 waves
+# each: two or three panels spend their sweeps in launches and host reads.  Measured, whole calls, 16 waves and panels, in
+# us: 256 real blocks of 33 columns 451 and 727, one 404 and 530; 36 columns 597 and 742, 550 and 608; 38 631 and 748, 595
+# and 602; 42 799 and 763, 731 and 618; 1000 of 33 1736 and 1344; complex 256 of 36 752 and 1127, one of 38 830 and 796, 1000
+# of 33 2368 and 2666, of 36 2970 and 2976.
+EIGH_SIXTEEN_WAVES_Q = 36
 # Panel width b of the panel Jacobi (a workgroup rotates 2b columns per round): smaller panels give more
 # workgroups per round but more rounds per sweep.  Tuning knob; the LDS limit may lower it further.
 PANEL_WIDTH = int(os.environ.get('YASTN_HIP_PANEL_WIDTH', '16'))
@@ -741,6 +747,22 @@ def panel_slices(cross, stripes, cplx, width):
         g = -(-cross * s // cu)
         return g * stripes * stripe / s / (1.0, 1.35, 1.55, 1.65)[min(g, 4) - 1] + sweep * (1 + 0.8 * (g - 1))
     return min(range(1, max(1, min(64, -(-stripes // 4))) + 1), key=lambda s: (cost(s), s))
+
+
+def sixteen_waves(shapes, mode, cplx, cu):
+    """Whether blocks (p, q) that one workgroup each can decompose go to yastn_hip_svd / yastn_hip_eigh (16 waves a block,
+    a pass over the columns per rotation) and not to yastn_hip_jacobi_small (4 waves, sweeps on the Gram matrix).
+
+    A Gram sweep of 16 or 32 columns has its fixed cost and one wave forms its matrix, so 16 waves win where the
+    columns are few or tall, as long as every CU has one block (more share its issue slots).  Whole calls
+    without the host's part, small against 16 waves, in us: one 4 x 4 block 43 and 33, 256 of them 94 and 71, 1000 254
+    and 247; 256 of 8 x 8 116 and 98, 1000 283 and 344; 30 of 9 x 9 81 and 75, of 10 x 10 82 and 85, of 16 x 16 92 and 140;
+    one real 1000 x 8 234 and 121, 500 x 12 178 and 131, 500 x 14 181 and 156, 500 x 16 182 and 181; complex 500 x 8 237 and
+    170, 500 x 10 286 and 291.  Eigendecompositions: 256 of 8 x 8 69 and 49, of 10 x 10 73 and 75.  All blocks of a call
+    take the same kernel: in one launch the slowest block counts, two launches would add up."""
+    if all(q <= 4 for _, q in shapes):
+        return True
+    return len(shapes) <= cu and all(q <= 9 or (mode == 0 and not cplx and q <= 14 and p >= 32 * q) for p, q in shapes)
 
 
 def _panel_steps(blocks, device):
@@ -776,20 +798,27 @@ class SvdPlan:
         lds_limit = min(L.YH_SVD_LDS_BYTES, dev_lds - 9 * 1024)
         qd = np.zeros((len(blocks), L.YH_QR_WORDS), dtype=np.int64)
         jwords = []
+        shapes = [(n, m) if mode == 0 and m < n else (m, n) for _, m, n, *_r in blocks]
+        cap = EIGH_LDS_MAX_Q if mode == 1 else SVD_LDS_MAX_Q if PRECOND else float('inf')
+        qmax, cu = max((q for _, q in shapes), default=0), L.device_cu_count()
+        if mode == 1 and cap < qmax <= EIGH_SIXTEEN_WAVES_Q and len(blocks) <= (4 * cu if itemsize == 16 else cu):
+            cap, waves16 = qmax, True
+        else:
+            waves16 = sixteen_waves([(p, q) for p, q in shapes if q <= min(cap, L.YH_SMALL_Q)
+                                     and (p * q + q * q) * itemsize <= lds_limit], mode, itemsize == 16, cu)
         for b, (a_off, m, n, u_off, s_off, v_off) in enumerate(blocks):
-            tr = mode == 0 and m < n
-            p, q = (n, m) if tr else (m, n)
+            p, q = shapes[b]
             need = p * q + q * q
             jw = None
-            cap = EIGH_LDS_MAX_Q if mode == 1 else SVD_LDS_MAX_Q if PRECOND else q
             h = 16 if q <= 16 else 32
             need_small = ((p | 1) * q + (q | 1) * q + 2 * h * (h + 1)) * itemsize
-            if q <= min(cap, L.YH_SMALL_Q) and need_small <= dev_lds - 2048 and need * itemsize <= lds_limit:
+            one_workgroup = q <= cap and need * itemsize <= lds_limit
+            if one_workgroup and q <= L.YH_SMALL_Q and not waves16 and need_small <= dev_lds - 2048:
                 small.append(b)
                 small_bytes = max(small_bytes, need_small)
                 lds_bytes = max(lds_bytes, need * itemsize)
                 w_off = 0
-            elif L.YH_SMALL_Q < q <= cap and need * itemsize <= lds_limit:
+            elif one_workgroup and (q > L.YH_SMALL_Q or waves16):
                 lds.append(b)
                 lds_bytes = max(lds_bytes, need * itemsize)
                 w_off = 0
