@@ -536,8 +536,12 @@ class DotDiag(_Fn):
 
 # while a HIP graph is captured the sweeps cannot stop on a host read: the captured SVD launches the most
 # sweeps an eager call of the same plan used, plus this margin (the extra ones exit at once on the device;
-# a replay that needed more reports non-convergence through the deferred checks)
+# a replay that needed more reports non-convergence through the deferred checks).  Hermitian blocks whose matrices fit one
+# workgroup iterate there until they have converged, whatever eager calls saw; those of them that run on the panel path, which is
+# faster, get CAPTURE_EIGH_SWEEPS at least, twice what random and graded blocks take (about 110 us of launches
+# that exit at once: one block of 64 columns 655 us a replay, 545 with the margin alone, 1878 in one workgroup).
 CAPTURE_SWEEP_MARGIN = 3
+CAPTURE_EIGH_SWEEPS = 20
 _DEFERRED = []  # stack of lists collecting convergence flags to check later (deferred_checks)
 
 
@@ -658,7 +662,10 @@ def _run_jacobi(mode, plan, data, out_a, out_s, out_b):
             capturing = torch.cuda.is_current_stream_capturing()
             budget = MAX_SWEEPS
             if capturing and getattr(plan, 'sweeps_seen', None):
-                budget = min(MAX_SWEEPS, plan.sweeps_seen + CAPTURE_SWEEP_MARGIN)
+                budget = plan.sweeps_seen + CAPTURE_SWEEP_MARGIN
+                if mode == 1 and plan.big_fits_lds:
+                    budget = max(budget, CAPTURE_EIGH_SWEEPS)
+                budget = min(MAX_SWEEPS, budget)
             launched = 0
             for sweep in range(budget):
                 L.call('yastn_hip_svd_panel_sweep', ptr(work), ptr(floors), dt, plan.d_jblocks.data_ptr(),

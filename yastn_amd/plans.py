@@ -793,6 +793,7 @@ class SvdPlan:
         words, small, lds, big, pre = [], [], [], [], []
         work = 0
         lds_bytes = small_bytes = 0
+        self.big_fits_lds = False
         dev_lds = L.device_lds_per_block()
         # the LDS kernel also holds ~8 KiB of static shared memory
         lds_limit = min(L.YH_SVD_LDS_BYTES, dev_lds - 9 * 1024)
@@ -838,6 +839,7 @@ class SvdPlan:
                 big.append(b)
                 w_off = work
                 work += need
+                self.big_fits_lds |= need * itemsize <= lds_limit
             words.append((a_off, m, n, u_off, s_off, v_off, w_off, 0))
             jwords.append(jw if jw is not None else words[-1])
         size = lambda b: blocks[b][1] * blocks[b][2] * min(blocks[b][1], blocks[b][2])
