@@ -984,7 +984,7 @@ __device__ __attribute__((always_inline)) inline double rsq_half(double x) {
 // two reciprocal square roots and no division.  An error of r only tilts the angle: it leaves 2^-45 of the
 // cosine rotated away, which the next sweep sees, and after the last one that is below 2^-45 sqrt(last2) (a second Newton
 // step in r left reconstruction, orthogonality and singular values of blocks of 60 to 1100 columns as they are, and
-// cost 0 to 4 %); an error of 1 / n scales c and s alike and is removed to rounding by one Newton step on c^2 + s^2 = 1, so that the
+// cost 0 to 1 %); an error of 1 / n scales c and s alike and is removed to rounding by one Newton step on c^2 + s^2 = 1, so that the
 // rotations stay orthogonal (c is exactly 1 for tiny angles).  Squares that leave the exponent range take
 // rotation() itself.  Returns false with c = 1, s = 0 where rotation() does not rotate.
 // `more` is set by a rotation after which another sweep is needed.  A sweep leaves of the cosine of a pair what its
@@ -2160,7 +2160,17 @@ __device__ __attribute__((always_inline)) inline void qr_pass(typename Num<CPLX>
 #pragma unroll
       for (int u = 0; u < RPL; ++u) x[u] = zero;
     }
-    const T sd = mul_by<CPLX>(N::make(dr, di), scr, -sci);  // conj(s) x^H y
+    T sd = mul_by<CPLX>(N::make(dr, di), scr, -sci);  // conj(s) x^H y
+    if constexpr (!CPLX) {
+      // x^T y overflows where (s x)^T y, with |s x| <= 1, need not: in the last column of a square block, whose own squares are
+      // not taken (those of a complex one are, to make its diagonal real)
+      if (__any(!(fabs(dr) < HUGE_VAL))) {
+        dr = 0.0;
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) dr = fma(x[u] * scr, Y[u], dr);
+        sd = group_sum<G>(dr);
+      }
+    }
     const T w = N::make(yr + N::re(sd), yi + N::im(sd));    // v^H y
     const T cw = mul_by<CPLX>(w, taur, -taui), fw = mul_by<CPLX>(cw, scr, sci);
     // columns up to j are updated by zero: a branch around the update would keep two copies of Y in registers
