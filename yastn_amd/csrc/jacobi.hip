@@ -2270,7 +2270,9 @@ __global__ void __launch_bounds__(INPLACE ? kThreads : kQrThreads)
     constexpr int xs = kQrRegRows<CPLX>;
     const int u = (int)((L + 63) / 64), l = (int)L;
 #define QR_PASSES(G, RPL) qr_passes<CPLX, G, RPL>(P, V, p, l, nb, s_x, xs, s_tr, s_ti, s_co, tid)
-    // the smallest instance in reach; a lane holds 2 RPL elements and at most 60 other registers
+    // the smallest instance in reach; a lane holds 2 RPL elements and at most 60 other registers.  Between 8 and 20 rows per
+    // lane, measured on the panels of 27 blocks of 130 ... 208 rows and 32 columns: complex 13 rows 59-63 us, 16 64-68, 20
+    // 71-75; real 13 rows 42-48, 16 48-54, 20 38-44, so that 20 follow 8 there
     if constexpr (CPLX) {
       if (u <= 1) QR_PASSES(16, 4);
       else if (u <= 2) QR_PASSES(16, 8);
@@ -2284,7 +2286,6 @@ __global__ void __launch_bounds__(INPLACE ? kThreads : kQrThreads)
     } else {
       if (u <= 1) QR_PASSES(16, 4);
       else if (u <= 2) QR_PASSES(16, 8);
-      else if (l <= 208) QR_PASSES(16, 13);
       else if (u <= 5) QR_PASSES(16, 20);
       else if (u <= 7) QR_PASSES(16, 28);
       else if (u <= 9) QR_PASSES(16, 36);
