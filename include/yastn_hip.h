@@ -35,7 +35,7 @@ extern "C" {
 #define YH_F64 0
 #define YH_C128 1
 
-#define YH_ABI_VERSION 18
+#define YH_ABI_VERSION 19
 
 /* ---- box-gather plan (one job per copied or zero-filled box) -------------
  * int64 words per job (YH_JOB_WORDS):
@@ -144,8 +144,9 @@ int yastn_hip_unmerge_adjoint(void* grad_src, const void* grad_new, int64_t nume
 #define YH_TILE_16x64 3   /* skinny M (e.g. MPO contractions) */
 #define YH_TILE_64x16 4   /* skinny N */
 #define YH_TILE_128x128 5 /* large sectors */
-#define YH_TILE_SMALLM 6  /* M <= 16: streaming kernel, a thread per column or two (16 x 512 tiles) */
+#define YH_TILE_SMALLM 6  /* M <= 16: streaming kernel, 16 x 256 tiles; 512 columns for M <= YH_SMALLM_WIDE_ROWS */
 #define YH_TILE_RD32 7    /* 32 x 32, operands read straight into registers, the 4 waves split K (long K) */
+#define YH_SMALLM_WIDE_ROWS 4
 
 int yastn_hip_check_gemm_plan(const int64_t* h_gemms, int64_t ngemms, const int64_t* h_terms, int64_t nterms,
                               const int32_t* h_tiles, int64_t ntiles, int tile_config,

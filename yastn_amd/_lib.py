@@ -12,7 +12,7 @@ LIB_PATH = os.environ.get('YASTN_HIP_LIB', os.path.join(HERE, 'libyastn_hip.so')
 # constants mirrored from include/yastn_hip.h
 YH_OK, YH_ERR_ARG, YH_ERR_HIP, YH_ERR_NUMERIC = 0, -1, -2, -3
 YH_F64, YH_C128 = 0, 1
-YH_ABI_VERSION = 18
+YH_ABI_VERSION = 19
 YH_MAXR = 8
 YH_JOB_WORDS = 32
 YH_JOB_BUFFER_WORD = 30
@@ -24,9 +24,10 @@ YH_MAX_BUFS = 4
 YH_TILE_32x32, YH_TILE_64x64, YH_TILE_128x64, YH_TILE_16x64, YH_TILE_64x16, YH_TILE_128x128 = 0, 1, 2, 3, 4, 5
 YH_TILE_SMALLM = 6
 YH_TILE_RD32 = 7
+YH_SMALLM_WIDE_ROWS = 4
 TILE_DIMS = {YH_TILE_32x32: (32, 32), YH_TILE_64x64: (64, 64), YH_TILE_128x64: (128, 64),
              YH_TILE_16x64: (16, 64), YH_TILE_64x16: (64, 16), YH_TILE_128x128: (128, 128),
-             YH_TILE_SMALLM: (16, 512), YH_TILE_RD32: (32, 32)}
+             YH_TILE_SMALLM: (16, 256), YH_TILE_RD32: (32, 32)}
 YH_SVD_WORDS = 8
 YH_SVD_MAX_Q = 2048
 YH_SMALL_Q = 32

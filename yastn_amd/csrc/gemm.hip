@@ -546,10 +546,15 @@ __global__ void __launch_bounds__(kThreads) splitk_reduce_kernel(Bufs bufs, cons
 // is all M rows times 512 columns; B and C are read / written along the columns.  Bound by latency: a workgroup does
 // little between finding its operands and its stores, so its reads go together.  Four steps of k at a time: lane l of
 // a wave reads A(l % 16, k0 + l / 16), every thread four elements of each of its columns of B, and the entries of A reach
-// the products through scalar registers.  Up to 4 rows, a thread holds two columns; more rows leave no registers
-// for that.  (One k at a time, A by scalar loads and 256 columns: 9.9 us for 280 real GEMMs with K = 4 and 20 MB in all,
-// 7.4 to 8.4 for 184 small complex ones; now 7.4 to 7.7 and 6.0 to 6.2.)
+// the products through scalar registers.  Up to 4 rows, a thread holds two columns where the tile has them; more rows leave
+// no registers for that and take tiles of 256 columns.  (One k at a time, A by scalar loads and 256 columns: 9.9 us for
+// 280 real GEMMs with K = 4 and 20 MB in all, 7.4 to 8.4 for 184 small complex ones; now 7.4 to 7.7 and 6.0 to 6.2.  With
+// 512 columns a workgroup also above 4 rows, in two passes, 100 real GEMMs of 8 x 1000 took 9.1 us, 7.4 one k at a time, now
+// 6.4; waves without columns leave at once: 2000 of 5 x 30 7.9, now 5.2.)
 constexpr int kSmallM = 16, kSmallN = 512;
+
+// Columns of a tile of the streaming kernel for a GEMM of M rows.
+__host__ __device__ inline int small_columns(int64_t M) { return M <= YH_SMALLM_WIDE_ROWS ? kSmallN : kSmallN / 2; }
 
 __device__ __attribute__((always_inline)) inline double lane_value(double v, int l) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
@@ -650,12 +655,14 @@ __global__ void __launch_bounds__(kThreads) gemm_smallm_kernel(Bufs bufs, const 
   const int64_t g = tl[0], j0 = (int64_t)tl[2] + threadIdx.x;
   const int64_t* gw = gemms + g * YH_GEMM_WORDS;
   const Term guess = load_term(g < nterms ? terms + g * YH_TERM_WORDS : gw);
-  if (gw[0] <= 4) {
-    smallm_columns<CPLX, 4, 2>(bufs, gw, terms, guess, g, j0);
-  } else {
+  static_assert(kSmallN == 2 * kThreads, "columns of a thread");
+  if ((int64_t)tl[2] + (threadIdx.x & ~63u) >= gw[1]) return;  // a wave without columns
+  if (gw[0] > YH_SMALLM_WIDE_ROWS)
     smallm_columns<CPLX, kSmallM, 1>(bufs, gw, terms, guess, g, j0);
-    if ((int64_t)tl[2] + kThreads < gw[1]) smallm_columns<CPLX, kSmallM, 1>(bufs, gw, terms, guess, g, j0 + kThreads);
-  }
+  else if ((int64_t)tl[2] + kThreads < gw[1])
+    smallm_columns<CPLX, YH_SMALLM_WIDE_ROWS, 2>(bufs, gw, terms, guess, g, j0);
+  else
+    smallm_columns<CPLX, YH_SMALLM_WIDE_ROWS, 1>(bufs, gw, terms, guess, g, j0);
 }
 
 // BK per configuration (measured on the Heff2 chi=1024 and U(1)xU(1) chi=2048 sector GEMMs): shorter
@@ -752,6 +759,7 @@ extern "C" int yastn_hip_check_gemm_plan(const int64_t* h_gemms, int64_t ngemms,
     const int32_t* x = h_tiles + 3 * t;
     YH_CHECK_ARG(x[0] >= 0 && x[0] < ngemms, "tile %lld: gemm index", (long long)t);
     const int64_t* w = h_gemms + (int64_t)x[0] * YH_GEMM_WORDS;
+    if (cfg == YH_TILE_SMALLM) bn = small_columns(w[0]);
     YH_CHECK_ARG(x[1] >= 0 && x[1] < w[0] && x[1] % bm == 0 && x[2] >= 0 && x[2] < w[1] && x[2] % bn == 0,
                  "tile %lld: origin", (long long)t);
   }

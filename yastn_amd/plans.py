@@ -464,8 +464,10 @@ class GemmPlan:
             tl = []
             for g, row in enumerate(self.h_gemms):
                 M, N = int(row[0]), int(row[1])
+                # the streaming kernel takes two columns per thread where the rows are few
+                cols = 2 * bn if cfg == L.YH_TILE_SMALLM and M <= L.YH_SMALLM_WIDE_ROWS else bn
                 for m0 in range(0, M, bm):
-                    for n0 in range(0, N, bn):
+                    for n0 in range(0, N, cols):
                         tl.append((int(self.k_of[g]), g, m0, n0))
             h = np.ascontiguousarray(np.array(_xcd_order(tl), dtype=np.int32).reshape(-1, 3))
             L.call('yastn_hip_check_gemm_plan', self.h_gemms.ctypes.data, self.ngemms, self.h_terms.ctypes.data,
