@@ -656,13 +656,15 @@ __global__ void __launch_bounds__(kThreads) gemm_smallm_kernel(Bufs bufs, const 
   const int64_t* gw = gemms + g * YH_GEMM_WORDS;
   const Term guess = load_term(g < nterms ? terms + g * YH_TERM_WORDS : gw);
   static_assert(kSmallN == 2 * kThreads, "columns of a thread");
-  if ((int64_t)tl[2] + (threadIdx.x & ~63u) >= gw[1]) return;  // a wave without columns
-  if (gw[0] > YH_SMALLM_WIDE_ROWS)
-    smallm_columns<CPLX, kSmallM, 1>(bufs, gw, terms, guess, g, j0);
-  else if ((int64_t)tl[2] + kThreads < gw[1])
+  if (gw[0] <= YH_SMALLM_WIDE_ROWS && (int64_t)tl[2] + kThreads < gw[1]) {
     smallm_columns<CPLX, YH_SMALLM_WIDE_ROWS, 2>(bufs, gw, terms, guess, g, j0);
-  else
+    return;
+  }
+  if ((int64_t)tl[2] + (threadIdx.x & ~63u) >= gw[1]) return;  // a wave without columns
+  if (gw[0] <= YH_SMALLM_WIDE_ROWS)
     smallm_columns<CPLX, YH_SMALLM_WIDE_ROWS, 1>(bufs, gw, terms, guess, g, j0);
+  else
+    smallm_columns<CPLX, kSmallM, 1>(bufs, gw, terms, guess, g, j0);
 }
 
 // BK per configuration (measured on the Heff2 chi=1024 and U(1)xU(1) chi=2048 sector GEMMs): shorter
