@@ -208,7 +208,8 @@ int yastn_hip_eigh(void* S, void* U, const void* A, int dtype, const int64_t* d_
  * plan too small); finalize writes U, S, Vh (or S, U) like yastn_hip_svd.  Columns whose squared norm
  * is below (eps ||A||_F)^2 (floors[b], set by init) are not rotated, here and in yastn_hip_svd: they are
  * at the rounding-noise level of the block.  maxch_p = ceil(max p / 64); part holds >= (max jobs per
- * round) maxch_p T (T + 1) / 2 256 (x2 complex) doubles, T = ceil(2b / 16).  b <= 32.
+ * round, at most 65535: a larger round is split) maxch_p T (T + 1) / 2 256 (x2 complex) doubles, T = ceil(2b / 16).
+ * b <= 32.
  * yastn_hip_check_panel_jobs validates a job list against the blocks on the host. */
 /* Blocks of A4 / A5 with min(m, n) <= 32: the listed blocks (order[0 ... n-1]; SVD words as for yastn_hip_svd) are each
  * decomposed by one workgroup in one launch, with the outputs and info words of yastn_hip_svd (mode 0) or

@@ -609,10 +609,10 @@ __device__ __attribute__((always_inline)) inline void stripe_mul_store(const typ
 // A round of the panel Jacobi runs two kernels over the (block, panel i, panel j) jobs of the round:
 //  1. panel_gram_kernel: the Gram matrix G = Wp^H Wp (nc x nc) of the pair's nc = |I| + |J| columns
 //     Wp, as partial sums over chunks of kGramRows rows, one workgroup per (chunk, job);
-//  2. panel_pair_kernel (panels of 16 columns) or panel_inner_kernel (other widths): per job, `slices` workgroups each sum the partials and run the same inner
-//     sweep of rotations on G (the same quantities and criterion as Hestenes rotations of the
-//     columns; identical arithmetic, so identical results), accumulating the rotation Q (nc x nc), and
-//     then update their slice of the pair's rows of W and V by Q in place.
+//  2. panel_pair_kernel (panels of 16 columns) or panel_inner_kernel (other widths): per job, `slices` workgroups each
+//     sum the partials and run the same inner sweep of rotations on G (the same quantities and criterion
+//     as Hestenes rotations of the columns; identical arithmetic, so identical results), accumulating the
+//     rotation Q (nc x nc), and then update their slice of the pair's rows of W and V by Q in place.
 // The Gram and update work, products over all p (and q) rows, is spread over many CUs; the inner
 // sweep is repeated per slice instead of being followed by another launch.  A pair that did not
 // rotate writes nothing.
@@ -984,9 +984,9 @@ __device__ __attribute__((always_inline)) inline double rsq_half(double x) {
 // two reciprocal square roots and no division.  An error of r only tilts the angle: it leaves 2^-45 of the
 // cosine rotated away, which the next sweep sees, and after the last one that is below 2^-45 sqrt(last2) (a second Newton
 // step in r left reconstruction, orthogonality and singular values of blocks of 60 to 1100 columns as they are, and
-// cost 0 to 1 %); an error of 1 / n scales c and s alike and is removed to rounding by one Newton step on c^2 + s^2 = 1, so that the
-// rotations stay orthogonal (c is exactly 1 for tiny angles).  Squares that leave the exponent range take
-// rotation() itself.  Returns false with c = 1, s = 0 where rotation() does not rotate.
+// cost 0 to 1 %).  An error of 1 / n scales c and s alike and is removed to rounding by one Newton step on
+// c^2 + s^2 = 1, so that the rotations stay orthogonal (c is exactly 1 for tiny angles).  Squares that leave the
+// exponent range take rotation() itself.  Returns false with c = 1, s = 0 where rotation() does not rotate.
 // `more` is set by a rotation after which another sweep is needed.  A sweep leaves of the cosine of a pair what its
 // later rotations bring back, at most 2 (q - 2) products of a sine and a cosine of the sweep (Drmac, Veselic, "New fast
 // and accurate Jacobi SVD algorithm II", SIAM J. Matrix Anal. Appl. 29 (2008), stop by such a product).  With squares of
@@ -2021,8 +2021,8 @@ __device__ __attribute__((always_inline)) inline void house_coeffs_short(typenam
 // Panels too tall for 32 columns in the registers take passes of 16 or 8, each after the reflectors of the passes before
 // it (read back from Vall), which need no barrier.
 // Means over the panels of a decomposition: 62 us with 16 waves, whole waves per column, the panel in LDS, two chained
-// reductions per column and IEEE divisions, 45 now (seven real blocks of up to 440 rows; 60 with this step but whole waves
-// per column, each wave issuing it for four columns in turn); 50 -> 36 (27 real blocks of up to 198 rows);
+// reductions per column and IEEE divisions, 44 now (seven real blocks of up to 440 rows; 60 with this step but whole waves
+// per column, each wave issuing it for four columns in turn); 50 -> 34 (27 real blocks of up to 198 rows);
 // 280 -> 125 (19 complex blocks of up to 1134 rows, which were factored in place in memory).
 constexpr int kQrWaves = 8, kQrThreads = 64 * kQrWaves;
 
@@ -3022,7 +3022,7 @@ __global__ void __launch_bounds__(kTileThreads)
 // residual), waves 1-7 form the sum of J - 1 over L > J on the matrix cores, so that only the 16 columns of X_J are left
 // to add; their parts are summed in wave order.  The rows' X stays in LDS (IN_LDS) or, where it does not fit, is
 // read back from gA, where this workgroup has written it.
-// 13 blocks of up to 440 columns: 175 us, against 523 with one row per workgroup, a barrier per column and R read along
+// 13 blocks of up to 440 columns: 143 us, against 523 with one row per workgroup, a barrier per column and R read along
 // its columns.  What a lane holds at once is kept to its 256 registers: with the reads of all parts and of R's triangle issued
 // together, 475 of them spilled (complex; 118 real), and QR with its adjoint of 200 complex 33 x 33 blocks took 383 us instead
 // of 250, of four 600 x 600 ones 3.79 ms instead of 3.26.
