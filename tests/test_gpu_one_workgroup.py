@@ -71,3 +71,18 @@ def test_eigh_lists(dims, cplx, counts):
         assert np.max(np.abs(w - np.linalg.eigvalsh(blk))) <= tol
         assert np.linalg.norm(ub * w @ ub.conj().T - blk) <= tol
         assert np.max(np.abs(ub.conj().T @ ub - np.eye(len(w)))) <= 2 * TOL
+
+
+def test_a_lower_cap_is_kept(monkeypatch):
+    from yastn_amd import backend_hip as B
+    n = 20
+    monkeypatch.setattr(P, 'EIGH_LDS_MAX_Q', 16)
+    monkeypatch.setattr(P, '_CACHE', P._Cache())
+    a = _blocks([(n, n)], False, np.random.default_rng(n))[0]
+    a = a + a.T
+    meta = (((0, n * n), (n, n), (0, n * n), (n, n), (0, n)),)
+    x = torch.as_tensor(a.ravel(), device=DEV)
+    plan = P.eigh_plan(meta, 8, n * n, (n, n * n), x.device)
+    assert (plan.n_small, plan.n_lds, plan.n_big) == (0, 0, 1)
+    S, _ = B.eigh(x, meta, (n, n * n))
+    assert np.max(np.abs(S.cpu().numpy() - np.linalg.eigvalsh(a))) <= TOL * np.sqrt(n) * np.linalg.norm(a)

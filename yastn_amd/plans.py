@@ -804,7 +804,8 @@ class SvdPlan:
         shapes = [(n, m) if mode == 0 and m < n else (m, n) for _, m, n, *_r in blocks]
         cap = EIGH_LDS_MAX_Q if mode == 1 else SVD_LDS_MAX_Q if PRECOND else float('inf')
         qmax, cu = max((q for _, q in shapes), default=0), L.device_cu_count()
-        if mode == 1 and cap < qmax <= EIGH_SIXTEEN_WAVES_Q and len(blocks) <= (4 * cu if itemsize == 16 else cu):
+        if mode == 1 and cap == L.YH_SMALL_Q < qmax <= EIGH_SIXTEEN_WAVES_Q \
+                and len(blocks) <= (4 * cu if itemsize == 16 else cu):
             cap, waves16 = qmax, True
         else:
             waves16 = sixteen_waves([(p, q) for p, q in shapes if q <= min(cap, L.YH_SMALL_Q)
